@@ -60,6 +60,23 @@ __device__ __forceinline__ cplx<R> rot(cplx<R> a, int m_in)
     return {a.x * c - a.y * s, a.x * s + a.y * c};
 }
 
+// Store that bypasses the L2's write-back (nt): for results in whole cache
+// lines, which otherwise sit dirty in the L2 until the launch ends and are
+// flushed then, after the last workgroup.
+template <typename R>
+__device__ __forceinline__ void store_nt(cplx<R>* p, cplx<R> v)
+{
+    typedef R vec __attribute__((ext_vector_type(2)));
+    vec w;
+    w.x = v.x;
+    w.y = v.y;
+    __builtin_nontemporal_store(w, reinterpret_cast<vec*>(p));
+}
+
+// Around the stores of a branch that differs from its sibling only in store_nt:
+// without it the optimiser merges the two branches into ordinary stores.
+__device__ __forceinline__ void keep_branch() { asm volatile("" ::: "memory"); }
+
 template <int R_, typename R>
 struct Dft;
 

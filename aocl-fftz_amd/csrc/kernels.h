@@ -5,28 +5,31 @@
 
 namespace fftz {
 
-enum class KernelKind { Pass, Bluestein };
+enum class KernelKind { Pass, Real, RealWide, Bluestein };
 
 // Device function symbol for hipLaunchKernel / hipFuncSetAttribute.
 // prec_bytes: 4 (complex64) or 8 (complex128).  all_radix: the variant that
 // carries the 3/5/6/7/9/10/11/12/13 stages (the power-of-two variant carries
-// only 2/4/8/16 and therefore needs fewer VGPRs).  E: complex values per
-// thread per stage (8 or 16).  maxt: block-size bound of the variant (256 or
-// 1024); the 256 variants get a larger VGPR budget.
-const void* kernel_symbol(KernelKind kind, int prec_bytes, bool all_radix, int E, int maxt);
+// only 2/4/8/16 and therefore needs fewer VGPRs).  nt: the variant whose
+// complex results bypass the L2's write-back (kNtStore).  maxt: block-size bound of
+// the variant, 256 or more (then 1024 threads in complex64, 512 in
+// complex128); the 256 variants get a larger VGPR budget.  Real: passes with a
+// real side (kRealFlags); RealWide: real-packed ones whose pair stage (last for
+// R2C, first for C2R) has radix 11 or 13.
+const void* kernel_symbol(KernelKind kind, int prec_bytes, bool all_radix, bool nt, int maxt);
 
-// Uneven-batch persistent kernel (k_batch) and the counter reset kernel
-// launched before it.  Classes: E = 8 with 256 threads, E = 16 with 512 or
-// 1024 threads.
-const void* kernel_symbol_batch(int prec_bytes, int E, int maxt);
+// Uneven-batch persistent kernel (k_batch) of a tile class (0 small: 256
+// threads, 1 medium: 512, 2 large: 1024 in complex64, 512 in complex128) and
+// the counter reset kernel launched before it.
+const void* kernel_symbol_batch(int prec_bytes, int cls);
 const void* kernel_symbol_reset();
 
 // Instantiation units behind kernel_symbol / kernel_symbol_batch (one
 // translation unit each, compiled in parallel).
-const void* kernel_symbol_pass_f32_mixed(KernelKind kind, int E, int maxt);
-const void* kernel_symbol_pass_f32_pow2(KernelKind kind, int E, int maxt);
-const void* kernel_symbol_pass_f64_mixed(KernelKind kind, int E, int maxt);
-const void* kernel_symbol_pass_f64_pow2(KernelKind kind, int E, int maxt);
+const void* kernel_symbol_pass_f32_mixed(KernelKind kind, bool nt, int maxt);
+const void* kernel_symbol_pass_f32_pow2(KernelKind kind, bool nt, int maxt);
+const void* kernel_symbol_pass_f64_mixed(KernelKind kind, bool nt, int maxt);
+const void* kernel_symbol_pass_f64_pow2(KernelKind kind, bool nt, int maxt);
 const void* kernel_symbol_batch_f32_small();
 const void* kernel_symbol_batch_f32_medium();
 const void* kernel_symbol_batch_f32_large();

@@ -2,19 +2,28 @@
 //
 // One workgroup owns a tile of C lines of length L.  The tile is loaded from
 // HBM once (coalesced along the line for row passes, across adjacent lines for
-// column passes), every Stockham stage of the length-L transform runs out of
+// column passes), every radix stage of the length-L transform runs out of
 // LDS through VGPRs, and the tile is written back once -- one HBM round trip
 // per pass.  Element-wise work that the reference runs as separate sweeps
 // (ele_mul, fused_twiddle_transpose, recombine/separate) is folded into the
 // load or store of the adjacent pass.
 //
-// Stage s of radix R (Stockham autosort, the geometry of the reference's
-// pow2_setup_stage_layout, core/solvers/complex/pow2_iterative_solver_dft.c:27-78):
-//   butterfly j = g*ls + c reads  x[i*(L/R) + j],             i < R
-//   multiplies leg i by w_{R*ls}^(i*c),
-//   writes   y[g*R*ls + i*ls + c].
-// Reads and writes happen in place with a workgroup barrier in between; each
-// thread holds its K = ceil(E/R) butterflies in VGPRs across the barrier.
+// The first stage takes its operands straight from HBM and the last stage
+// stores straight to it.  In between a line sits in LDS as mixed-radix digits
+// and stage s transforms digit s in place: a butterfly writes the positions
+// that it read, so a stage needs one barrier, one set of addresses, no
+// registers held across a barrier and no particular number of butterflies per
+// thread (threads loop over the line's butterflies).  The output order comes
+// from the last stage's numbering of its butterflies.  What bounds it: vector
+// issue and LDS latency rather than HBM, at 75 VALU instructions per element
+// for three stages (a self-sorting form with its results moved and guarded
+// took 112).  Measured, before -> after: 3001 complex64 lines of 1200
+// (12 x 10 x 10) 26.7 -> 17.9 us; 9 lines of 1,000,000 as three passes of 100
+// 187 -> 112 us; 1500 complex128 lines of 1009 (Bluestein, M = 2048)
+// 37.1 -> 30.8 us; 2000 uneven items 2.87 -> 2.32 ms.  (The reference's
+// self-sorting geometry, core/solvers/complex/pow2_iterative_solver_dft.c:27-78,
+// moves every stage's results instead.)
+//
 // Included by the instantiation units kernels_pass_{f32,f64}_{mixed,pow2}.hip
 // and kernels_batch_{f32,f64}_{small,medium,large}.hip (compiled in
 // parallel); kernels.hip holds the launch-table dispatch.
@@ -90,9 +99,6 @@ __device__ __forceinline__ SlotLine slot_line(const PassDesc& p, const TileIo& i
     return SlotLine{l, cc < p.ln0.d && (int64_t)l < io.nlines};
 }
 
-template <typename R>
-__device__ __forceinline__ cplx<R> to_prec(double x, double y) { return {R(x), R(y)}; }
-
 // w_N^p from the two-level FP64 table: hi[p >> b] * lo[p & (2^b - 1)].
 __device__ __forceinline__ cplx<double> tw4_root(const PassDesc& p, int64_t q)
 {
@@ -103,373 +109,589 @@ __device__ __forceinline__ cplx<double> tw4_root(const PassDesc& p, int64_t q)
     return cmul(hi, lo);
 }
 
-// ---------------------------------------------------------------------------
-// Tile load / store.
-// Row passes: thread -> (line c = tid / TL, lane t = tid % TL): a wavefront
-// walks consecutive elements of one line.  Column passes: (c = tid % C,
-// t = tid / C): a wavefront walks the same element of C adjacent lines.
-// ---------------------------------------------------------------------------
-template <typename R, int E>
-__device__ __forceinline__ void load_tile(const PassDesc& p, const TileIo& io, cplx<R>* lds, int64_t l_base, int tid)
+__device__ __forceinline__ uint32_t sdiv(uint32_t n, const SmallDiv& f) { return __umul24(n, f.mul) >> f.shift; }
+
+// Workgroup barrier that waits only for this wave's LDS traffic (the stages
+// exchange data through LDS alone; twiddle loads and result stores in flight
+// are not waited for).  Lines that sit in one wavefront each need no barrier:
+// a wave's own LDS operations complete in order once counted down.
+__device__ __forceinline__ void stage_sync(bool wave_local)
 {
-    const bool col = (p.flags & kInCol) != 0;
-    const int c = col ? (tid & (p.C - 1)) : (tid >> p.tl_shift);
-    const int t = col ? (tid >> p.c_shift) : (tid & (p.TL - 1));
-    const SlotLine sl = slot_line(p, io, l_base, c);
-    if (!sl.live) return;
-    LineIdx li = line_index(p, io, sl.l);
-    cplx<R>* line = lds + c * p.LP;
-    if (p.flags & kRealIn) {
-        // R2C: element j of the L-point complex line is (x[2j], x[2j+1])
-        const R* src = reinterpret_cast<const R*>(io.in) + li.ioff;
-        cplx<R> v[E];
+    if (wave_local)
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    else
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+// ---------------------------------------------------------------------------
+// LDS positions.  A line is kept as mixed-radix digits: position
+// d0 A0 + d1 A1 + ... + d(S-1), As = p.lst[s], where digit s holds the input
+// digit n_s before stage s and the output digit k_s after it (input index
+// n0 L/R0 + n1 L/(R0 R1) + ..., output index k0 + R0 k1 + R0 R1 k2 + ...).
+// Stage s transforms digit s, so it reads and writes the same R_s positions.
+// ---------------------------------------------------------------------------
+
+// Leg 0 of butterfly j of the last stage (j = k0 + R0 k1 + ..., so that the
+// outputs j + i L/R of neighbouring lanes are neighbours); legs are adjacent.
+__device__ __forceinline__ int last_base(const PassDesc& p, int j)
+{
+    const int S = p.nst;
+    uint32_t rem = (uint32_t)j, base = 0;
+    for (int s = 0; s + 2 < S; s++) {
+        const uint32_t q = sdiv(rem, p.rdiv[s]);
+        base += __umul24(rem - __umul24(q, (uint32_t)p.radix[s]), (uint32_t)p.lst[s]);
+        rem = q;
+    }
+    return (int)(base + __umul24(rem, (uint32_t)p.lst[S - 2]));
+}
+
+// Leg 0 of butterfly j of a middle stage s; m is the index below digit s
+// (the stage's twiddle column).  Only A0 is padded, so the digits between 0
+// and s are one dense run.
+__device__ __forceinline__ int mid_base(const PassDesc& p, int s, int j, uint32_t& m)
+{
+    const uint32_t o = sdiv((uint32_t)j, p.mdiv[s]);
+    m = (uint32_t)j - __umul24(o, (uint32_t)p.lst[s]);
+    const uint32_t d0 = sdiv(o, p.odiv[s]);
+    const uint32_t r = o - __umul24(d0, (uint32_t)p.on[s]);
+    return (int)(__umul24(d0, (uint32_t)p.lst[0]) + __umul24(r, (uint32_t)(p.radix[s] * p.lst[s])) + m);
+}
+
+// Stage twiddles, one row per output digit k >= 1 and one column per index m
+// below the digit: w_{Rs As}^(k m), so neighbouring lanes read neighbours.
+template <typename R>
+__device__ __forceinline__ const cplx<R>* stage_tw(const PassDesc& p, int s)
+{
+    return reinterpret_cast<const cplx<R>*>(p.stw) + p.twoff[s];
+}
+
+template <typename R, int RAD>
+__device__ __forceinline__ void load_twiddles(const cplx<R>* tw, uint32_t m, int cols, cplx<R> (&w)[RAD - 1])
+{
 #pragma unroll
-        for (int k = 0; k < E; k++) {
-            const int e = t + k * p.TL;
-            if (e < p.L) {
-                v[k].x = src[(int64_t)(2 * e) * p.ies];
-                v[k].y = src[(int64_t)(2 * e + 1) * p.ies];
+    for (int i = 0; i < RAD - 1; i++) w[i] = tw[m + (uint32_t)(i * cols)];
+}
+
+template <typename R, int RAD>
+__device__ __forceinline__ void apply_twiddles(cplx<R> (&v)[RAD], const cplx<R> (&w)[RAD - 1])
+{
+#pragma unroll
+    for (int i = 1; i < RAD; i++) v[i] = cmul(v[i], w[i - 1]);
+}
+
+// Middle stage in place: DFT then twiddle (decimation in frequency), or, for
+// the second transform of a Bluestein pass, twiddle then DFT with the same
+// table (decimation in time: digits return from output to input order).
+// Addresses and twiddles of the first butterfly are fetched before the
+// barrier that makes the previous stage's results visible: their latency
+// (tables of long lines live in the L2 or beyond) overlaps the barrier.
+template <typename R, int RAD, bool DIT>
+__device__ __forceinline__ void mid_stage(const PassDesc& p, cplx<R>* line, int t, int s, bool live, bool wave_local)
+{
+    const int nbl = live ? p.nbl[s] : 0, step = p.lst[s];
+    const cplx<R>* tw = stage_tw<R>(p, s);
+    int j = t, base = 0;
+    cplx<R> w[RAD - 1];
+    auto fetch = [&]() {
+        if (j < nbl) {
+            uint32_t m;
+            base = mid_base(p, s, j, m);
+            load_twiddles<R, RAD>(tw, m, step, w);
+        }
+    };
+    fetch();
+    stage_sync(wave_local);
+#pragma unroll 1
+    while (j < nbl) {
+        cplx<R>* q = line + base;
+        cplx<R> v[RAD];
+#pragma unroll
+        for (int i = 0; i < RAD; i++) v[i] = q[i * step];
+        if constexpr (DIT) apply_twiddles<R, RAD>(v, w);
+        Dft<RAD, R>::run(v);
+        if constexpr (!DIT) apply_twiddles<R, RAD>(v, w);
+#pragma unroll
+        for (int i = 0; i < RAD; i++) q[i * step] = v[i];
+        j += p.TL;
+        fetch();
+    }
+}
+
+#define FFTZ_RADIX_CASE(r, CALL) \
+    case r: {                    \
+        constexpr int RAD = r;   \
+        CALL;                    \
+    } break;
+
+#define FFTZ_RADIX_SWITCH(rad, ALLRAD, CALL)       \
+    switch (rad) {                                 \
+        FFTZ_RADIX_CASE(2, CALL)                   \
+        FFTZ_RADIX_CASE(4, CALL)                   \
+        FFTZ_RADIX_CASE(8, CALL)                   \
+        FFTZ_RADIX_CASE(16, CALL)                  \
+        default:                                   \
+            if constexpr (ALLRAD) {                \
+                switch (rad) {                     \
+                    FFTZ_RADIX_CASE(3, CALL)       \
+                    FFTZ_RADIX_CASE(5, CALL)       \
+                    FFTZ_RADIX_CASE(6, CALL)       \
+                    FFTZ_RADIX_CASE(7, CALL)       \
+                    FFTZ_RADIX_CASE(9, CALL)       \
+                    FFTZ_RADIX_CASE(10, CALL)      \
+                    FFTZ_RADIX_CASE(11, CALL)      \
+                    FFTZ_RADIX_CASE(12, CALL)      \
+                    FFTZ_RADIX_CASE(13, CALL)      \
+                    default: break;                \
+                }                                  \
+            }                                      \
+            break;                                 \
+    }
+
+// Radices of the stage that holds mirrored butterfly pairs (kRealPair: up to
+// 10, kRealWide: 11 and 13).
+#define FFTZ_PAIR_SWITCH(rad, ALLRAD, REAL, CALL)  \
+    if constexpr (REAL == kRealWide) {             \
+        switch (rad) {                             \
+            FFTZ_RADIX_CASE(11, CALL)              \
+            FFTZ_RADIX_CASE(13, CALL)              \
+            default: break;                        \
+        }                                          \
+    } else {                                       \
+        switch (rad) {                             \
+            FFTZ_RADIX_CASE(2, CALL)               \
+            FFTZ_RADIX_CASE(4, CALL)               \
+            FFTZ_RADIX_CASE(8, CALL)               \
+            default:                               \
+                if constexpr (ALLRAD) {            \
+                    switch (rad) {                 \
+                        FFTZ_RADIX_CASE(3, CALL)   \
+                        FFTZ_RADIX_CASE(5, CALL)   \
+                        FFTZ_RADIX_CASE(6, CALL)   \
+                        FFTZ_RADIX_CASE(7, CALL)   \
+                        FFTZ_RADIX_CASE(9, CALL)   \
+                        FFTZ_RADIX_CASE(10, CALL)  \
+                        default: break;            \
+                    }                              \
+                }                                  \
+                break;                             \
+        }                                          \
+    }
+
+// ---------------------------------------------------------------------------
+// HBM side.  The first stage loads its butterflies' operands x[i nbl + j]
+// straight into registers and the last stage stores y[i nbl + j] straight from
+// them, both coalesced over j.
+// ---------------------------------------------------------------------------
+
+// Two adjacent real elements as one complex value; a real line may start at
+// an odd element, so only the real type's alignment is assumed.
+template <typename R>
+struct RealPair {
+    typedef R vec __attribute__((ext_vector_type(2), aligned(sizeof(R))));
+};
+
+template <typename R>
+__device__ __forceinline__ cplx<R> load_pair(const R* s, int64_t es)
+{
+    if (es == 1) {
+        const auto w = *reinterpret_cast<const typename RealPair<R>::vec*>(s);
+        return {w.x, w.y};
+    }
+    return {s[0], s[es]};
+}
+
+template <typename R>
+__device__ __forceinline__ void store_pair(R* d, int64_t es, cplx<R> v)
+{
+    if (es == 1) {
+        typename RealPair<R>::vec w;
+        w.x = v.x;
+        w.y = v.y;
+        *reinterpret_cast<typename RealPair<R>::vec*>(d) = w;
+    } else {
+        d[0] = v.x;
+        d[es] = v.y;
+    }
+}
+
+// Operands of butterfly j of stage 0, as the transform takes them (conjugated
+// for the backward direction).  src is the line's element 0; for the flags
+// that read reals it points at real elements.
+template <typename R, int RAD, bool REAL>
+__device__ __forceinline__ void load_butterfly(const PassDesc& p, const cplx<R>* src, int j, int64_t gbase,
+                                               cplx<R> (&v)[RAD])
+{
+    const int nbl = p.nbl[0];
+    if constexpr (REAL) {
+        const R* s = reinterpret_cast<const R*>(src);
+        if (p.flags & kRealIn) {
+            const R* q = s + (int64_t)(2 * j) * p.ies;
+            const int64_t step = (int64_t)(2 * nbl) * p.ies;
+#pragma unroll
+            for (int i = 0; i < RAD; i++) v[i] = load_pair<R>(q + i * step, p.ies);
+            return;
+        }
+        if (p.flags & kRealPromote) {
+            const R* q = s + (int64_t)j * p.ies;
+            const int64_t step = (int64_t)nbl * p.ies;
+#pragma unroll
+            for (int i = 0; i < RAD; i++) v[i] = {q[i * step], R(0)};
+            return;
+        }
+        if (p.flags & kHermIn) {
+            // bins 0..n/2 are stored; bin e > n/2 is conj(bin n - e)
+            const int n = p.nvalid_in;
+#pragma unroll
+            for (int i = 0; i < RAD; i++) {
+                const int e = i * nbl + j;
+                const bool up = 2 * e > n;
+                v[i] = src[(int64_t)(up ? n - e : e) * p.ies];
+                if (up) v[i].y = -v[i].y;
             }
         }
+    } else if (p.flags & kChirpIn) {
+        // x * chirp[g] for g < nchirp, 0 beyond (the input holds only nchirp elements)
 #pragma unroll
-        for (int k = 0; k < E; k++) {
-            const int e = t + k * p.TL;
-            if (e < p.L) line[lds_pad(e)] = v[k];
+        for (int i = 0; i < RAD; i++) {
+            const int e = i * nbl + j;
+            const int64_t g = gbase + (int64_t)e * p.gin[3];
+            v[i] = {R(0), R(0)};
+            if (g < p.nchirp) {
+                v[i] = src[(int64_t)e * p.ies];
+                if (p.flags & kConjIn) v[i].y = -v[i].y;
+                v[i] = cmul(v[i], reinterpret_cast<const cplx<R>*>(p.chirp)[g]);
+            }
         }
         return;
     }
-    if (p.flags & (kRealPromote | kHermIn)) {
-        // full-length real transforms: real x[e] as (x[e], 0), or the Hermitian
-        // extension of bins 0..n/2 (n = nvalid_in)
-        const int n = p.nvalid_in;
-        cplx<R> v[E];
+    if (!REAL || !(p.flags & kHermIn)) {
+        const cplx<R>* q = src + (int64_t)j * p.ies;
+        const int64_t step = (int64_t)nbl * p.ies;
 #pragma unroll
-        for (int k = 0; k < E; k++) {
-            const int e = t + k * p.TL;
-            v[k] = {R(0), R(0)};
-            if (e < n) {
-                if (p.flags & kRealPromote) {
-                    const R* srcr = reinterpret_cast<const R*>(io.in) + li.ioff;
-                    v[k].x = srcr[(int64_t)e * p.ies];
-                } else {
-                    const cplx<R>* srcc = reinterpret_cast<const cplx<R>*>(io.in) + li.ioff;
-                    const int m = 2 * e <= n ? e : n - e;
-                    v[k] = srcc[(int64_t)m * p.ies];
-                    if (2 * e > n) v[k].y = -v[k].y;
-                }
-                if (p.flags & kConjIn) v[k].y = -v[k].y;
-            }
-        }
-#pragma unroll
-        for (int k = 0; k < E; k++) {
-            const int e = t + k * p.TL;
-            if (e < p.L) line[lds_pad(e)] = v[k];
-        }
-        return;
-    }
-    const cplx<R>* src = reinterpret_cast<const cplx<R>*>(io.in) + li.ioff;
-    const int nv = p.nvalid_in;
-    const int ncover = (p.flags & kC2RPre) ? p.L + 1 : p.L;
-    cplx<R> v[E + 1];
-#pragma unroll
-    for (int k = 0; k < E + 1; k++) {
-        const int e = t + k * p.TL;
-        v[k] = {R(0), R(0)};
-        if (e < nv) v[k] = src[(int64_t)e * p.ies];
+        for (int i = 0; i < RAD; i++) v[i] = q[i * step];
     }
     if (p.flags & kConjIn) {
 #pragma unroll
-        for (int k = 0; k < E + 1; k++) v[k].y = -v[k].y;
-    }
-#pragma unroll
-    for (int k = 0; k < E + 1; k++) {
-        const int e = t + k * p.TL;
-        if (e < ncover) line[lds_pad(e)] = v[k];
+        for (int i = 0; i < RAD; i++) v[i].y = -v[i].y;
     }
 }
 
-// Real-packed separate (C2R pre-processing), in LDS, on the L+1 loaded bins:
-//   Z_k = E_k + i O_k,  E_k = X_k + conj(X_{L-k}),
-//   O_k = (X_k - conj(X_{L-k})) exp(+2 pi i k / 2L);
-// stored conjugated so the forward stages compute the inverse transform.
-template <typename R>
-__device__ __forceinline__ void c2r_separate(const PassDesc& p, cplx<R>* lds, int tid)
+// One result; NT: past the L2's write-back (kNtStore).  A kernel's parameter
+// rather than a branch: both forms of the store in one kernel measured 2-3%
+// slower (3001 lines of 1200: 16.9 against 16.5 us).
+template <typename R, bool NT>
+__device__ __forceinline__ void put(cplx<R>* d, cplx<R> v)
 {
-    const int c = tid >> p.tl_shift;
-    const int t = tid & (p.TL - 1);
-    if (c >= p.C) return;
-    cplx<R>* line = lds + c * p.LP;
-    const cplx<R>* rtw = reinterpret_cast<const cplx<R>*>(p.rtw);
-    const int L = p.L;
-    for (int k = t; k <= L / 2; k += p.TL) {
-        cplx<R> xk = line[lds_pad(k)];
-        cplx<R> xm = line[lds_pad(L - k)];
-        cplx<R> w = rtw[k];  // exp(-2 pi i k / 2L)
-        // k side
-        cplx<R> ek = {xk.x + xm.x, xk.y - xm.y};
-        cplx<R> dk = {xk.x - xm.x, xk.y + xm.y};
-        cplx<R> ok = cmul(dk, cconj(w));
-        cplx<R> zk = {ek.x - ok.y, ek.y + ok.x};
-        // L-k side: E = conj(ek), O = (X_{L-k} - conj(X_k)) * (-w)
-        cplx<R> em = {ek.x, -ek.y};
-        cplx<R> dm = {xm.x - xk.x, xm.y + xk.y};
-        cplx<R> om = cmul(dm, cplx<R>{-w.x, -w.y});
-        cplx<R> zm = {em.x - om.y, em.y + om.x};
-        if (k == 0) {
-            line[lds_pad(0)] = cconj(zk);
-        } else {
-            line[lds_pad(k)] = cconj(zk);
-            if (k != L - k) line[lds_pad(L - k)] = cconj(zm);
-        }
-    }
-}
-
-// Legs b0 + i * stride (i < RAD) of a line in the padded LDS layout.  When
-// the stride is a multiple of 16 (LIN) the pad term carries nothing between
-// legs: lds_pad(b0 + i stride) = lds_pad(b0) + i (stride + stride / 16), so
-// each leg's slot is one add of a uniform step from the first.  Callers pick
-// LIN with a uniform branch so the two address forms are separate code
-// (complex64 only: the complex128 1024-thread variants, at their 128-VGPR
-// bound, spill with both forms present).
-template <typename R, int RAD, bool LIN>
-__device__ __forceinline__ void lds_gather(const cplx<R>* line, int b0, int stride, cplx<R> (&v)[RAD])
-{
-    if constexpr (LIN) {
-        const int step = stride + (stride >> 4);
-        const cplx<R>* q = line + lds_pad(b0);
-#pragma unroll
-        for (int i = 0; i < RAD; i++) v[i] = q[i * step];
-    } else {
-#pragma unroll
-        for (int i = 0; i < RAD; i++) v[i] = line[lds_pad(b0 + i * stride)];
-    }
-}
-
-template <typename R, int RAD, bool LIN>
-__device__ __forceinline__ void lds_scatter(cplx<R>* line, int b0, int stride, const cplx<R> (&v)[RAD])
-{
-    if constexpr (LIN) {
-        const int step = stride + (stride >> 4);
-        cplx<R>* q = line + lds_pad(b0);
-#pragma unroll
-        for (int i = 0; i < RAD; i++) q[i * step] = v[i];
-    } else {
-#pragma unroll
-        for (int i = 0; i < RAD; i++) line[lds_pad(b0 + i * stride)] = v[i];
-    }
-}
-
-// Stage twiddles held in registers across a stage's barrier: only while a
-// thread's share stays within 32 VGPRs (K (R - 1) <= 16 complex64 or 8
-// complex128 values), else they are fetched after it.
-template <typename R, int E, int RAD>
-constexpr bool kTwEarly = ((E + RAD - 1) / RAD) * (RAD - 1) * (int)sizeof(R) <= 64;
-
-// One in-place Stockham stage out of LDS (LIN: both the read stride L / R and
-// the write stride ls are multiples of 16).
-template <typename R, int E, int RAD, bool LIN>
-__device__ __forceinline__ void stage_impl(const PassDesc& p, cplx<R>* lds, int tid, int s)
-{
-    constexpr int K = (E + RAD - 1) / RAD;
-    constexpr bool EARLY = kTwEarly<R, E, RAD>;
-    const int c = tid >> p.tl_shift;
-    const int t = tid & (p.TL - 1);
-    const int nbl = p.L / RAD;
-    const int ls = p.ls[s];
-    cplx<R>* line = lds + c * p.LP;
-    const bool act = c < p.C;  // batch kernel: threads beyond C * TL idle
-    const cplx<R>* tw = reinterpret_cast<const cplx<R>*>(p.stw) + p.twoff[s];
-    cplx<R> v[K][RAD];
-    cplx<R> w[EARLY ? K : 1][RAD - 1];
-    if constexpr (EARLY) {
-        // fetched before the LDS reads: the latency overlaps them and the barrier
-#pragma unroll
-        for (int k = 0; k < K; k++) {
-            const int j = t + k * p.TL;
-            const int g = (int)fdiv((uint32_t)j, p.lsdiv[s]);
-            const int cc = j - g * ls;
-            if (act && j < nbl && ls > 1) {
-#pragma unroll
-                for (int i = 1; i < RAD; i++) w[k][i - 1] = tw[cc * (RAD - 1) + i - 1];
-            }
-        }
-    }
-#pragma unroll
-    for (int k = 0; k < K; k++) {
-        const int j = t + k * p.TL;
-        if (act && j < nbl) lds_gather<R, RAD, LIN>(line, j, nbl, v[k]);
-    }
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < K; k++) {
-        const int j = t + k * p.TL;
-        if (act && j < nbl) {
-            const int g = (int)fdiv((uint32_t)j, p.lsdiv[s]);
-            const int cc = j - g * ls;
-            if (ls > 1) {
-#pragma unroll
-                for (int i = 1; i < RAD; i++) {
-                    if constexpr (EARLY)
-                        v[k][i] = cmul(v[k][i], w[k][i - 1]);
-                    else
-                        v[k][i] = cmul(v[k][i], tw[cc * (RAD - 1) + i - 1]);
-                }
-            }
-            Dft<RAD, R>::run(v[k]);
-            lds_scatter<R, RAD, LIN>(line, g * RAD * ls + cc, ls, v[k]);
-        }
-    }
-    __syncthreads();
-}
-
-template <typename R, int E, int RAD>
-__device__ __forceinline__ void stage(const PassDesc& p, cplx<R>* lds, int tid, int s)
-{
-    if (sizeof(R) == 4 && ((p.L / RAD) & 15) == 0 && (p.ls[s] & 15) == 0)
-        stage_impl<R, E, RAD, true>(p, lds, tid, s);
+    if constexpr (NT)
+        store_nt<R>(d, v);
     else
-        stage_impl<R, E, RAD, false>(p, lds, tid, s);
+        *d = v;
 }
 
-template <typename R, bool ALLRAD, int E>
-__device__ __forceinline__ void run_stages(const PassDesc& p, cplx<R>* lds, int tid, int s0, int s1)
+// Results y[i nbl + j] of butterfly j of the last stage: fused four-step
+// twiddle, scale, Bluestein products, conjugation, store.
+template <typename R, int RAD, bool REAL, bool NT>
+__device__ __forceinline__ void store_butterfly(const PassDesc& p, cplx<R> (&v)[RAD], int j, int nbl, cplx<R>* dst,
+                                                uint32_t l0, int64_t gbase)
 {
-    for (int s = s0; s < s1; s++) {
-        switch (p.radix[s]) {
-            case 2: stage<R, E, 2>(p, lds, tid, s); break;
-            case 4: stage<R, E, 4>(p, lds, tid, s); break;
-            case 8: stage<R, E, 8>(p, lds, tid, s); break;
-            case 16: stage<R, E, 16>(p, lds, tid, s); break;
-            default:
-                if constexpr (ALLRAD) {
-                    switch (p.radix[s]) {
-                        case 3: stage<R, E, 3>(p, lds, tid, s); break;
-                        case 5: stage<R, E, 5>(p, lds, tid, s); break;
-                        case 6: stage<R, E, 6>(p, lds, tid, s); break;
-                        case 7: stage<R, E, 7>(p, lds, tid, s); break;
-                        case 9: stage<R, E, 9>(p, lds, tid, s); break;
-                        case 10: stage<R, E, 10>(p, lds, tid, s); break;
-                        case 11: stage<R, E, 11>(p, lds, tid, s); break;
-                        case 12: stage<R, E, 12>(p, lds, tid, s); break;
-                        case 13: stage<R, E, 13>(p, lds, tid, s); break;
-                        default: break;
-                    }
-                }
-                break;
-        }
-    }
-}
-
-// Real-packed recombine (R2C post-processing) straight from LDS to HBM:
-// bins k and L-k of the N = 2L real transform from Z_k, Z_{L-k}
-// (core/kernels/non_dft/real_packed/packed_rdft_common.h:19-60).
-template <typename R>
-__device__ __forceinline__ void r2c_recombine_store(const PassDesc& p, const TileIo& io, const cplx<R>* lds, int64_t l_base, int tid)
-{
-    const int c = tid >> p.tl_shift;
-    const int t = tid & (p.TL - 1);
-    const SlotLine sl = slot_line(p, io, l_base, c);
-    if (!sl.live) return;
-    LineIdx li = line_index(p, io, sl.l);
-    const cplx<R>* line = lds + c * p.LP;
-    cplx<R>* dst = reinterpret_cast<cplx<R>*>(io.out) + li.ooff;
-    const cplx<R>* rtw = reinterpret_cast<const cplx<R>*>(p.rtw);
-    const int L = p.L;
-    const R half = R(0.5);
-    for (int k = t; k <= L / 2; k += p.TL) {
-        cplx<R> zk = line[lds_pad(k == 0 ? 0 : k)];
-        cplx<R> zm = line[lds_pad(k == 0 ? 0 : L - k)];
-        cplx<R> w = rtw[k];
-        R sum_re = zk.x + zm.x, diff_im = zk.y - zm.y;
-        R ra_re = zk.y + zm.y, ra_im = zm.x - zk.x;
-        // rot = (0.5 w) * (ra_re + i ra_im)
-        R rot_re = half * (w.x * ra_re - w.y * ra_im);
-        R rot_im = half * (w.x * ra_im + w.y * ra_re);
-        R h_re = half * sum_re, h_im = half * diff_im;
-        cplx<R> xk = {h_re + rot_re, h_im + rot_im};
-        cplx<R> xm = {h_re - rot_re, rot_im - h_im};
-        if (k == 0) {
-            xk = {zk.x + zk.y, R(0)};
-            xm = {zk.x - zk.y, R(0)};
-        }
-        if (p.flags & kScale) {
-            xk = cscale(xk, R(sizeof(R) == 4 ? p.scale_f : p.scale_d));
-            xm = cscale(xm, R(sizeof(R) == 4 ? p.scale_f : p.scale_d));
-        }
-        dst[(int64_t)k * p.oes] = xk;
-        if (k != L - k) dst[(int64_t)(L - k) * p.oes] = xm;
-    }
-}
-
-template <typename R, int E>
-__device__ __forceinline__ void store_tile(const PassDesc& p, const TileIo& io, const cplx<R>* lds, int64_t l_base, int tid)
-{
-    const bool col = (p.flags & kOutCol) != 0;
-    const int c = col ? (tid & (p.C - 1)) : (tid >> p.tl_shift);
-    const int t = col ? (tid >> p.c_shift) : (tid & (p.TL - 1));
-    const SlotLine sl = slot_line(p, io, l_base, c);
-    if (!sl.live) return;
-    LineIdx li = line_index(p, io, sl.l);
-    const cplx<R>* line = lds + c * p.LP;
-    cplx<R> v[E];
+    if (!REAL && (p.flags & kTw4)) {
+        // w_N^(l0 e), e = i*nbl + j: two table products, then an FP64
+        // recurrence over i
+        cplx<double> wc = tw4_root(p, (int64_t)l0 * j);
+        const cplx<double> ws = tw4_root(p, (int64_t)l0 * nbl);
 #pragma unroll
-    for (int k = 0; k < E; k++) {
-        const int e = t + k * p.TL;
-        if (e < p.nvalid_out) v[k] = line[lds_pad(e)];
-    }
-    if (p.flags & kTw4) {
-        // w^(l0 e) for e = t + k TL: two table products, then an FP64
-        // recurrence over k
-        cplx<double> wc = tw4_root(p, (int64_t)li.l0 * t);
-        const cplx<double> ws = tw4_root(p, (int64_t)li.l0 * p.TL);
-#pragma unroll
-        for (int k = 0; k < E; k++) {
-            const int e = t + k * p.TL;
-            if (e < p.nvalid_out) {
-                cplx<double> vd = {double(v[k].x), double(v[k].y)};
-                vd = cmul(vd, wc);
-                v[k] = {R(vd.x), R(vd.y)};
-            }
+        for (int i = 0; i < RAD; i++) {
+            cplx<double> vd = {double(v[i].x), double(v[i].y)};
+            vd = cmul(vd, wc);
+            v[i] = {R(vd.x), R(vd.y)};
             wc = cmul(wc, ws);
         }
     }
     if (p.flags & kScale) {
-        const R s = R(sizeof(R) == 4 ? p.scale_f : p.scale_d);
+        const R sc = R(sizeof(R) == 4 ? p.scale_f : p.scale_d);
 #pragma unroll
-        for (int k = 0; k < E; k++) v[k] = cscale(v[k], s);
+        for (int i = 0; i < RAD; i++) v[i] = cscale(v[i], sc);
+    }
+    if (!REAL && (p.flags & (kSpecOut | kChirpOut))) {
+        // multi-pass Bluestein: Z = conj(A) * spec after the first M-point
+        // transform; conj(chirp) * W after the second (stored for g < n only)
+#pragma unroll
+        for (int i = 0; i < RAD; i++) {
+            const int64_t g = gbase + (int64_t)(i * nbl + j) * p.gout[3];
+            if (p.flags & kSpecOut) {
+                v[i] = cmul(cconj(v[i]), reinterpret_cast<const cplx<R>*>(p.spec)[g]);
+            } else if (g < p.nchirp) {
+                v[i] = cmul(cconj(reinterpret_cast<const cplx<R>*>(p.chirp)[g]), v[i]);
+            }
+        }
     }
     if (p.flags & kConjOut) {
 #pragma unroll
-        for (int k = 0; k < E; k++) v[k].y = -v[k].y;
+        for (int i = 0; i < RAD; i++) v[i].y = -v[i].y;
     }
-    if (p.flags & kRealPart) {
-        R* dst = reinterpret_cast<R*>(io.out) + li.ooff;
+    if constexpr (REAL) {
+        R* d = reinterpret_cast<R*>(dst);
+        if (p.flags & kRealOut) {
+            R* q = d + (int64_t)(2 * j) * p.oes;
+            const int64_t step = (int64_t)(2 * nbl) * p.oes;
 #pragma unroll
-        for (int k = 0; k < E; k++) {
-            const int e = t + k * p.TL;
-            if (e < p.nvalid_out) dst[(int64_t)e * p.oes] = v[k].x;
+            for (int i = 0; i < RAD; i++) store_pair<R>(q + i * step, p.oes, v[i]);
+            return;
+        }
+        if (p.flags & kRealPart) {
+#pragma unroll
+            for (int i = 0; i < RAD; i++) d[(int64_t)(i * nbl + j) * p.oes] = v[i].x;
+            return;
+        }
+        // promoted real input: only bins 0..n/2 are stored
+        const int nvo = p.nvalid_out;
+#pragma unroll
+        for (int i = 0; i < RAD; i++) {
+            const int e = i * nbl + j;
+            if (e < nvo) dst[(int64_t)e * p.oes] = v[i];
         }
         return;
     }
-    if (p.flags & kRealOut) {
-        // C2R: element j is (x[2j], x[2j+1]); stored conjugated-domain value
-        // was already flipped back by kConjOut.
-        R* dst = reinterpret_cast<R*>(io.out) + li.ooff;
+    if (p.flags & kChirpOut) {
 #pragma unroll
-        for (int k = 0; k < E; k++) {
-            const int e = t + k * p.TL;
-            if (e < p.nvalid_out) {
-                dst[(int64_t)(2 * e) * p.oes] = v[k].x;
-                dst[(int64_t)(2 * e + 1) * p.oes] = v[k].y;
+        for (int i = 0; i < RAD; i++) {
+            const int e = i * nbl + j;
+            if (gbase + (int64_t)e * p.gout[3] < p.nchirp) dst[(int64_t)e * p.oes] = v[i];
+        }
+        return;
+    }
+    cplx<R>* q = dst + (int64_t)j * p.oes;
+    const int64_t step = (int64_t)nbl * p.oes;
+#pragma unroll
+    for (int i = 0; i < RAD; i++) put<R, NT>(q + i * step, v[i]);
+}
+
+// Stage 0: load, DFT, twiddle, write digit 0 (lanes contiguous).
+template <typename R, int RAD>
+__device__ __forceinline__ void first_to_lds(const PassDesc& p, cplx<R>* line, int j, cplx<R> (&v)[RAD])
+{
+    cplx<R> w[RAD - 1];
+    load_twiddles<R, RAD>(stage_tw<R>(p, 0), (uint32_t)j, p.nbl[0], w);
+    Dft<RAD, R>::run(v);
+    apply_twiddles<R, RAD>(v, w);
+    const int step = p.lst[0];
+#pragma unroll
+    for (int i = 0; i < RAD; i++) line[j + i * step] = v[i];
+}
+
+template <typename R, int RAD, bool REAL>
+__device__ __forceinline__ void first_stage(const PassDesc& p, cplx<R>* line, int t, const cplx<R>* src, int64_t gbase)
+{
+    const int nbl = p.nbl[0];
+#pragma unroll 1
+    for (int j = t; j < nbl; j += p.TL) {
+        cplx<R> v[RAD];
+        load_butterfly<R, RAD, REAL>(p, src, j, gbase, v);
+        first_to_lds<R, RAD>(p, line, j, v);
+    }
+}
+
+template <typename R, int RAD>
+__device__ __forceinline__ void last_from_lds(const PassDesc& p, const cplx<R>* line, int j, cplx<R> (&v)[RAD])
+{
+    const cplx<R>* q = line + last_base(p, j);
+#pragma unroll
+    for (int i = 0; i < RAD; i++) v[i] = q[i];
+    Dft<RAD, R>::run(v);
+}
+
+template <typename R, int RAD, bool REAL, bool NT>
+__device__ __forceinline__ void last_stage(const PassDesc& p, const cplx<R>* line, int t, cplx<R>* dst, uint32_t l0,
+                                           int64_t gbase)
+{
+    // small radices: several butterflies at a time, for the LDS reads in flight
+    constexpr int U = RAD <= 3 ? 4 : RAD <= 5 ? 2 : 1;
+    const int nbl = p.nbl[p.nst - 1];
+#pragma unroll 1
+    for (int j = t; j < nbl; j += U * p.TL) {
+        cplx<R> v[U][RAD];
+#pragma unroll
+        for (int u = 0; u < U; u++)
+            if (u == 0 || j + u * p.TL < nbl) last_from_lds<R, RAD>(p, line, j + u * p.TL, v[u]);
+#pragma unroll
+        for (int u = 0; u < U; u++)
+            if (u == 0 || j + u * p.TL < nbl)
+                store_butterfly<R, RAD, REAL, NT>(p, v[u], j + u * p.TL, nbl, dst, l0, gbase);
+    }
+}
+
+// One-stage lengths (L <= 16): load, DFT, store, no LDS.
+template <typename R, int RAD, bool REAL, bool NT>
+__device__ __forceinline__ void single_stage(const PassDesc& p, const cplx<R>* src, cplx<R>* dst, uint32_t l0,
+                                             int64_t gin, int64_t gout)
+{
+    cplx<R> v[RAD];
+    load_butterfly<R, RAD, REAL>(p, src, 0, gin, v);
+    Dft<RAD, R>::run(v);
+    store_butterfly<R, RAD, REAL, NT>(p, v, 0, 1, dst, l0, gout);
+}
+
+// ---------------------------------------------------------------------------
+// Real-packed transforms (core/kernels/non_dft/real_packed/packed_rdft_common.h:19-60).
+// Bin k and its mirror L - k of the L-point complex transform belong to legs
+// i and R-1-i of butterflies j and nbl - j, so one thread that holds both
+// butterflies recombines (R2C) or separates (C2R) them in registers: no LDS
+// round trip, no further barrier.  Butterflies 0 and nbl/2 are their own
+// mirrors; lane 0 takes them both, so nbl butterflies are (nbl + 1) / 2 items.
+// The planner gives that stage a radix of at most 10 (11 and 13, for lengths
+// that have no other, run in a kernel of their own): the pair's registers set
+// the whole kernel's VGPR count.
+// ---------------------------------------------------------------------------
+
+// Slot i of an item: the bins (k, L - k) that it pairs.  An ordinary lane pairs
+// v[i] with u[R-1-i].  Lane 0 pairs v[i] with v[R-i] in slots 1.., then u[q]
+// with u[R-1-q]; slot 0 is bin 0 (with L), and bin L/2, its own mirror, stands
+// apart: v[R/2] when R is even, the middle leg of u when it is odd.
+template <int RAD>
+struct PairSlots {
+    static constexpr int U0 = (RAD + 1) / 2;  // first slot of u's pairs in lane 0
+    static __device__ __forceinline__ int bin(int i, int j, int nbl)
+    {
+        if (i < U0) return i * nbl + j;
+        return j == 0 ? (i - U0) * nbl + (nbl >> 1) : i * nbl + j;
+    }
+};
+
+template <typename R>
+__device__ __forceinline__ cplx<R> pick(bool first, cplx<R> a, cplx<R> b)
+{
+    return {first ? a.x : b.x, first ? a.y : b.y};
+}
+
+template <typename R, int RAD>
+__device__ __forceinline__ void r2c_last_stage(const PassDesc& p, const cplx<R>* line, int t, cplx<R>* dst,
+                                               const cplx<R>* src)
+{
+    using PS = PairSlots<RAD>;
+    const int nbl = p.nbl[p.nst - 1], L = p.L;
+    const bool even = (nbl & 1) == 0;
+    const cplx<R>* rtw = reinterpret_cast<const cplx<R>*>(p.rtw);
+    const R half = R(0.5);
+    const R sc = (p.flags & kScale) ? R(sizeof(R) == 4 ? p.scale_f : p.scale_d) : R(1);
+#pragma unroll 1
+    for (int j = t; 2 * j < nbl; j += p.TL) {
+        cplx<R> v[RAD], u[RAD];
+        if (p.nst == 1) {
+            if (j != 0) return;  // one butterfly
+            load_butterfly<R, RAD, true>(p, src, 0, 0, v);
+            Dft<RAD, R>::run(v);
+#pragma unroll
+            for (int i = 0; i < RAD; i++) u[i] = v[i];
+        } else {
+            last_from_lds<R, RAD>(p, line, j, v);
+            last_from_lds<R, RAD>(p, line, j == 0 ? nbl >> 1 : nbl - j, u);
+        }
+        const bool z = j == 0;
+#pragma unroll
+        for (int i = 0; i < RAD; i++) {
+            const int k = PS::bin(i, j, nbl);
+            cplx<R> zk = v[i], zm = u[RAD - 1 - i];
+            if (i < PS::U0) {
+                zm = pick<R>(z, v[(RAD - i) % RAD], zm);
+            } else {
+                zk = pick<R>(z, u[i - PS::U0], zk);
+                zm = pick<R>(z, u[RAD - 1 - (i - PS::U0)], zm);
             }
+            const cplx<R> w = rtw[k];
+            const R sum_re = zk.x + zm.x, diff_im = zk.y - zm.y;
+            const R ra_re = zk.y + zm.y, ra_im = zm.x - zk.x;
+            // rot = (0.5 w) * (ra_re + i ra_im)
+            const R rot_re = half * (w.x * ra_re - w.y * ra_im);
+            const R rot_im = half * (w.x * ra_im + w.y * ra_re);
+            const R h_re = half * sum_re, h_im = half * diff_im;
+            cplx<R> xk = {h_re + rot_re, h_im + rot_im};
+            cplx<R> xm = {h_re - rot_re, rot_im - h_im};
+            if (i == 0 && z) {
+                xk = {zk.x + zk.y, R(0)};
+                xm = {zk.x - zk.y, R(0)};
+            }
+            if (i < PS::U0 || !z || even) {
+                dst[(int64_t)k * p.oes] = cscale(xk, sc);
+                dst[(int64_t)(L - k) * p.oes] = cscale(xm, sc);
+            }
+            // four twiddles in flight at a time (all RAD would cost a wave per SIMD)
+            if ((i & 3) == 3) __builtin_amdgcn_sched_barrier(0);
         }
-        return;
+        if (z && (L & 1) == 0) {
+            // X_{L/2} = conj(Z_{L/2})
+            const cplx<R> h = (RAD & 1) == 0 ? v[RAD / 2] : u[RAD / 2];
+            dst[(int64_t)(L >> 1) * p.oes] = cscale(cconj(h), sc);
+        }
     }
-    cplx<R>* dst = reinterpret_cast<cplx<R>*>(io.out) + li.ooff;
+}
+
+// Z_k = E_k + i O_k,  E_k = X_k + conj(X_{L-k}),
+// O_k = (X_k - conj(X_{L-k})) exp(+2 pi i k / 2L), and the mirror Z_{L-k};
+// conjugated, so the forward stages compute the inverse transform.
+template <typename R>
+__device__ __forceinline__ void separate(cplx<R> xk, cplx<R> xm, cplx<R> w, cplx<R>& zk, cplx<R>& zm)
+{
+    const cplx<R> ek = {xk.x + xm.x, xk.y - xm.y};
+    const cplx<R> dk = {xk.x - xm.x, xk.y + xm.y};
+    const cplx<R> ok = cmul(dk, cconj(w));
+    zk = {ek.x - ok.y, -(ek.y + ok.x)};
+    // L-k side: E = conj(ek), O = (X_{L-k} - conj(X_k)) * (-w)
+    const cplx<R> dm = {xm.x - xk.x, xm.y + xk.y};
+    const cplx<R> om = cmul(dm, cplx<R>{-w.x, -w.y});
+    zm = {ek.x - om.y, ek.y - om.x};
+}
+
+template <typename R, int RAD>
+__device__ __forceinline__ void c2r_first_stage(const PassDesc& p, cplx<R>* line, int t, const cplx<R>* src,
+                                                cplx<R>* dst)
+{
+    using PS = PairSlots<RAD>;
+    const int nbl = p.nbl[0], L = p.L;
+    const bool even = (nbl & 1) == 0;
+    const cplx<R>* rtw = reinterpret_cast<const cplx<R>*>(p.rtw);
+#pragma unroll 1
+    for (int j = t; 2 * j < nbl; j += p.TL) {
+        const bool z = j == 0;
+        cplx<R> a[RAD], b[RAD], h = {R(0), R(0)};
+        // (an odd nbl has no butterfly nbl/2: lane 0 reads in range and drops it)
 #pragma unroll
-    for (int k = 0; k < E; k++) {
-        const int e = t + k * p.TL;
-        if (e < p.nvalid_out) dst[(int64_t)e * p.oes] = v[k];
+        for (int i = 0; i < RAD; i++) {
+            const int k = PS::bin(i, j, nbl);
+            a[i] = src[(int64_t)k * p.ies];
+            b[i] = src[(int64_t)(L - k) * p.ies];
+        }
+        if (z && (L & 1) == 0) h = src[(int64_t)(L >> 1) * p.ies];
+#pragma unroll
+        for (int i = 0; i < RAD; i++) {
+            cplx<R> zk, zm;
+            separate<R>(a[i], b[i], rtw[PS::bin(i, j, nbl)], zk, zm);
+            a[i] = zk;
+            b[i] = zm;
+            if ((i & 3) == 3) __builtin_amdgcn_sched_barrier(0);
+        }
+        h = {h.x + h.x, h.y + h.y};  // conj(Z_{L/2}) = 2 X_{L/2}
+        // slots back to the legs of butterflies j (v) and nbl - j (u), or 0 and nbl/2
+        cplx<R> v[RAD], u[RAD];
+#pragma unroll
+        for (int i = 0; i < RAD; i++) {
+            // v[i] is slot i's k side; lane 0's upper legs are the mirror sides of slots R - i
+            v[i] = i < PS::U0 ? a[i] : pick<R>(z, i == RAD - i ? h : b[RAD - i], a[i]);
+            // u[r] is slot R-1-r's mirror side; in lane 0 u[q] / u[R-1-q] are slot U0 + q's two sides
+            constexpr int NU = RAD - PS::U0;  // pairs of u in lane 0
+            const cplx<R> lane0 = i < NU ? a[PS::U0 + (i < NU ? i : 0)]
+                                  : RAD - 1 - i < NU ? b[PS::U0 + (RAD - 1 - i < NU ? RAD - 1 - i : 0)]
+                                                     : h;
+            u[i] = pick<R>(z, lane0, b[RAD - 1 - i]);
+        }
+        if (p.nst == 1) {
+            if (j != 0) return;  // one butterfly
+            Dft<RAD, R>::run(v);
+            store_butterfly<R, RAD, true, false>(p, v, 0, 1, dst, 0, 0);
+            return;
+        }
+        first_to_lds<R, RAD>(p, line, j, v);
+        __builtin_amdgcn_sched_barrier(0);
+        if (!z || even) first_to_lds<R, RAD>(p, line, z ? nbl >> 1 : nbl - j, u);
     }
 }
 
@@ -496,309 +718,151 @@ __device__ __forceinline__ uint32_t tile_of_block(const PassDesc& p)
     return tile;
 }
 
-// ---------------------------------------------------------------------------
-// Register-direct first and last stages (complex in / complex or real-pair
-// out, no real-packed step).  Stage 0 (ls = 1) of butterfly j reads
-// x[i*nbl + j], i < R -- coalesced across j -- so a thread loads exactly its
-// butterflies' operands from HBM, runs the DFT and writes y[j*R + i] to LDS.
-// The last stage (ls = nbl, one group) writes y[i*nbl + j] straight to HBM
-// with the fused four-step twiddle, scale and conjugation.  This drops the
-// LDS round trip and barrier of a staged load and of a staged store.
-// (c, t) is the side's thread mapping (row or column).
-// ---------------------------------------------------------------------------
-template <typename R>
-struct LineIo {
-    const cplx<R>* src;
-    cplx<R>* dst;
-    uint32_t l0;
-    bool live_in, live_out;
-};
-
-// Element e of a line whose element 0 has sequence index gbase, as loaded:
-// with kChirpIn, (conjugated if backward) x * chirp[g] for g < nchirp and 0
-// beyond (the input holds only nchirp elements); else x for e < nvalid_in.
-template <typename R>
-__device__ __forceinline__ cplx<R> load_elem(const PassDesc& p, const cplx<R>* src, int e, int64_t gbase)
+// Length-1 lines: the transform is the identity.
+template <typename R, bool REAL>
+__device__ __forceinline__ void identity_line(const PassDesc& p, const cplx<R>* src, cplx<R>* dst, uint32_t l0,
+                                              int64_t gin, int64_t gout)
 {
-    cplx<R> v = {R(0), R(0)};
-    if (p.flags & kChirpIn) {
-        const int64_t g = gbase + (int64_t)e * p.gin[3];
-        if (g < p.nchirp) {
-            v = src[(int64_t)e * p.ies];
-            if (p.flags & kConjIn) v.y = -v.y;
-            v = cmul(v, reinterpret_cast<const cplx<R>*>(p.chirp)[g]);
-        }
-    } else if (e < p.nvalid_in) {
-        v = src[(int64_t)e * p.ies];
-    }
-    return v;
-}
-
-template <typename R, int E, int RAD>
-__device__ __forceinline__ void first_stage_direct(const PassDesc& p, cplx<R>* lds, int c, int t, const cplx<R>* src,
-                                                   bool live, int64_t gbase)
-{
-    constexpr int K = (E + RAD - 1) / RAD;
-    const int nbl = p.L / RAD;
-    cplx<R> v[K][RAD];
-#pragma unroll
-    for (int k = 0; k < K; k++) {
-        const int j = t + k * p.TL;
-        if (live && j < nbl) {
-#pragma unroll
-            for (int i = 0; i < RAD; i++) v[k][i] = load_elem<R>(p, src, i * nbl + j, gbase);
-        }
-    }
-    cplx<R>* line = lds + c * p.LP;
-    // (with kChirpIn the conjugation happened before the chirp product)
-    const bool cj = (p.flags & (kConjIn | kChirpIn)) == kConjIn;
-#pragma unroll
-    for (int k = 0; k < K; k++) {
-        const int j = t + k * p.TL;
-        if (live && j < nbl) {
-            if (cj) {
-#pragma unroll
-                for (int i = 0; i < RAD; i++) v[k][i].y = -v[k][i].y;
-            }
-            Dft<RAD, R>::run(v[k]);
-#pragma unroll
-            for (int i = 0; i < RAD; i++) line[lds_pad(j * RAD + i)] = v[k][i];
-        }
-    }
-}
-
-// Output side of the last stage for one butterfly: element e = i*nbl + j.
-template <typename R, int RAD>
-__device__ __forceinline__ void store_butterfly(const PassDesc& p, cplx<R>* v, int j, int nbl, cplx<R>* dst,
-                                                uint32_t l0, int64_t gbase)
-{
-    if (p.flags & kTw4) {
-        // w_N^(l0 e), e = i*nbl + j: two table products, then an FP64
-        // recurrence over i
-        cplx<double> wc = tw4_root(p, (int64_t)l0 * j);
-        const cplx<double> ws = tw4_root(p, (int64_t)l0 * nbl);
-#pragma unroll
-        for (int i = 0; i < RAD; i++) {
-            cplx<double> vd = {double(v[i].x), double(v[i].y)};
-            vd = cmul(vd, wc);
-            v[i] = {R(vd.x), R(vd.y)};
-            wc = cmul(wc, ws);
-        }
-    }
-    if (p.flags & kScale) {
-        const R sc = R(sizeof(R) == 4 ? p.scale_f : p.scale_d);
-#pragma unroll
-        for (int i = 0; i < RAD; i++) v[i] = cscale(v[i], sc);
-    }
-    if (p.flags & (kSpecOut | kChirpOut)) {
-        // multi-pass Bluestein: Z = conj(A) * spec after the first M-point
-        // transform; conj(chirp) * W after the second (stored for g < n only)
-#pragma unroll
-        for (int i = 0; i < RAD; i++) {
-            const int64_t g = gbase + (int64_t)(i * nbl + j) * p.gout[3];
-            if (p.flags & kSpecOut) {
-                v[i] = cmul(cconj(v[i]), reinterpret_cast<const cplx<R>*>(p.spec)[g]);
-            } else if (g < p.nchirp) {
-                v[i] = cmul(cconj(reinterpret_cast<const cplx<R>*>(p.chirp)[g]), v[i]);
-            }
-        }
-    }
-    if (p.flags & kConjOut) {
-#pragma unroll
-        for (int i = 0; i < RAD; i++) v[i].y = -v[i].y;
-    }
-    if (p.flags & kChirpOut) {
-#pragma unroll
-        for (int i = 0; i < RAD; i++) {
-            const int e = i * nbl + j;
-            if (gbase + (int64_t)e * p.gout[3] < p.nchirp) dst[(int64_t)e * p.oes] = v[i];
-        }
-        return;
-    }
-    const int nvo = p.nvalid_out;
-    if (p.flags & kRealOut) {
+    cplx<R> v[1];
+    if constexpr (REAL) {
+        // real-packed with L = 1: (x0, x1) <-> bins 0 and 1
+        const R* s = reinterpret_cast<const R*>(src);
         R* d = reinterpret_cast<R*>(dst);
-#pragma unroll
-        for (int i = 0; i < RAD; i++) {
-            const int e = i * nbl + j;
-            if (e < nvo) {
-                d[(int64_t)(2 * e) * p.oes] = v[i].x;
-                d[(int64_t)(2 * e + 1) * p.oes] = v[i].y;
-            }
+        const R sc = (p.flags & kScale) ? R(sizeof(R) == 4 ? p.scale_f : p.scale_d) : R(1);
+        if (p.flags & kR2CPost) {
+            v[0] = load_pair<R>(s, p.ies);
+            dst[0] = {(v[0].x + v[0].y) * sc, R(0)};
+            dst[p.oes] = {(v[0].x - v[0].y) * sc, R(0)};
+        } else if (p.flags & kC2RPre) {
+            const cplx<R> a = src[0], b = src[p.ies];
+            cplx<R> zk, zm;
+            separate<R>(a, b, cplx<R>{R(1), R(0)}, zk, zm);
+            v[0] = zk;
+            store_butterfly<R, 1, true, false>(p, v, 0, 1, dst, 0, 0);
+        } else if (p.flags & kRealPromote) {
+            dst[0] = {s[0] * sc, R(0)};
+        } else {
+            d[0] = src[0].x * sc;  // kHermIn | kRealPart
         }
-        return;
-    }
-#pragma unroll
-    for (int i = 0; i < RAD; i++) {
-        const int e = i * nbl + j;
-        if (e < nvo) dst[(int64_t)e * p.oes] = v[i];
+    } else {
+        v[0] = src[0];
+        if (p.flags & kConjIn) v[0].y = -v[0].y;
+        store_butterfly<R, 1, false, false>(p, v, 0, 1, dst, l0, gout);
     }
 }
 
-template <typename R, int E, int RAD, bool LIN>
-__device__ __forceinline__ void last_stage_direct_impl(const PassDesc& p, const cplx<R>* lds, int c, int t,
-                                                       cplx<R>* dst, uint32_t l0, bool live, int s, int64_t gbase)
+// Every middle stage begins with the barrier that ends the stage before it.
+template <typename R, bool ALLRAD, bool DIT>
+__device__ __forceinline__ void mid_stage_any(const PassDesc& p, cplx<R>* line, int t, int s, bool live,
+                                              bool wave_local)
 {
-    constexpr int K = (E + RAD - 1) / RAD;
-    const int nbl = p.L / RAD;  // = ls of the last stage; g = 0, cc = j
-    const cplx<R>* line = lds + c * p.LP;
-    cplx<R> v[K][RAD];
-#pragma unroll
-    for (int k = 0; k < K; k++) {
-        const int j = t + k * p.TL;
-        if (live && j < nbl) lds_gather<R, RAD, LIN>(line, j, nbl, v[k]);
-    }
-    const cplx<R>* tw = reinterpret_cast<const cplx<R>*>(p.stw) + p.twoff[s];
-#pragma unroll
-    for (int k = 0; k < K; k++) {
-        const int j = t + k * p.TL;
-        if (live && j < nbl) {
-            if (nbl > 1 && s > 0) {
-                const cplx<R>* w = tw + j * (RAD - 1);
-#pragma unroll
-                for (int i = 1; i < RAD; i++) v[k][i] = cmul(v[k][i], w[i - 1]);
-            }
-            Dft<RAD, R>::run(v[k]);
-            store_butterfly<R, RAD>(p, v[k], j, nbl, dst, l0, gbase);
-        }
-    }
+    FFTZ_RADIX_SWITCH(p.radix[s], ALLRAD, (mid_stage<R, RAD, DIT>(p, line, t, s, live, wave_local)))
 }
 
-template <typename R, int E, int RAD>
-__device__ __forceinline__ void last_stage_direct(const PassDesc& p, const cplx<R>* lds, int c, int t, cplx<R>* dst,
-                                                  uint32_t l0, bool live, int s, int64_t gbase)
-{
-    if (sizeof(R) == 4 && ((p.L / RAD) & 15) == 0)
-        last_stage_direct_impl<R, E, RAD, true>(p, lds, c, t, dst, l0, live, s, gbase);
-    else
-        last_stage_direct_impl<R, E, RAD, false>(p, lds, c, t, dst, l0, live, s, gbase);
-}
+// Forms of the generic pass kernel: complex on both sides; a real side, with
+// pair stages of radix <= 10; the same with pair stages of radix 11 or 13.
+enum RealForm : int { kRealNone = 0, kRealPair = 1, kRealWide = 2 };
 
-// One-stage lengths (L <= 16): load, DFT, store, no LDS.
-template <typename R, int E, int RAD>
-__device__ __forceinline__ void single_stage_direct(const PassDesc& p, int t, const cplx<R>* src, cplx<R>* dst,
-                                                    uint32_t l0, bool live, int64_t gin, int64_t gout)
+// One tile: C lines, threads (c, t) per side's mapping -- row (a wavefront
+// walks along a line) or column (it walks the same element of adjacent lines).
+// REAL passes carry the real-packed and promoted forms and are row-mapped.
+template <typename R, bool ALLRAD, int REALK, bool NT>
+__device__ __forceinline__ void pass_body(const PassDesc& p, const TileIo& io, cplx<R>* lds, int64_t l_base, int tid)
 {
-    if (!live || t != 0) return;
-    cplx<R> v[RAD];
-    const bool cj = (p.flags & (kConjIn | kChirpIn)) == kConjIn;
-#pragma unroll
-    for (int i = 0; i < RAD; i++) {
-        v[i] = load_elem<R>(p, src, i, gin);
-        if (cj) v[i].y = -v[i].y;
-    }
-    Dft<RAD, R>::run(v);
-    store_butterfly<R, RAD>(p, v, 0, 1, dst, l0, gout);
-}
-
-#define FFTZ_RADIX_SWITCH(r, ALLRAD, CALL)                 \
-    switch (r) {                                           \
-        case 2: { constexpr int RAD = 2; CALL; } break;    \
-        case 4: { constexpr int RAD = 4; CALL; } break;    \
-        case 8: { constexpr int RAD = 8; CALL; } break;    \
-        case 16: { constexpr int RAD = 16; CALL; } break;  \
-        default:                                           \
-            if constexpr (ALLRAD) {                        \
-                switch (r) {                               \
-                    case 3: { constexpr int RAD = 3; CALL; } break;   \
-                    case 5: { constexpr int RAD = 5; CALL; } break;   \
-                    case 6: { constexpr int RAD = 6; CALL; } break;   \
-                    case 7: { constexpr int RAD = 7; CALL; } break;   \
-                    case 9: { constexpr int RAD = 9; CALL; } break;   \
-                    case 10: { constexpr int RAD = 10; CALL; } break; \
-                    case 11: { constexpr int RAD = 11; CALL; } break; \
-                    case 12: { constexpr int RAD = 12; CALL; } break; \
-                    case 13: { constexpr int RAD = 13; CALL; } break; \
-                    default: break;                        \
-                }                                          \
-            }                                              \
-            break;                                         \
-    }
-
-// Complex-in pass with register-direct first / last stages.
-template <typename R, bool ALLRAD, int E>
-__device__ __forceinline__ void pass_body_direct(const PassDesc& p, const TileIo& io, cplx<R>* lds, int64_t l_base, int tid)
-{
-    const bool in_col = (p.flags & kInCol) != 0, out_col = (p.flags & kOutCol) != 0;
-    const int ci = in_col ? (tid & (p.C - 1)) : (tid >> p.tl_shift);
-    const int ti = in_col ? (tid >> p.c_shift) : (tid & (p.TL - 1));
-    const int co = out_col ? (tid & (p.C - 1)) : (tid >> p.tl_shift);
-    const int to = out_col ? (tid >> p.c_shift) : (tid & (p.TL - 1));
+    constexpr bool REAL = REALK != kRealNone;
+    const bool in_col = !REAL && (p.flags & kInCol) != 0, out_col = !REAL && (p.flags & kOutCol) != 0;
+    const int cr = tid >> p.tl_shift, tr = tid & (p.TL - 1);
+    const int cc = tid & (p.C - 1), tc = tid >> p.c_shift;
+    const int ci = in_col ? cc : cr, ti = in_col ? tc : tr;
+    const int co = out_col ? cc : cr, to = out_col ? tc : tr;
     const SlotLine sli = slot_line(p, io, l_base, ci);
-    const SlotLine slo = slot_line(p, io, l_base, co);
     const bool live_in = ci < p.C && sli.live;
-    const bool live_out = co < p.C && slo.live;
     const cplx<R>* src = nullptr;
-    int64_t gin = 0;
-    if (live_in) {
-        LineIdx li = line_index(p, io, sli.l);
-        src = reinterpret_cast<const cplx<R>*>(io.in) + li.ioff;
-        gin = li.gin;
-    }
     cplx<R>* dst = nullptr;
     uint32_t l0 = 0;
-    int64_t gout = 0;
-    if (live_out) {
-        LineIdx li = line_index(p, io, slo.l);
-        dst = reinterpret_cast<cplx<R>*>(io.out) + li.ooff;
+    int64_t gin = 0, gout = 0;
+    const bool real_in = REAL && (p.flags & (kRealIn | kRealPromote));
+    const bool real_out = REAL && (p.flags & (kRealOut | kRealPart));
+    bool live_out = live_in;
+    if (live_in) {
+        const LineIdx li = line_index(p, io, sli.l);
+        src = real_in ? reinterpret_cast<const cplx<R>*>(reinterpret_cast<const R*>(io.in) + li.ioff)
+                      : reinterpret_cast<const cplx<R>*>(io.in) + li.ioff;
+        dst = real_out ? reinterpret_cast<cplx<R>*>(reinterpret_cast<R*>(io.out) + li.ooff)
+                       : reinterpret_cast<cplx<R>*>(io.out) + li.ooff;
         l0 = li.l0;
+        gin = li.gin;
         gout = li.gout;
     }
     const int S = p.nst;
-    if (S == 1) {
-        // the loading thread stores: use the input-side line for both
-        cplx<R>* d1 = nullptr;
-        uint32_t l01 = 0;
-        int64_t gout1 = 0;
-        if (live_in) {
-            LineIdx li = line_index(p, io, sli.l);
-            d1 = reinterpret_cast<cplx<R>*>(io.out) + li.ooff;
-            l01 = li.l0;
-            gout1 = li.gout;
+    if (S <= 1) {
+        // the loading thread stores
+        if (!live_in || ti != 0) return;
+        if (S == 0) {
+            identity_line<R, REAL>(p, src, dst, l0, gin, gout);
+            return;
         }
-        FFTZ_RADIX_SWITCH(p.radix[0], ALLRAD,
-                          (single_stage_direct<R, E, RAD>(p, ti, src, d1, l01, live_in, gin, gout1)))
+        if constexpr (REAL) {
+            if (p.flags & kR2CPost) {
+                FFTZ_PAIR_SWITCH(p.radix[0], ALLRAD, REALK, (r2c_last_stage<R, RAD>(p, lds, 0, dst, src)))
+                return;
+            }
+            if (p.flags & kC2RPre) {
+                FFTZ_PAIR_SWITCH(p.radix[0], ALLRAD, REALK, (c2r_first_stage<R, RAD>(p, lds, 0, src, dst)))
+                return;
+            }
+        }
+        FFTZ_RADIX_SWITCH(p.radix[0], ALLRAD, (single_stage<R, RAD, REAL, NT>(p, src, dst, l0, gin, gout)))
         return;
     }
-    FFTZ_RADIX_SWITCH(p.radix[0], ALLRAD, (first_stage_direct<R, E, RAD>(p, lds, ci, ti, src, live_in, gin)))
-    __syncthreads();
-    run_stages<R, ALLRAD, E>(p, lds, tid, 1, S - 1);
-    FFTZ_RADIX_SWITCH(p.radix[S - 1], ALLRAD,
-                      (last_stage_direct<R, E, RAD>(p, lds, co, to, dst, l0, live_out, S - 1, gout)))
+    const bool wave_local = p.TL <= 64 && !in_col && !out_col;
+    if (live_in) {
+        cplx<R>* line = lds + ci * p.LP;
+        bool packed = false;
+        if constexpr (REAL) {
+            packed = (p.flags & kC2RPre) != 0;
+            if (packed) {
+                FFTZ_PAIR_SWITCH(p.radix[0], ALLRAD, REALK, (c2r_first_stage<R, RAD>(p, line, ti, src, dst)))
+            }
+        }
+        if (!packed) {
+            FFTZ_RADIX_SWITCH(p.radix[0], ALLRAD, (first_stage<R, RAD, REAL>(p, line, ti, src, gin)))
+        }
+    }
+    for (int s = 1; s + 1 < S; s++)
+        mid_stage_any<R, ALLRAD, false>(p, lds + cr * p.LP, tr, s, cr < p.C, wave_local);
+    stage_sync(wave_local);
+    if (in_col != out_col) {
+        const SlotLine slo = slot_line(p, io, l_base, co);
+        live_out = co < p.C && slo.live;
+        if (live_out) {
+            const LineIdx li = line_index(p, io, slo.l);
+            dst = reinterpret_cast<cplx<R>*>(io.out) + li.ooff;
+            l0 = li.l0;
+            gout = li.gout;
+        }
+    }
+    if (!live_out) return;
+    const cplx<R>* line = lds + co * p.LP;
+    if constexpr (REAL) {
+        if (p.flags & kR2CPost) {
+            FFTZ_PAIR_SWITCH(p.radix[S - 1], ALLRAD, REALK, (r2c_last_stage<R, RAD>(p, line, to, dst, src)))
+            return;
+        }
+    }
+    FFTZ_RADIX_SWITCH(p.radix[S - 1], ALLRAD, (last_stage<R, RAD, REAL, NT>(p, line, to, dst, l0, gout)))
 }
 
-template <typename R, bool ALLRAD, int E>
-__device__ __forceinline__ void pass_body(const PassDesc& p, const TileIo& io, cplx<R>* lds, int64_t l_base, int tid)
-{
-    // (a zero-stage plan, L = 1, is a strided copy: the staged path below)
-    if (!(p.flags & kStagedFlags) && p.nst >= 1) {
-        pass_body_direct<R, ALLRAD, E>(p, io, lds, l_base, tid);
-        return;
-    }
-    load_tile<R, E>(p, io, lds, l_base, tid);
-    __syncthreads();
-    if (p.flags & kC2RPre) {
-        c2r_separate<R>(p, lds, tid);
-        __syncthreads();
-    }
-    run_stages<R, ALLRAD, E>(p, lds, tid, 0, p.nst);
-    if (p.flags & kR2CPost) {
-        r2c_recombine_store<R>(p, io, lds, l_base, tid);
-    } else {
-        store_tile<R, E>(p, io, lds, l_base, tid);
-    }
-}
-
-template <typename R, bool ALLRAD, int E, int MAXT>
-__global__ void __launch_bounds__(MAXT) k_fft_pass(const PassDesc p_arg)
+template <typename R, bool ALLRAD, int REALK, bool NT, int MAXT>
+__global__ void __launch_bounds__(MAXT)
+    __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 && REALK == kRealPair ? 4 : 1))) k_fft_pass(const PassDesc p_arg)
 {
     (void)p_arg;
     const PassDesc& p = kernarg_desc();
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
     cplx<R>* lds = reinterpret_cast<cplx<R>*>(smem_raw);
-    const int tid = threadIdx.x;
     const int64_t l_base = (int64_t)tile_of_block(p) * p.C;
-    pass_body<R, ALLRAD, E>(p, io_of(p), lds, l_base, tid);
+    pass_body<R, ALLRAD, REALK, NT>(p, io_of(p), lds, l_base, threadIdx.x);
 }
 
 // ---------------------------------------------------------------------------
@@ -806,213 +870,145 @@ __global__ void __launch_bounds__(MAXT) k_fft_pass(const PassDesc p_arg)
 // single pass over an M-point LDS tile (M = smooth length >= 2n-1, the
 // reference's get_extended_length, core/common/bluestein_utils.c:39-70):
 //   a = x * conj(B) zero-padded to M     (load)
-//   A = FFT_M(a)                         (stages)
-//   Z = conj(A) * conj(FFT_M(B)) / M      (in LDS)
-//   W = FFT_M(Z) = conj(IFFT_M(A * FFT_M(B)) / M)
+//   A = FFT_M(a)                         (stages 0 .. S-1)
+//   Z = conj(A) * conj(FFT_M(B)) / M      (in registers)
+//   W = FFT_M(Z) = conj(IFFT_M(A * FFT_M(B)) / M)   (stages S-1 .. 0)
 //   X = conj(B * W)                       (store)
 // which is core/solvers/complex/bluestein_solver_dft.c:137-234 with its five
 // sweeps (pre_mul, memset, FFT, mul, IFFT, post_mul) in one HBM round trip.
+// The first transform leaves its digits in output order and the second runs
+// the stages backwards, so nothing is reordered between them and the last
+// stage of the first, the product and the first stage of the second share one
+// butterfly's registers: 2 S - 2 LDS exchanges for the two transforms.
 // ---------------------------------------------------------------------------
-template <typename R, bool ALLRAD, int E>
-__device__ __forceinline__ void bluestein_body(const PassDesc& p, const TileIo& io, cplx<R>* lds, int64_t l_base, int tid)
+template <typename R, int RAD>
+__device__ __forceinline__ void bs_first(const PassDesc& p, cplx<R>* line, int t, const cplx<R>* src)
 {
-    const int c = tid >> p.tl_shift;
-    const int t = tid & (p.TL - 1);
-    const SlotLine sl = slot_line(p, io, l_base, c);
-    const bool live = sl.live;
-    LineIdx li = {0, 0, 0};
-    if (live) li = line_index(p, io, sl.l);
-    cplx<R>* line = lds + c * p.LP;
-    const cplx<R>* chirp = reinterpret_cast<const cplx<R>*>(p.chirp);
-    const cplx<R>* spec = reinterpret_cast<const cplx<R>*>(p.spec);
-    const int n = p.nvalid_in;
-    const int M = p.L;
-    if (live) {
-        const cplx<R>* src = reinterpret_cast<const cplx<R>*>(io.in) + li.ioff;
-        for (int e = t; e < M; e += p.TL) {
-            cplx<R> a = {R(0), R(0)};
-            if (e < n) {
-                cplx<R> x = src[(int64_t)e * p.ies];
-                if (p.flags & kConjIn) x.y = -x.y;
-                a = cmul(x, chirp[e]);
-            }
-            line[lds_pad(e)] = a;
-        }
-    }
-    __syncthreads();
-    run_stages<R, ALLRAD, E>(p, lds, tid, 0, p.nst);
-    if (c < p.C) {
-        for (int e = t; e < M; e += p.TL) {
-            cplx<R> a = line[lds_pad(e)];
-            line[lds_pad(e)] = cmul(cconj(a), spec[e]);
-        }
-    }
-    __syncthreads();
-    run_stages<R, ALLRAD, E>(p, lds, tid, 0, p.nst);
-    if (live) {
-        cplx<R>* dst = reinterpret_cast<cplx<R>*>(io.out) + li.ooff;
-        for (int k = t; k < n; k += p.TL) {
-            cplx<R> w = line[lds_pad(k)];
-            cplx<R> b = cconj(chirp[k]);
-            cplx<R> y = cmul(b, w);  // B * W
-            if (!(p.flags & kConjOut)) y.y = -y.y;  // forward result is conj(B W)
-            dst[(int64_t)k * p.oes] = y;
-        }
-    }
-}
-
-// Register-direct Bluestein stages (M-point plan with at least two stages):
-//   bs_first:  stage 0 of FFT_M(a) on operands a_e = x_e conj(B_e) (e < n,
-//              zero beyond), loaded straight from HBM;
-//   bs_spec:   last stage of FFT_M(a); each thread rewrites exactly the
-//              positions it read with conj(A_e) * spec_e (no barrier needed);
-//   bs_final:  last stage of the second FFT_M, X_k = conj(B_k W_k) (forward),
-//              stored straight to HBM for k < n.
-template <typename R, int E, int RAD>
-__device__ __forceinline__ void bs_first(const PassDesc& p, cplx<R>* lds, int c, int t, const cplx<R>* src, bool live)
-{
-    constexpr int K = (E + RAD - 1) / RAD;
-    const int nbl = p.L / RAD;
+    const int nbl = p.nbl[0];
     const int n = p.nvalid_in;
     const cplx<R>* chirp = reinterpret_cast<const cplx<R>*>(p.chirp);
     const bool cj = (p.flags & kConjIn) != 0;
-    cplx<R> v[K][RAD];
-#pragma unroll
-    for (int k = 0; k < K; k++) {
-        const int j = t + k * p.TL;
-        if (live && j < nbl) {
+#pragma unroll 1
+    for (int j = t; j < nbl; j += p.TL) {
+        cplx<R> v[RAD];
+        if (p.flags & (kRealPromote | kHermIn)) {
 #pragma unroll
             for (int i = 0; i < RAD; i++) {
                 const int e = i * nbl + j;
-                v[k][i] = {R(0), R(0)};
+                v[i] = {R(0), R(0)};
                 if (e < n) {
-                    cplx<R> x;
                     if (p.flags & kRealPromote) {
-                        x = {reinterpret_cast<const R*>(src)[(int64_t)e * p.ies], R(0)};
-                    } else if (p.flags & kHermIn) {
-                        const int m = 2 * e <= n ? e : n - e;
-                        x = src[(int64_t)m * p.ies];
-                        if (2 * e > n) x.y = -x.y;
+                        v[i] = {reinterpret_cast<const R*>(src)[(int64_t)e * p.ies], R(0)};
                     } else {
-                        x = src[(int64_t)e * p.ies];
+                        const bool up = 2 * e > n;
+                        v[i] = src[(int64_t)(up ? n - e : e) * p.ies];
+                        if (up) v[i].y = -v[i].y;
                     }
-                    if (cj) x.y = -x.y;
-                    v[k][i] = cmul(x, chirp[e]);
+                    if (cj) v[i].y = -v[i].y;
+                    v[i] = cmul(v[i], chirp[e]);
                 }
             }
-        }
-    }
-    cplx<R>* line = lds + c * p.LP;
+        } else {
+            // at most (R + 1) / 2 legs hold data (n <= (M + 1) / 2)
+            constexpr int H = (RAD + 1) / 2;
+            const cplx<R>* q = src + (int64_t)j * p.ies;
+            const int64_t step = (int64_t)nbl * p.ies;
 #pragma unroll
-    for (int k = 0; k < K; k++) {
-        const int j = t + k * p.TL;
-        if (live && j < nbl) {
-            Dft<RAD, R>::run(v[k]);
+            for (int i = 0; i < RAD; i++) v[i] = {R(0), R(0)};
 #pragma unroll
-            for (int i = 0; i < RAD; i++) line[lds_pad(j * RAD + i)] = v[k][i];
-        }
-    }
-}
-
-template <typename R, int E, int RAD, bool LIN>
-__device__ __forceinline__ void bs_last_common(const PassDesc& p, const cplx<R>* line, int t, bool live, int s,
-                                               cplx<R> (&v)[(E + RAD - 1) / RAD][RAD])
-{
-    constexpr int K = (E + RAD - 1) / RAD;
-    const int nbl = p.L / RAD;
-#pragma unroll
-    for (int k = 0; k < K; k++) {
-        const int j = t + k * p.TL;
-        if (live && j < nbl) lds_gather<R, RAD, LIN>(line, j, nbl, v[k]);
-    }
-    const cplx<R>* tw = reinterpret_cast<const cplx<R>*>(p.stw) + p.twoff[s];
-#pragma unroll
-    for (int k = 0; k < K; k++) {
-        const int j = t + k * p.TL;
-        if (live && j < nbl) {
-            if (nbl > 1) {
-                const cplx<R>* w = tw + j * (RAD - 1);
-#pragma unroll
-                for (int i = 1; i < RAD; i++) v[k][i] = cmul(v[k][i], w[i - 1]);
-            }
-            Dft<RAD, R>::run(v[k]);
-        }
-    }
-}
-
-template <typename R, int E, int RAD, bool LIN>
-__device__ __forceinline__ void bs_spec_impl(const PassDesc& p, cplx<R>* lds, int c, int t, bool live, int s)
-{
-    constexpr int K = (E + RAD - 1) / RAD;
-    const int nbl = p.L / RAD;
-    cplx<R>* line = lds + c * p.LP;
-    cplx<R> v[K][RAD];
-    bs_last_common<R, E, RAD, LIN>(p, line, t, live, s, v);
-    const cplx<R>* spec = reinterpret_cast<const cplx<R>*>(p.spec);
-#pragma unroll
-    for (int k = 0; k < K; k++) {
-        const int j = t + k * p.TL;
-        if (live && j < nbl) {
-#pragma unroll
-            for (int i = 0; i < RAD; i++) v[k][i] = cmul(cconj(v[k][i]), spec[i * nbl + j]);
-            lds_scatter<R, RAD, LIN>(line, j, nbl, v[k]);
-        }
-    }
-}
-
-template <typename R, int E, int RAD>
-__device__ __forceinline__ void bs_spec(const PassDesc& p, cplx<R>* lds, int c, int t, bool live, int s)
-{
-    if (sizeof(R) == 4 && ((p.L / RAD) & 15) == 0)
-        bs_spec_impl<R, E, RAD, true>(p, lds, c, t, live, s);
-    else
-        bs_spec_impl<R, E, RAD, false>(p, lds, c, t, live, s);
-}
-
-template <typename R, int E, int RAD, bool LIN>
-__device__ __forceinline__ void bs_final_impl(const PassDesc& p, const cplx<R>* lds, int c, int t, cplx<R>* dst,
-                                              bool live, int s)
-{
-    constexpr int K = (E + RAD - 1) / RAD;
-    const int nbl = p.L / RAD;
-    const int n = p.nvalid_out;
-    const cplx<R>* line = lds + c * p.LP;
-    cplx<R> v[K][RAD];
-    bs_last_common<R, E, RAD, LIN>(p, line, t, live, s, v);
-    const cplx<R>* chirp = reinterpret_cast<const cplx<R>*>(p.chirp);
-    const bool fwd = !(p.flags & kConjOut);
-#pragma unroll
-    for (int k = 0; k < K; k++) {
-        const int j = t + k * p.TL;
-        if (live && j < nbl) {
-#pragma unroll
-            for (int i = 0; i < RAD; i++) {
+            for (int i = 0; i < H; i++) {
                 const int e = i * nbl + j;
                 if (e < n) {
-                    cplx<R> y = cmul(cconj(chirp[e]), v[k][i]);  // B * W
-                    if (fwd) y.y = -y.y;                          // forward result is conj(B W)
-                    if (p.flags & kRealPart)
-                        reinterpret_cast<R*>(dst)[(int64_t)e * p.oes] = y.x;
-                    else
-                        dst[(int64_t)e * p.oes] = y;
+                    v[i] = q[i * step];
+                    if (cj) v[i].y = -v[i].y;
+                    v[i] = cmul(v[i], chirp[e]);
                 }
             }
         }
+        first_to_lds<R, RAD>(p, line, j, v);
     }
 }
 
-template <typename R, int E, int RAD>
-__device__ __forceinline__ void bs_final(const PassDesc& p, const cplx<R>* lds, int c, int t, cplx<R>* dst, bool live,
-                                         int s)
+template <typename R, int RAD>
+__device__ __forceinline__ void bs_center(const PassDesc& p, cplx<R>* line, int t, bool live, bool wave_local)
 {
-    if (sizeof(R) == 4 && ((p.L / RAD) & 15) == 0)
-        bs_final_impl<R, E, RAD, true>(p, lds, c, t, dst, live, s);
-    else
-        bs_final_impl<R, E, RAD, false>(p, lds, c, t, dst, live, s);
+    const int full = p.nbl[p.nst - 1], nbl = live ? full : 0;
+    const cplx<R>* spec = reinterpret_cast<const cplx<R>*>(p.spec);
+    int j = t, base = 0;
+    cplx<R> w[RAD];
+    auto fetch = [&]() {
+        if (j < nbl) {
+            base = last_base(p, j);
+#pragma unroll
+            for (int i = 0; i < RAD; i++) w[i] = spec[(uint32_t)(i * full + j)];
+        }
+    };
+    fetch();
+    stage_sync(wave_local);
+#pragma unroll 1
+    while (j < nbl) {
+        cplx<R>* q = line + base;
+        cplx<R> v[RAD];
+#pragma unroll
+        for (int i = 0; i < RAD; i++) v[i] = q[i];
+        Dft<RAD, R>::run(v);
+#pragma unroll
+        for (int i = 0; i < RAD; i++) v[i] = cmul(cconj(v[i]), w[i]);
+        Dft<RAD, R>::run(v);
+#pragma unroll
+        for (int i = 0; i < RAD; i++) q[i] = v[i];
+        j += p.TL;
+        fetch();
+    }
 }
 
-template <typename R, bool ALLRAD, int E>
-__device__ __forceinline__ void bluestein_body_direct(const PassDesc& p, const TileIo& io, cplx<R>* lds, int64_t l_base, int tid)
+template <typename R, int RAD, bool NT>
+__device__ __forceinline__ void bs_final(const PassDesc& p, const cplx<R>* line, int t, cplx<R>* dst, bool live,
+                                         bool wave_local)
+{
+    const int full = p.nbl[0], nbl = live ? full : 0, step = p.lst[0];
+    const int n = p.nvalid_out;
+    const cplx<R>* chirp = reinterpret_cast<const cplx<R>*>(p.chirp);
+    const cplx<R>* tw = stage_tw<R>(p, 0);
+    const bool fwd = !(p.flags & kConjOut);
+    const bool part = (p.flags & kRealPart) != 0;
+    constexpr int H = (RAD + 1) / 2;  // outputs beyond n <= (M + 1) / 2 are not wanted
+    int j = t;
+    cplx<R> w[RAD - 1];
+    if (j < nbl) load_twiddles<R, RAD>(tw, (uint32_t)j, full, w);
+    stage_sync(wave_local);
+#pragma unroll 1
+    while (j < nbl) {
+        cplx<R> v[RAD];
+#pragma unroll
+        for (int i = 0; i < RAD; i++) v[i] = line[j + i * step];
+        apply_twiddles<R, RAD>(v, w);
+        Dft<RAD, R>::run(v);
+#pragma unroll
+        for (int i = 0; i < H; i++) {
+            const int e = i * full + j;
+            if (e < n) {
+                v[i] = cmul(cconj(chirp[e]), v[i]);  // B * W
+                if (fwd) v[i].y = -v[i].y;            // forward result is conj(B W)
+            }
+        }
+        if (part) {
+            R* d = reinterpret_cast<R*>(dst);
+#pragma unroll
+            for (int i = 0; i < H; i++)
+                if (i * full + j < n) d[(int64_t)(i * full + j) * p.oes] = v[i].x;
+        } else {
+#pragma unroll
+            for (int i = 0; i < H; i++)
+                if (i * full + j < n) put<R, NT>(dst + (int64_t)(i * full + j) * p.oes, v[i]);
+        }
+        j += p.TL;
+        if (j < nbl) load_twiddles<R, RAD>(tw, (uint32_t)j, full, w);
+    }
+}
+
+template <typename R, bool ALLRAD, bool NT>
+__device__ __forceinline__ void bluestein_body(const PassDesc& p, const TileIo& io, cplx<R>* lds, int64_t l_base, int tid)
 {
     const int c = tid >> p.tl_shift;
     const int t = tid & (p.TL - 1);
@@ -1031,53 +1027,38 @@ __device__ __forceinline__ void bluestein_body_direct(const PassDesc& p, const T
                                     : reinterpret_cast<cplx<R>*>(io.out) + li.ooff;
     }
     const int S = p.nst;
-    FFTZ_RADIX_SWITCH(p.radix[0], ALLRAD, (bs_first<R, E, RAD>(p, lds, c, t, src, live)))
-    __syncthreads();
-    run_stages<R, ALLRAD, E>(p, lds, tid, 1, S - 1);
-    FFTZ_RADIX_SWITCH(p.radix[S - 1], ALLRAD, (bs_spec<R, E, RAD>(p, lds, c, t, live, S - 1)))
-    __syncthreads();
-    run_stages<R, ALLRAD, E>(p, lds, tid, 0, S - 1);
-    FFTZ_RADIX_SWITCH(p.radix[S - 1], ALLRAD, (bs_final<R, E, RAD>(p, lds, c, t, dst, live, S - 1)))
+    const bool wave_local = p.TL <= 64;
+    cplx<R>* line = lds + c * p.LP;
+    if (live) {
+        FFTZ_RADIX_SWITCH(p.radix[0], ALLRAD, (bs_first<R, RAD>(p, line, t, src)))
+    }
+    for (int s = 1; s + 1 < S; s++) mid_stage_any<R, ALLRAD, false>(p, line, t, s, live, wave_local);
+    FFTZ_RADIX_SWITCH(p.radix[S - 1], ALLRAD, (bs_center<R, RAD>(p, line, t, live, wave_local)))
+    for (int s = S - 2; s >= 1; s--) mid_stage_any<R, ALLRAD, true>(p, line, t, s, live, wave_local);
+    FFTZ_RADIX_SWITCH(p.radix[0], ALLRAD, (bs_final<R, RAD, NT>(p, line, t, dst, live, wave_local)))
 }
 
-template <typename R, bool ALLRAD, int E, int MAXT>
+template <typename R, bool ALLRAD, bool NT, int MAXT>
 __global__ void __launch_bounds__(MAXT) k_bluestein(const PassDesc p_arg)
 {
     (void)p_arg;
     const PassDesc& p = kernarg_desc();
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
     cplx<R>* lds = reinterpret_cast<cplx<R>*>(smem_raw);
-    const TileIo io = io_of(p);
-    if (p.nst >= 2)
-        bluestein_body_direct<R, ALLRAD, E>(p, io, lds, (int64_t)blockIdx.x * p.C, threadIdx.x);
-    else
-        bluestein_body<R, ALLRAD, E>(p, io, lds, (int64_t)blockIdx.x * p.C, threadIdx.x);
-}
-
-// Length-1 items of an uneven batch: the transform is the identity (the
-// backward direction's two conjugations cancel).
-template <typename R>
-__device__ __forceinline__ void batch_identity(const PassDesc& p, const TileIo& io, int64_t l_base, int tid)
-{
-    const int c = tid >> p.tl_shift;
-    const SlotLine sl = slot_line(p, io, l_base, c);
-    if (c >= p.C || !sl.live || (tid & (p.TL - 1)) != 0) return;
-    const LineIdx li = line_index(p, io, sl.l);
-    reinterpret_cast<cplx<R>*>(io.out)[li.ooff] = reinterpret_cast<const cplx<R>*>(io.in)[li.ioff];
+    bluestein_body<R, ALLRAD, NT>(p, io_of(p), lds, (int64_t)blockIdx.x * p.C, threadIdx.x);
 }
 
 // ---------------------------------------------------------------------------
 // Uneven batches in one persistent launch.  A device work queue lists tiles
 // (size class, first line, line count, offsets); each workgroup takes the
-// next tile from an atomic counter, copies the size class's pass descriptor
-// into LDS, patches the tile's buffers in, and runs the same pass or
-// Bluestein body as the single-size kernels.  Tiles are sorted by cost on
-// the host, largest first.  The arithmetic of a tile does not depend on the
-// workgroup that runs it, so results are bitwise identical run to run.
+// next tile from an atomic counter, reads the size class's pass descriptor in
+// place, and runs the same pass or Bluestein body as the single-size kernels.
+// Tiles are sorted by cost on the host, largest first.  The arithmetic of a
+// tile does not depend on the workgroup that runs it, so results are bitwise
+// identical run to run.
 // ---------------------------------------------------------------------------
-template <typename R, int E, int MAXT>
-__global__ void __launch_bounds__(MAXT) __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 4 : 2)))
-k_batch(const BatchArgs a)
+template <typename R, int MAXT>
+__global__ void __launch_bounds__(MAXT) k_batch(const BatchArgs a)
 {
     // dynamic LDS: [tile index | tile data].  The tile index is made uniform
     // with readfirstlane, and the queue entry and its size class's descriptor
@@ -1105,15 +1086,10 @@ k_batch(const BatchArgs a)
         const int C = p.C;
         // a queue entry covers one or more rounds of C lines
         for (int64_t lb = 0; lb < io.nlines; lb += C) {
-            // only the register-direct bodies: batch items are plain complex
-            // transforms (no staged real-packed steps), and a Bluestein
-            // extended length (M >= 33) always has two or more stages
             if (blue)
-                bluestein_body_direct<R, true, E>(p, io, lds, lb, tid);
-            else if (p.nst >= 1)
-                pass_body_direct<R, true, E>(p, io, lds, lb, tid);
+                bluestein_body<R, true, true>(p, io, lds, lb, tid);
             else
-                batch_identity<R>(p, io, lb, tid);
+                pass_body<R, true, kRealNone, true>(p, io, lds, lb, tid);
             __syncthreads();
         }
         if (tid == 0) s_tile = nxt;
@@ -1122,19 +1098,33 @@ k_batch(const BatchArgs a)
 }
 
 // ---------------------------------------------------------------------------
-// Launch table: precision x radix set x elements per thread x block limit.
+// Launch table: precision x radix set x block limit.  The larger block is
+// 1024 threads in complex64 and 512 in complex128, half of that for real passes:
+// they hold a butterfly and its mirror.
 // ---------------------------------------------------------------------------
-template <typename R, bool A, int E, int T>
-inline const void* sym(KernelKind kind)
+template <typename R>
+constexpr int kBigBlock = sizeof(R) == 4 ? 1024 : 512;
+
+template <typename R, bool A, int T>
+inline const void* sym(KernelKind kind, bool nt)
 {
-    return kind == KernelKind::Pass ? (const void*)&k_fft_pass<R, A, E, T> : (const void*)&k_bluestein<R, A, E, T>;
+    constexpr int TR = T > kBigBlock<R> / 2 ? kBigBlock<R> / 2 : T;
+    switch (kind) {
+        case KernelKind::Pass:
+            return nt ? (const void*)&k_fft_pass<R, A, kRealNone, true, T>
+                      : (const void*)&k_fft_pass<R, A, kRealNone, false, T>;
+        case KernelKind::Real: return (const void*)&k_fft_pass<R, A, kRealPair, false, TR>;
+        case KernelKind::RealWide:
+            if constexpr (A) return (const void*)&k_fft_pass<R, A, kRealWide, false, TR>;
+            return nullptr;
+        default: return nt ? (const void*)&k_bluestein<R, A, true, T> : (const void*)&k_bluestein<R, A, false, T>;
+    }
 }
 
 template <typename R, bool A>
-inline const void* sym_et(KernelKind kind, int E, int maxt)
+inline const void* sym_t(KernelKind kind, bool nt, int maxt)
 {
-    if (E == 8) return maxt <= 256 ? sym<R, A, 8, 256>(kind) : sym<R, A, 8, 1024>(kind);
-    return maxt <= 256 ? sym<R, A, 16, 256>(kind) : sym<R, A, 16, 1024>(kind);
+    return maxt <= 256 ? sym<R, A, 256>(kind, nt) : sym<R, A, kBigBlock<R>>(kind, nt);
 }
 
 }  // namespace fftz

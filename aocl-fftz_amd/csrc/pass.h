@@ -46,11 +46,12 @@ enum PassFlags : uint32_t {
     kChirpIn = 1u << 14,   // load: x[g] * chirp[g] for g < nchirp, 0 beyond
     kSpecOut = 1u << 15,   // store: conj(y[g]) * spec[g]
     kChirpOut = 1u << 16,  // store: conj(chirp[g]) * y[g], only g < nchirp
+    kNtStore = 1u << 17,   // results bypass the L2's write-back (whole cache lines)
 };
 // Flags of the multi-pass Bluestein products (generic kernel only).
 constexpr uint32_t kChirpFlags = kChirpIn | kSpecOut | kChirpOut;
-// Flags whose passes stage the tile through LDS before the first stage.
-constexpr uint32_t kStagedFlags = kRealIn | kC2RPre | kR2CPost | kRealPromote | kHermIn | kRealPart;
+// Flags of passes with a real side (their own generic kernel).
+constexpr uint32_t kRealFlags = kRealIn | kRealOut | kC2RPre | kR2CPost | kRealPromote | kHermIn | kRealPart;
 
 // Operand precision of the matrix-core radix-16 pass (kernels_mfma.hip).
 enum MfmaMode : int {
@@ -79,6 +80,23 @@ inline FastDiv make_fastdiv(uint32_t d)
     return f;
 }
 
+// n / d for 0 <= n < 2^14, 1 <= d <= 2^14: one 24-bit multiply and a shift
+// (mul = floor(2^shift / d) + 1 <= 2^15 overshoots 1/d by at most d / 2^shift
+// <= 2^-14 per unit of n, so the quotient is exact and the product fits 2^29).
+struct SmallDiv {
+    uint32_t mul;
+    uint32_t shift;
+};
+
+inline SmallDiv make_smalldiv(uint32_t d)
+{
+    SmallDiv f;
+    f.shift = 14;
+    while ((1u << (f.shift - 14)) < d) f.shift++;
+    f.mul = (uint32_t)((1ull << f.shift) / d) + 1;
+    return f;
+}
+
 struct PassDesc {
     const void* in;
     void* out;
@@ -86,7 +104,7 @@ struct PassDesc {
     const void* tw4;       // four-step twiddles: double2 lo[1<<tw4_lobits] then hi[]
     const void* chirp;     // Bluestein: conj(B_k), k < nvalid (plan precision)
     const void* spec;      // Bluestein: conj(FFT_M(B)) / M (plan precision)
-    const void* rtw;       // real-packed twiddles exp(-2 pi i k / 2L), k <= L/2;
+    const void* rtw;       // real-packed twiddles exp(-2 pi i k / 2L), k < L;
                            // matrix-core pass: its lane-ordered stage twiddles
     int64_t ies, oes;      // element strides along the transform axis
     int64_t ils[3], ols[3];// line strides for line levels l0, l1, l2
@@ -118,9 +136,14 @@ struct PassDesc {
     float scale_f;
     double scale_d;
     int radix[kMaxStages];
-    int ls[kMaxStages];
-    FastDiv lsdiv[kMaxStages];
-    int twoff[kMaxStages];
+    int twoff[kMaxStages];     // stage s's twiddles in stw, in elements
+    // generic kernels (kernels_body.h): a line in LDS as mixed-radix digits
+    int nbl[kMaxStages];       // butterflies of stage s: L / radix[s]
+    int lst[kMaxStages];       // LDS stride of digit s (lst[0] padded)
+    int on[kMaxStages];        // values of the digits between 0 and s
+    SmallDiv mdiv[kMaxStages]; // by lst[s] (s >= 1)
+    SmallDiv odiv[kMaxStages]; // by on[s]
+    SmallDiv rdiv[kMaxStages]; // by radix[s]
 };
 
 // One tile of an uneven batch: `nlines` consecutive transforms of size class
@@ -147,8 +170,9 @@ struct BatchArgs {
     void* out;
 };
 
-// LDS index of element e inside one line: one pad slot every 16 elements so
-// the stride-R writes of the first Stockham stages spread over the banks.
+// LDS index of element e inside one line of the fixed-length and matrix-core
+// kernels: one pad slot every 16 elements so the stride-R writes of the first
+// Stockham stages spread over the banks.
 __host__ __device__ inline int lds_pad(int e) { return e + (e >> 4); }
 
 }  // namespace fftz

@@ -52,12 +52,12 @@ const DeviceInfo& device_info()
         // Allow every kernel to use the full LDS of a workgroup.
         for (int prec : {4, 8})
             for (bool all : {false, true})
-                for (KernelKind k : {KernelKind::Pass, KernelKind::Bluestein})
-                    for (int e : {8, 16})
+                for (KernelKind k : {KernelKind::Pass, KernelKind::Real, KernelKind::RealWide, KernelKind::Bluestein})
+                    for (bool nt : {false, true})
                         for (int t : {256, 1024})
-                            (void)hipFuncSetAttribute(kernel_symbol(k, prec, all, e, t),
-                                                      hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                      (int)info.lds_per_block);
+                            if (const void* f = kernel_symbol(k, prec, all, nt, t))
+                                (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                          (int)info.lds_per_block);
         for (int prec : {4, 8})
             for (int L = 64; L <= 4096; L *= 2)
                 for (int t : {256, 512})
@@ -196,6 +196,24 @@ static bool factor_radices(int L, std::vector<int>& out)
         n /= r;
     }
     std::sort(out.begin(), out.end(), std::greater<int>());
+    // A radix-2 stage costs nearly as much LDS traffic and addressing as any
+    // other: 16 16 16 2 becomes 16 8 8 8 (8192-point complex64 lines).  The
+    // lengths of the fixed kernels keep their plan.
+    if (out.size() >= 3 && out.back() == 2 && !((L & (L - 1)) == 0 && L <= 4096)) {
+        std::vector<int> r = out;
+        const size_t S = r.size();
+        for (size_t i = 0; i + 1 < S && r[S - 1] == 2; i++)
+            for (int f : {4, 3})
+                if (r[S - 1] == 2 && r[i] % f == 0 && r[i] / f >= 3) {
+                    r[i] /= f;
+                    r[S - 1] *= f;
+                }
+        std::sort(r.begin(), r.end(), std::greater<int>());
+        if (std::all_of(r.begin(), r.end(), [](int v) {
+                return std::find(std::begin(kRadices), std::end(kRadices), v) != std::end(kRadices);
+            }))
+            out = r;
+    }
     return (int)out.size() <= kMaxStages;
 }
 
@@ -250,6 +268,42 @@ std::vector<std::vector<int>> radix_orders(int L, int maxn)
     return out;
 }
 
+static int env_int(const char* name, int dflt)
+{
+    const char* v = getenv(name);
+    return v ? atoi(v) : dflt;
+}
+
+static double radix_stage_cost(int r);
+
+// Radices of a real-packed pass: the smallest goes to the stage that holds
+// mirrored butterfly pairs (last for R2C, first for C2R).  Pairs above radix 10
+// would double the kernel's VGPRs, so where the default plan has no smaller
+// radix (16 x 16, 16 x 12, ...) the least-cost order that has one, with one
+// more stage, is taken; products of 11s and 13s have none.
+static std::vector<int> packed_radices(int L, std::vector<int> r, bool c2r)
+{
+    auto least = [](const std::vector<int>& o) { return *std::min_element(o.begin(), o.end()); };
+    if (!r.empty() && least(r) > 10) {
+        std::vector<std::vector<int>> sets = radix_orders(L, 1 << 20);
+        if (L == 16) sets = {{8, 2}, {4, 4}};
+        if (L == 12) sets = {{6, 2}, {4, 3}};
+        double best = 1e300;
+        for (auto& o : sets) {
+            if (least(o) > 10) continue;
+            double c = 0.0;
+            for (int v : o) c += radix_stage_cost(v);
+            if (c < best) {
+                best = c;
+                r = o;
+            }
+        }
+    }
+    std::sort(r.begin(), r.end());
+    if (!c2r) std::reverse(r.begin(), r.end());
+    return r;
+}
+
 static int next_pow2(int64_t v)
 {
     int p = 1;
@@ -288,20 +342,153 @@ struct TableBuilder {
     }
 };
 
-// Stage twiddles for radices r[0..]: per stage, for c < ls, i in [1, R):
-// w_{R ls}^{i c} -- the per-column layout of core/common/twiddle.c:46-66.
-static int64_t stage_twiddles(TableBuilder& tb, int prec, const std::vector<int>& radix, int* twoff, int* ls_out)
+// Stage twiddles of the fixed-length kernels: per stage, for c < ls, i in
+// [1, R): w_{R ls}^{i c} -- the per-column layout of core/common/twiddle.c:46-66.
+static int64_t stage_twiddles(TableBuilder& tb, int prec, const std::vector<int>& radix, int* twoff)
 {
     std::vector<d2> tw;
     int ls = 1;
     for (size_t s = 0; s < radix.size(); s++) {
         const int R = radix[s];
         twoff[s] = (int)tw.size();
-        ls_out[s] = ls;
         for (int c = 0; c < ls; c++)
             for (int i = 1; i < R; i++) tw.push_back(root_fwd((int64_t)i * c, (int64_t)R * ls));
         ls *= R;
     }
+    if (tw.empty()) tw.push_back({1.0, 0.0});
+    return tb.add_complex(tw, prec);
+}
+
+// Threads per line of a generic pass: a power of two in [mint, maxt].  A stage
+// runs ceil(nbl / TL) rounds of TL butterflies and lanes idle in its last one;
+// the work of a choice is the sum over stages of rounds x TL x R x (cost per
+// element).
+//   * Wide enough that neighbouring lanes cover 64 bytes of a line, and a
+//     column tile fills a wavefront (mint).
+//   * At most 16 elements per thread: beyond that too few wavefronts fit next
+//     to the lines' LDS (1,000,000-point complex64, passes of 100: 12 per
+//     thread 97 us, 25 per thread 104 us).  Short complex128 lines may take up
+//     to 32, for at least 15% less work: their registers allow no more than
+//     eight wavefronts per CU in any case (100 x 120 x 144 grid, pass of 100:
+//     25 per thread 16.6 us, 12 per thread 18.7 us).
+//   * Among the widths within 8% of the least work, short lines take the
+//     narrowest (room for more lines) and long ones and pair stages the widest
+//     (more loads in flight per line).
+//   * Where the lines are too few for eight wavefronts per CU (two in
+//     complex128, which holds eight at most), wider, up to 1.6 times the least
+//     work: the launch is latency-bound.
+// lines: how many there are; pair: the stage whose threads take two
+// butterflies at a time, or -1.
+static int line_threads(const std::vector<int>& radix, int L, int mint, int maxt, int pair, int64_t lines, int prec)
+{
+    int widest = 1;
+    for (int r : radix) widest = std::max(widest, next_pow2(L / r));
+    widest = std::min(widest, maxt);
+    auto work = [&](int tl) {
+        double w = 0.0;
+        for (int s = 0; s < (int)radix.size(); s++) {
+            const int r = radix[(size_t)s], per = s == pair ? 2 : 1;
+            const int items = (L / r + per - 1) / per;
+            w += (double)((items + tl - 1) / tl) * tl * per * r * radix_stage_cost(r);
+        }
+        return tl * 16 < L ? 1.15 * w : w;
+    };
+    const int most = prec == 8 && L <= 128 ? 32 : 16;
+    int first = 1;
+    while (first < widest && (first * most < L || first < mint)) first *= 2;
+    double least = 1e300;
+    for (int tl = first; tl <= widest; tl *= 2) least = std::min(least, work(tl));
+    int tl = first;
+    while (work(tl) > 1.08 * least) tl *= 2;
+    if (L >= 1024 || pair >= 0) {
+        tl = widest;
+        while (work(tl) > 1.08 * least) tl /= 2;
+    }
+    const int64_t fill = 64 * (prec == 4 ? 2048 : 512);
+    while (tl < widest && lines * tl < fill && work(tl * 2) <= 1.6 * least) tl *= 2;
+    return tl;
+}
+
+// LDS layout, stage geometry and twiddles of a generic pass (kernels_body.h)
+// of length L = product of radix, TL threads per line: fills the stage
+// fields and the pitch LP of d (at least lp_min, odd) and returns the table's
+// offset.  Row k >= 1, column m of stage s: w_{Rs As}^{k m}, As = the product
+// of the later radices.
+//
+// lst[0] is padded: the digits below digit 0 are dense, so consecutive values
+// of digit 0 would otherwise sit a multiple of the later radices apart and
+// meet in the same LDS banks in the middle and last stages.  The pad is the
+// one of 0..7 with the fewest bank conflicts over the first wavefront's
+// accesses of those stages (16 8-byte or 8 16-byte lanes per LDS cycle, banks
+// of 128 bytes in all), the smallest on ties.
+static int64_t digit_layout(TableBuilder& tb, int prec, const std::vector<int>& radix, int L, int TL, int lp_min,
+                            PassDesc& d)
+{
+    const int S = (int)radix.size();
+    d.nst = S;
+    std::vector<d2> tw;
+    int A = L;
+    for (int s = 0; s < S; s++) {
+        const int R = radix[(size_t)s];
+        d.radix[s] = R;
+        d.nbl[s] = L / R;
+        A /= R;
+        d.lst[s] = A;
+        d.on[s] = s >= 2 ? d.on[s - 1] * radix[(size_t)s - 1] : 1;
+        d.mdiv[s] = make_smalldiv((uint32_t)A);
+        d.odiv[s] = make_smalldiv((uint32_t)d.on[s]);
+        d.rdiv[s] = make_smalldiv((uint32_t)R);
+        d.twoff[s] = (int)tw.size();
+        if (s + 1 < S)
+            for (int k = 1; k < R; k++)
+                for (int m = 0; m < A; m++) tw.push_back(root_fwd((int64_t)k * m, (int64_t)R * A));
+    }
+    int LP = std::max(lp_min, L);
+    if (S >= 2) {
+        const int lanes = prec == 4 ? 16 : 8;  // lanes (and banks, in elements) per LDS cycle
+        const int A0 = d.lst[0];
+        int best = 0;
+        long best_cost = -1;
+        for (int pad = 0; pad < 8; pad++) {
+            const int a0 = A0 + pad;
+            if (pad && radix[0] * a0 > std::max(lp_min, L + radix[0])) break;
+            const int pitch = std::max(lp_min, radix[0] * a0) | 1;
+            long cost = 0;
+            for (int s = 1; s < S; s++) {
+                int bank[16];
+                for (int l0 = 0; l0 < 64; l0 += lanes) {
+                    for (int b = 0; b < lanes; b++) bank[b] = 0;
+                    int worst = 0;
+                    for (int l = l0; l < l0 + lanes; l++) {
+                        const int c = l / std::min(TL, 64), j = l % std::min(TL, 64);
+                        if (j >= d.nbl[s]) continue;
+                        int pos = 0;
+                        if (s + 1 == S) {
+                            int rem = j;
+                            for (int i = 0; i + 2 < S; i++) {
+                                pos += (rem % radix[(size_t)i]) * (i ? d.lst[i] : a0);
+                                rem /= radix[(size_t)i];
+                            }
+                            pos += rem * (S >= 3 ? d.lst[S - 2] : a0);
+                        } else {
+                            const int o = j / d.lst[s], m = j % d.lst[s];
+                            pos = (o / d.on[s]) * a0 + (o % d.on[s]) * radix[(size_t)s] * d.lst[s] + m;
+                        }
+                        worst = std::max(worst, ++bank[(pos + c * pitch) % lanes]);
+                    }
+                    // a middle stage reads and writes, the last only reads
+                    cost += (long)worst * radix[(size_t)s] * (s + 1 == S ? 1 : 2);
+                }
+            }
+            if (best_cost < 0 || cost < best_cost) {
+                best_cost = cost;
+                best = pad;
+            }
+        }
+        d.lst[0] = A0 + best;
+        LP = std::max(LP, radix[0] * d.lst[0]);
+    }
+    d.LP = LP | 1;
     if (tw.empty()) tw.push_back({1.0, 0.0});
     return tb.add_complex(tw, prec);
 }
@@ -346,12 +533,6 @@ struct PassReq {
     int64_t gie = 0, goe = 0;  // element coefficients of the sequence index (kChirpFlags)
     int64_t nchirp = 0;
 };
-
-static int env_int(const char* name, int dflt)
-{
-    const char* v = getenv(name);
-    return v ? atoi(v) : dflt;
-}
 
 // Merge line axes that form one dense run for both input and output.
 static std::vector<LineAxis> merge_axes(std::vector<LineAxis> ax)
@@ -478,49 +659,31 @@ static bool build_pass(Plan* plan, TableBuilder& tb, const PassReq& q, std::stri
     }
     // a tuned radix order for this length (plain passes; the matrix-core
     // pass needs the all-16 plan)
+    const bool r2c = (q.flags & kR2CPost) != 0, c2r = (q.flags & kC2RPre) != 0;
+    if (r2c || c2r) radix = packed_radices(q.L, radix, c2r);
     if (const std::vector<int>* tr = plan->spec.tune.radices(q.L))
-        if (q.kind == KernelKind::Pass && plan->spec.mfma_mode == kMfmaNone && radix_order_ok(q.L, *tr)) radix = *tr;
+        if (q.kind == KernelKind::Pass && plan->spec.mfma_mode == kMfmaNone && radix_order_ok(q.L, *tr) &&
+            !(r2c && tr->back() > 10) && !(c2r && tr->front() > 10))
+            radix = *tr;
     d.nst = (int)radix.size();
     ln.all_radix = false;
     for (size_t s = 0; s < radix.size(); s++) {
         d.radix[s] = radix[s];
         if (radix[s] != 2 && radix[s] != 4 && radix[s] != 8 && radix[s] != 16) ln.all_radix = true;
     }
-    ln.stw_off = stage_twiddles(tb, prec, radix, d.twoff, d.ls);
-    for (int s = 0; s < d.nst; s++) d.lsdiv[s] = make_fastdiv((uint32_t)d.ls[s]);
-
-    // elements per thread: 16 for power-of-two radices; 8 for the mixed
-    // radix variant (fewer live VGPRs) unless that needs > 512 threads/line
-    int E = 16;
-    if (ln.all_radix && next_pow2((q.L + 7) / 8) <= 512) E = 8;
-    // complex128 outside the fixed-kernel range: 8 values per thread keeps
-    // the 1024-thread variant within its 128 VGPRs (16 would spill)
-    const bool fixed_range = q.L >= 64 && q.L <= 4096 && (q.L & (q.L - 1)) == 0;
-    if (prec == 8 && !fixed_range && next_pow2((q.L + 7) / 8) <= 1024) E = 8;
-    {
-        const int e = plan->spec.tune.elems ? plan->spec.tune.elems : env_int("FFTZ_E", 0);
-        if ((e == 8 || e == 16) && next_pow2((q.L + e - 1) / e) <= 1024) E = e;
-    }
-    ln.E = E;
-    // threads per line
-    int TL = next_pow2((q.L + E - 1) / E);
-    if (TL < 1) TL = 1;
-    d.TL = TL;
-    d.tl_shift = ilog2(TL);
-    int need = q.L + q.extra_lds_elems;
-    int LP = lds_pad(need - 1) + 1;
-    if ((LP & 1) == 0) LP++;
-    d.LP = LP;
+    // a tuned number of values per thread
+    const int tuned_e = plan->spec.tune.elems ? plan->spec.tune.elems : env_int("FFTZ_E", 0);
+    const int need = q.L + q.extra_lds_elems;
 
     // fixed-length kernel: power-of-two L in [64, 4096], plain C2C pass
     const bool pow2L = q.L >= 64 && q.L <= 4096 && (q.L & (q.L - 1)) == 0;
-    if ((q.flags & kChirpFlags) && (q.kind != KernelKind::Pass || (q.flags & (kStagedFlags | kRealOut)))) {
-        err = "internal: Bluestein products on a staged pass";
+    if ((q.flags & kChirpFlags) && (q.kind != KernelKind::Pass || (q.flags & kRealFlags))) {
+        err = "internal: Bluestein products on a real pass";
         return false;
     }
-    const bool fixed_ok = q.kind == KernelKind::Pass && pow2L && E == 16 && d.nvalid_in == q.L &&
+    const bool fixed_ok = q.kind == KernelKind::Pass && pow2L && tuned_e != 8 && d.nvalid_in == q.L &&
                           d.nvalid_out == q.L &&
-                          !(q.flags & (kStagedFlags | kRealOut | kChirpFlags)) && env_int("FFTZ_FIXED", 1);
+                          !(q.flags & (kRealFlags | kChirpFlags)) && env_int("FFTZ_FIXED", 1);
     bool plan_match = fixed_ok;
     if (fixed_ok) {
         // the fixed kernels hard-code 16, 16, ..., 2^rem (kernels_fixed.hip)
@@ -531,13 +694,33 @@ static bool build_pass(Plan* plan, TableBuilder& tb, const PassReq& q, std::stri
     }
     // fixed kernels come in 256- and 512-thread variants (512 for wide column
     // tiles of L >= 256)
-    const int tmax = plan_match ? (q.L >= 256 ? 512 : 256) : 1024;
+    const int tbig = (prec == 4 ? 1024 : 512) / ((q.flags & kRealFlags) && q.kind == KernelKind::Pass ? 2 : 1);
+    const int tmax = plan_match ? (q.L >= 256 ? 512 : 256) : tbig;
+    int64_t nl_total = 1;
+    for (auto& a : q.lines) nl_total *= a.n;
+    // threads per line, and the table and layout that go with the kernel
+    int TL;
+    if (plan_match) {
+        TL = q.L / 16;
+        ln.E = 16;
+        ln.stw_off = stage_twiddles(tb, prec, radix, d.twoff);
+        d.LP = (lds_pad(need - 1) + 1) | 1;
+    } else {
+        TL = line_threads(radix, q.L, q.want_in_col || q.want_out_col ? 4 : 64 / esize, tmax,
+                          r2c ? (int)radix.size() - 1 : c2r ? 0 : -1, nl_total, prec);
+        if (tuned_e == 8 || tuned_e == 16) TL = std::min(next_pow2((q.L + tuned_e - 1) / tuned_e), tmax);
+        ln.E = std::max(tuned_e == 8 || tuned_e == 16 ? tuned_e : 1, (q.L + TL - 1) / TL);
+        ln.stw_off = digit_layout(tb, prec, radix, q.L, TL, lds_pad(need - 1) + 1, d);
+    }
+    const int LP = d.LP;
+    d.TL = TL;
+    d.tl_shift = ilog2(TL);
     // matrix-core pass: complex64, L = 16^2 or 16^3 with the plain 16-radix
     // plan, row mapping, no fused twiddle / real-packed step
     const int mm = plan->spec.mfma_mode;
     const bool use_mfma = mm != kMfmaNone && prec == 4 && plan_match && (q.L == 256 || q.L == 4096) &&
                           !q.want_in_col && !q.want_out_col &&
-                          !(q.flags & (kTw4 | kStagedFlags | kRealOut | kChirpFlags));
+                          !(q.flags & (kTw4 | kRealFlags | kChirpFlags));
 
     // line axes: choose l0
     std::vector<LineAxis> ax = merge_axes(q.lines);
@@ -584,14 +767,21 @@ static bool build_pass(Plan* plan, TableBuilder& tb, const PassReq& q, std::stri
         // element-strided row tiles
         while (C * 2 <= cmax && (size_t)(C * 2) * line_bytes <= budget && C * 2 <= n0 && C * 2 * TL <= tmax)
             C *= 2;
+        // fewer than two tiles per CU: narrower ones, down to 16 lines (128- or
+        // 256-byte segments); fewer than one for two CUs: down to four lines
+        while (!plan->spec.tune.col_c &&
+               ((C > 16 && nl_total / C < 2 * dev.cus) || (C > 4 && nl_total / C < dev.cus / 2)))
+            C /= 2;
         if (C < 2) { in_col = false; out_col = false; C = 1; }
     }
     if (!(in_col || out_col) && !use_mfma) {
         const int tgt = plan->spec.tune.row_t ? plan->spec.tune.row_t : env_int("FFTZ_ROW_T", 256);
-        const size_t budget = std::min(lds_cap, (size_t)env_int("FFTZ_ROW_LDS", 64 * 1024));
-        int64_t nl_total = 1;
-        for (auto& a : ax) nl_total *= a.n;
-        while (C * TL < tgt && (size_t)(C * 2) * line_bytes <= budget && C * 2 * TL <= tmax && C < nl_total) C *= 2;
+        const size_t budget = std::min(lds_cap, (size_t)env_int("FFTZ_ROW_LDS", plan_match ? 64 * 1024 : 40 * 1024));
+        // lines per tile: up to tgt threads; beyond a wavefront only while
+        // every CU keeps two tiles
+        while (C * TL < tgt && (size_t)(C * 2) * line_bytes <= budget && C * 2 * TL <= tmax && C < nl_total &&
+               (C * TL < 64 || nl_total / (C * 2) >= 2 * dev.cus || plan->spec.tune.row_t))
+            C *= 2;
     }
     if (C * TL > 1024) {
         err = "tile too large";
@@ -1268,8 +1458,8 @@ static bool plan_real(Plan* plan, TableBuilder& tb, std::vector<AxisSpec> dims, 
     const int64_t nbins = n0 / 2 + 1;
     int64_t rtw_off = -1;
     if (packed) {
-        std::vector<d2> rtw((size_t)(L / 2 + 1));
-        for (int64_t k = 0; k <= L / 2; k++) rtw[(size_t)k] = root_fwd(k, n0);
+        std::vector<d2> rtw((size_t)L);
+        for (int64_t k = 0; k < L; k++) rtw[(size_t)k] = root_fwd(k, n0);
         rtw_off = tb.add_complex(rtw, prec);
     }
     // complex geometry of the half-spectrum side
@@ -1374,7 +1564,7 @@ struct SizeInfo {
 };
 }  // namespace
 
-static bool batch_size_desc(TableBuilder& tb, int prec, int64_t n, int E, int maxt, size_t lds_budget,
+static bool batch_size_desc(TableBuilder& tb, int prec, int64_t n, int maxt, size_t lds_budget,
                             SizeInfo& si, std::string& err)
 {
     si.n = n;
@@ -1389,27 +1579,15 @@ static bool batch_size_desc(TableBuilder& tb, int prec, int64_t n, int E, int ma
         return false;
     }
     d.L = (int)L;
-    d.nst = (int)radix.size();
-    if (si.bluestein && d.nst < 2) {
-        // the batch kernel runs the register-direct Bluestein body only
+    if (si.bluestein && radix.size() < 2) {
         err = "internal: Bluestein batch length " + std::to_string(L) + " with one stage";
         return false;
     }
-    for (size_t s = 0; s < radix.size(); s++) d.radix[s] = radix[s];
-    const int64_t stw = stage_twiddles(tb, prec, radix, d.twoff, d.ls);
-    for (int s = 0; s < d.nst; s++) d.lsdiv[s] = make_fastdiv((uint32_t)d.ls[s]);
-    int TL = next_pow2((L + E - 1) / E);
-    if (TL < 1) TL = 1;
-    if (TL > maxt) {
-        err = "batch length " + std::to_string(L) + " too long for its tile class";
-        return false;
-    }
+    const int TL = line_threads(radix, (int)L, 32 / prec, maxt, -1, INT32_MAX, prec);
+    const int64_t stw = digit_layout(tb, prec, radix, (int)L, TL, lds_pad((int)L - 1) + 1, d);
     d.TL = TL;
     d.tl_shift = ilog2(TL);
-    int LP = lds_pad((int)L - 1) + 1;
-    if ((LP & 1) == 0) LP++;
-    d.LP = LP;
-    const size_t line_bytes = (size_t)LP * 2 * prec;
+    const size_t line_bytes = (size_t)d.LP * 2 * prec;
     if (line_bytes > lds_budget) {
         err = "batch length " + std::to_string(L) + " exceeds LDS";
         return false;
@@ -1456,8 +1634,10 @@ Plan* batch_plan_create(const std::vector<BatchItem>& items, int prec, int dir, 
     const DeviceInfo& dev = device_info();
     const int esize = 2 * prec;
     TableBuilder tb{plan->host_tables};
-    // size classes: small tiles (E = 8, 256 threads, <= 64 KiB LDS, several
-    // workgroups per CU) and large tiles (E = 16, 1024 threads, whole LDS)
+    // size classes: small tiles (256 threads, <= 64 KiB LDS, several
+    // workgroups per CU) and large tiles (whole LDS; 1024 threads, 512 in
+    // complex128)
+    const int big_threads = prec == 4 ? 1024 : 512;
     const size_t static_lds = kBatchHdrBytes;
     const size_t small_budget = (size_t)env_int("FFTZ_BATCH_SMALL_LDS", 64 * 1024);
     const size_t big_budget = dev.lds_per_block - static_lds;
@@ -1494,7 +1674,7 @@ Plan* batch_plan_create(const std::vector<BatchItem>& items, int prec, int dir, 
     // spectrum) are independent: build them on worker threads into separate
     // arenas, then append each arena to the plan's and rebase its offsets.
     {
-        const int cE[3] = {8, 16, 16}, cT[3] = {256, 512, 1024};
+        const int cT[3] = {256, 512, big_threads};
         const size_t cB[3] = {small_budget, medium_budget, big_budget};
         std::vector<std::vector<unsigned char>> arenas(sizes.size());
         std::vector<std::string> errs(sizes.size());
@@ -1505,7 +1685,7 @@ Plan* batch_plan_create(const std::vector<BatchItem>& items, int prec, int dir, 
                 TableBuilder ltb{arenas[i]};
                 SizeInfo& si = sizes[i];
                 const int cls = si.cls;
-                ok[i] = batch_size_desc(ltb, prec, si.n, cE[cls], cT[cls], cB[cls], si, errs[i]) ? 1 : 0;
+                ok[i] = batch_size_desc(ltb, prec, si.n, cT[cls], cB[cls], si, errs[i]) ? 1 : 0;
                 si.cls = cls;
             }
         };
@@ -1574,8 +1754,7 @@ Plan* batch_plan_create(const std::vector<BatchItem>& items, int prec, int dir, 
         auto& tl = tiles[(size_t)c];
         std::stable_sort(tl.begin(), tl.end(), [](const auto& a, const auto& b) { return a.first > b.first; });
         BatchClass bc;
-        bc.E = c == 0 ? 8 : 16;
-        bc.maxt = c == 0 ? 256 : (c == 1 ? 512 : 1024);
+        bc.maxt = c == 0 ? 256 : (c == 1 ? 512 : big_threads);
         bc.ntiles = (int)tl.size();
         size_t lds = 0;
         for (const SizeInfo& si : sizes)
@@ -1629,7 +1808,7 @@ Plan* batch_plan_create(const std::vector<BatchItem>& items, int prec, int dir, 
         return nullptr;
     }
     for (size_t c = 0; c < plan->bclasses.size(); c++)
-        (void)hipFuncSetAttribute(kernel_symbol_batch(prec, plan->bclasses[c].E, plan->bclasses[c].maxt),
+        (void)hipFuncSetAttribute(kernel_symbol_batch(prec, (int)c),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)dev.lds_per_block);
     plan->host_tables.clear();
     plan->host_tables.shrink_to_fit();
@@ -1951,7 +2130,7 @@ static std::string batch_json(const Plan* p)
     os << "],\"classes\":[";
     for (size_t c = 0; c < p->bclasses.size(); c++) {
         const BatchClass& bc = p->bclasses[c];
-        os << (c ? "," : "") << "{\"E\":" << bc.E << ",\"maxt\":" << bc.maxt << ",\"lds\":" << bc.lds_bytes
+        os << (c ? "," : "") << "{\"maxt\":" << bc.maxt << ",\"lds\":" << bc.lds_bytes
            << ",\"grid\":" << bc.grid << ",\"tiles\":[";
         const BatchTile* t = hd ? reinterpret_cast<const BatchTile*>(p->host_tables.data() + bc.tiles_off) : nullptr;
         for (int i = 0; t && i < bc.ntiles; i++)
@@ -1988,8 +2167,6 @@ std::string plan_json(const Plan* p)
            << d.gout[0] << "," << d.gout[1] << "," << d.gout[2] << "," << d.gout[3] << "],\"gin_base\":" << d.gin_base
            << ",\"gout_base\":" << d.gout_base << ",\"radix\":[";
         for (int s = 0; s < d.nst; s++) os << (s ? "," : "") << d.radix[s];
-        os << "],\"ls\":[";
-        for (int s = 0; s < d.nst; s++) os << (s ? "," : "") << d.ls[s];
         os << "]}";
         first = false;
     }
@@ -2097,13 +2274,21 @@ static hipError_t launch_batch(Plan* p, unsigned* counters, const void* in, void
             a.in = in;
             a.out = out;
             void* args[] = {&a};
-            e = hipLaunchKernel(kernel_symbol_batch(p->spec.prec_bytes, bc.E, bc.maxt), dim3(bc.grid),
+            e = hipLaunchKernel(kernel_symbol_batch(p->spec.prec_bytes, (int)c), dim3(bc.grid),
                                 dim3(bc.maxt), args, bc.lds_bytes, stream);
             if (e != hipSuccess) return e;
         }
         if (prof && (e = record_prof(p, stream)) != hipSuccess) return e;
     }
     return hipGetLastError();
+}
+
+static KernelKind pass_kind(const Launch& ln)
+{
+    const PassDesc& d = ln.d;
+    if (ln.kind != KernelKind::Pass || !(d.flags & kRealFlags)) return ln.kind;
+    const int pair = (d.flags & kR2CPost) && d.nst ? d.radix[d.nst - 1] : (d.flags & kC2RPre) && d.nst ? d.radix[0] : 1;
+    return pair > 10 ? KernelKind::RealWide : KernelKind::Real;
 }
 
 static hipError_t launch_all(Plan* p, void* work, unsigned* counters, const void* in, void* out, hipStream_t stream,
@@ -2129,7 +2314,8 @@ static hipError_t launch_all(Plan* p, void* work, unsigned* counters, const void
         void* args[] = {&d, &frag};
         const void* fn = ln.mfma ? kernel_symbol_mfma(ln.mfma, ln.d.L, ln.mfma_nb)
                          : ln.fixed ? kernel_symbol_fixed(p->spec.prec_bytes, ln.d.L, ln.maxt)
-                                    : kernel_symbol(ln.kind, p->spec.prec_bytes, ln.all_radix, ln.E, ln.maxt);
+                                    : kernel_symbol(pass_kind(ln), p->spec.prec_bytes, ln.all_radix,
+                                                    (d.flags & kNtStore) != 0, ln.maxt);
         hipError_t e = hipLaunchKernel(fn, dim3(ln.grid),
                                        dim3(ln.block), args, ln.lds_bytes, stream);
         if (e != hipSuccess) return e;

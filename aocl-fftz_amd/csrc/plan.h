@@ -67,7 +67,7 @@ struct BatchItem {
 
 // A persistent-kernel class of the uneven batch (small or large tiles).
 struct BatchClass {
-    int E = 8, maxt = 256;
+    int maxt = 256;
     uint32_t lds_bytes = 0;
     uint32_t grid = 0;
     int ntiles = 0;
@@ -77,7 +77,7 @@ struct BatchClass {
 struct Launch {
     KernelKind kind = KernelKind::Pass;
     bool all_radix = false;
-    int E = 16;        // complex values per thread per stage
+    int E = 16;        // complex values of a line per thread
     int maxt = 256;    // block-size bound of the kernel variant
     bool fixed = false;  // fixed-length kernel (kernels_fixed.hip)
     int mfma = 0;        // MfmaMode of a matrix-core pass (kernels_mfma.hip)
