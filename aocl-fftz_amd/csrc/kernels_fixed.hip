@@ -264,7 +264,6 @@ __global__ void __launch_bounds__(MAXT) k_fixed_pass(const PassDesc p)
         if (tw4) wc = root((int64_t)lo.l0 * j);
 #pragma unroll
         for (int i = 0; i < RL; i++) {
-            const int e = i * lsL + j;
             cplx<R> y = w[k][i];
             if (tw4) {
                 cplx<double> yd = {double(y.x), double(y.y)};
@@ -274,7 +273,18 @@ __global__ void __launch_bounds__(MAXT) k_fixed_pass(const PassDesc p)
             }
             if (p.flags & kScale) y = cscale(y, R(sizeof(R) == 4 ? p.scale_f : p.scale_d));
             if (p.flags & kConjOut) y.y = -y.y;
-            dst[(int64_t)e * p.oes] = y;
+            w[k][i] = y;
+        }
+        cplx<R>* q = dst + (int64_t)j * p.oes;
+        const int64_t step = (int64_t)lsL * p.oes;
+        if (p.flags & kNtStore) {
+            keep_branch();
+#pragma unroll
+            for (int i = 0; i < RL; i++) store_nt<R>(q + i * step, w[k][i]);
+            keep_branch();
+        } else {
+#pragma unroll
+            for (int i = 0; i < RL; i++) q[i * step] = w[k][i];
         }
     }
 }

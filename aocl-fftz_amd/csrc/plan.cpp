@@ -858,6 +858,19 @@ static bool build_pass(Plan* plan, TableBuilder& tb, const PassReq& q, std::stri
     const bool straddle = in_col && ((q.ies * esize) % 128) != 0;
     if (((out_col && !in_col) || straddle) && tiles >= 64 && env_int("FFTZ_XCD_REMAP", 1)) d.flags |= kXcdRemap;
 
+    // Results in whole 128-byte lines may bypass the L2's write-back; those of
+    // a pass whose output a later launch reads are put back by plan_create.
+    // Lines of 4 KiB and more count as whole (one partial line in 32); one store
+    // has to cover 128 bytes of a row (64-point complex64 lines, 32 bytes: 13 -> 19
+    // us), 256 of a column tile (128: 512^3 R2C's last pass 231 -> 234 us).
+    if (!(q.flags & kRealFlags) && q.out_role == Role::Out) {
+        bool aligned = true;
+        for (int k = out_col ? 1 : 0; k < 3; k++)
+            if (ax[k].n > 1 && (ax[k].os * (int64_t)esize) % 128 != 0) aligned = false;
+        const bool rows = !out_col && q.oes == 1 && TL * esize >= 128 && (aligned || (int64_t)d.nvalid_out * esize >= 4096);
+        const bool cols = out_col && aligned && (q.oes * esize) % 128 == 0 && C * esize >= 256 && n0 % C == 0;
+        if (rows || cols) d.flags |= kNtStore;
+    }
     // expand host-looped axes
     std::vector<int64_t> ioffs{q.in_base}, ooffs{q.out_base}, gis{0}, gos{0};
     // real-side strides count real elements (packed R2C / C2R and the
@@ -2080,6 +2093,11 @@ Plan* plan_create(const ProblemSpec& spec_in, std::string& err, bool dry_run)
         delete plan;
         return nullptr;
     }
+    // results that a later launch reads (N-D passes in place on the output)
+    // stay in the caches
+    for (size_t i = 0; i < plan->launches.size(); i++)
+        for (size_t j = i + 1; j < plan->launches.size(); j++)
+            if (plan->launches[j].in_role == plan->launches[i].out_role) plan->launches[i].d.flags &= ~kNtStore;
     if (dry_run) return plan;
     // upload tables and resolve pointers
     if (!plan->host_tables.empty()) {
