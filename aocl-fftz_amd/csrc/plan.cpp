@@ -761,7 +761,10 @@ static bool build_pass(Plan* plan, TableBuilder& tb, const PassReq& q, std::stri
         d.tl_shift = 4;
     } else if (in_col || out_col) {
         const int cmax = plan->spec.tune.col_c ? plan->spec.tune.col_c : env_int("FFTZ_COL_C", prec == 8 ? 16 : 32);
-        const size_t budget = std::min(lds_cap, (size_t)env_int("FFTZ_COL_LDS", 96 * 1024));
+        // complex128 tiles of the fixed kernels take the whole LDS from 1024
+        // points on: columns of 8 lines 35 us, of 4 lines 40 us (64 MiB each way)
+        const bool whole = plan_match && prec == 8 && q.L >= 1024;
+        const size_t budget = std::min(lds_cap, (size_t)env_int("FFTZ_COL_LDS", whole ? 160 * 1024 : 96 * 1024));
         // a row of n0 lines that C does not divide is tiled raggedly (the
         // last tile of each row partly idle) rather than falling back to
         // element-strided row tiles
@@ -1121,6 +1124,47 @@ static bool split_factors(int64_t N, int64_t fmax, std::vector<int64_t>& f)
     return false;
 }
 
+// Time of a four-step pass over factor f, relative to a first pass of 256 in
+// complex64 (fits to passes over 64 MiB, read and written: 30 us for 256).  A
+// first or middle pass works on columns: its tile has as many lines as the LDS
+// holds, so from 512 points on the segments of a row shrink below 256 bytes
+// (complex128 tiles of 2^k take the whole LDS and hold out longer).  The last
+// pass reads rows and is affected on its store only.  The generic kernel adds
+// by its stages.
+static double pass_cost(int64_t f, bool last, int prec)
+{
+    static const double col[2][6] = {{0.97, 1.0, 1.17, 1.4, 2.3, 4.0}, {0.95, 0.95, 1.12, 1.17, 1.45, 2.3}};  // 128 ..
+    static const double row[2][7] = {{0.8, 0.83, 0.95, 1.03, 1.1, 1.17, 1.35},
+                                     {0.8, 0.8, 0.82, 1.02, 1.02, 1.13, 1.27}};  // 64 .. 4096
+    const double* t = last ? row[prec == 8] : col[prec == 8];
+    const int n = last ? 7 : 6;
+    const double x = std::min(std::max(std::log2((double)f) - (last ? 6.0 : 7.0), 0.0), n - 1.0);
+    const int i = std::min((int)x, n - 2);
+    double c = t[i] + (x - i) * (t[i + 1] - t[i]);
+    std::vector<int> r;
+    if ((f & (f - 1)) != 0 && factor_radices((int)f, r)) c *= r.size() <= 2 ? 1.1 : r.size() == 3 ? 1.12 : 1.3;
+    return c;
+}
+
+// The cheapest two-pass split of N, each factor at most 2048; false when there is none.
+static bool split_two(int64_t N, int prec, std::vector<int64_t>& f, double& cost)
+{
+    cost = 1e300;
+    for (int64_t a = 16; a <= 2048 && a <= N; a++) {
+        const int64_t b = N / a;
+        if (N % a || b < 16 || b > 2048 || !smooth13(a) || !smooth13(b)) continue;
+        // wide generic passes leave one or two lines per tile
+        const int64_t generic = prec == 4 ? 2048 : 1536;
+        if (((a & (a - 1)) && a > generic) || ((b & (b - 1)) && b > generic)) continue;
+        const double c = pass_cost(a, false, prec) + pass_cost(b, true, prec);
+        if (c < cost) {
+            cost = c;
+            f = {a, b};
+        }
+    }
+    return cost < 1e300;
+}
+
 static bool split_ok(int64_t N, const std::vector<int64_t>& f, int64_t fmax)
 {
     if (f.size() < 2 || f.size() > 3) return false;
@@ -1203,10 +1247,28 @@ static bool plan_long_axis(Plan* plan, TableBuilder& tb, const LongAxis& a, std:
     }
     // power-of-two factors last: the final (transposing) pass then runs on
     // the fixed-length kernel
-    if (!use_tuned && !getenv("FFTZ_FACTORS"))
+    if (!use_tuned && !getenv("FFTZ_FACTORS")) {
         std::stable_sort(f.begin(), f.end(), [](int64_t x, int64_t y) {
             return ((x & (x - 1)) != 0) > ((y & (y - 1)) != 0);
         });
+        // two wider passes where they cost clearly less than these (64 MiB in
+        // all: 8 x 2^20 complex64 as 512 x 2048 65 us, as 128 x 128 x 64 75 us;
+        // 9 x 1,000,000 as 1000 x 1000 81 us, as 100 x 100 x 100 98 us), but not
+        // the widest powers of two on data beyond the Infinity Cache, where
+        // segments below a cache line cost more than a third pass (16 x 2^20
+        // there and back 327 against 288 us; complex128 8 x 2^21 583 against 562)
+        double three = 0.0, two = 0.0;
+        bool pow2 = true;
+        for (size_t i = 0; i < f.size(); i++) {
+            three += pass_cost(f[i], i + 1 == f.size(), prec);
+            pow2 = pow2 && (f[i] & (f[i] - 1)) == 0;
+        }
+        int64_t total = N * 2 * prec;
+        for (auto& b : a.batch) total *= b.n;
+        const bool far = pow2 && total > ((int64_t)96 << 20) && N > (prec == 4 ? 1 << 19 : 1 << 20);
+        std::vector<int64_t> g;
+        if (!far && split_two(N, prec, g, two) && two < 0.93 * three) f = g;
+    }
     // dense intermediate: batch axis i at stride N * prod_{j<i} n_j
     std::vector<int64_t> wst(a.batch.size());
     int64_t B = 1;
