@@ -146,19 +146,20 @@ __device__ __forceinline__ int last_base(const PassDesc& p, int j)
 }
 
 // Leg 0 of butterfly j of a middle stage s; m is the index below digit s
-// (the stage's twiddle column).  Only A0 is padded, so the digits between 0
-// and s are one dense run.
+// (the stage's twiddle column).  Digit 0 runs fastest over the lanes: its odd
+// stride spreads them over the LDS banks whatever the later radices are, and
+// neighbouring lanes share a twiddle.
 __device__ __forceinline__ int mid_base(const PassDesc& p, int s, int j, uint32_t& m)
 {
-    const uint32_t o = sdiv((uint32_t)j, p.mdiv[s]);
-    m = (uint32_t)j - __umul24(o, (uint32_t)p.lst[s]);
-    const uint32_t d0 = sdiv(o, p.odiv[s]);
-    const uint32_t r = o - __umul24(d0, (uint32_t)p.on[s]);
-    return (int)(__umul24(d0, (uint32_t)p.lst[0]) + __umul24(r, (uint32_t)(p.radix[s] * p.lst[s])) + m);
+    const uint32_t q = sdiv((uint32_t)j, p.rdiv[0]);
+    const uint32_t d0 = (uint32_t)j - __umul24(q, (uint32_t)p.radix[0]);
+    const uint32_t o = sdiv(q, p.mdiv[s]);
+    m = q - __umul24(o, (uint32_t)p.lst[s]);
+    return (int)(__umul24(d0, (uint32_t)p.lst[0]) + __umul24(o, (uint32_t)(p.radix[s] * p.lst[s])) + m);
 }
 
 // Stage twiddles, one row per output digit k >= 1 and one column per index m
-// below the digit: w_{Rs As}^(k m), so neighbouring lanes read neighbours.
+// below the digit: w_{Rs As}^(k m).
 template <typename R>
 __device__ __forceinline__ const cplx<R>* stage_tw(const PassDesc& p, int s)
 {

@@ -140,9 +140,7 @@ struct PassDesc {
     // generic kernels (kernels_body.h): a line in LDS as mixed-radix digits
     int nbl[kMaxStages];       // butterflies of stage s: L / radix[s]
     int lst[kMaxStages];       // LDS stride of digit s (lst[0] padded)
-    int on[kMaxStages];        // values of the digits between 0 and s
     SmallDiv mdiv[kMaxStages]; // by lst[s] (s >= 1)
-    SmallDiv odiv[kMaxStages]; // by on[s]
     SmallDiv rdiv[kMaxStages]; // by radix[s]
 };
 

@@ -415,9 +415,9 @@ static int line_threads(const std::vector<int>& radix, int L, int mint, int maxt
 // offset.  Row k >= 1, column m of stage s: w_{Rs As}^{k m}, As = the product
 // of the later radices.
 //
-// lst[0] is padded: the digits below digit 0 are dense, so consecutive values
-// of digit 0 would otherwise sit a multiple of the later radices apart and
-// meet in the same LDS banks in the middle and last stages.  The pad is the
+// lst[0] is padded: consecutive lanes of the middle and last stages hold
+// consecutive values of digit 0, which would otherwise sit a multiple of the
+// later radices apart and meet in the same LDS banks.  The pad is the
 // one of 0..7 with the fewest bank conflicts over the first wavefront's
 // accesses of those stages (16 8-byte or 8 16-byte lanes per LDS cycle, banks
 // of 128 bytes in all), the smallest on ties.
@@ -434,9 +434,7 @@ static int64_t digit_layout(TableBuilder& tb, int prec, const std::vector<int>& 
         d.nbl[s] = L / R;
         A /= R;
         d.lst[s] = A;
-        d.on[s] = s >= 2 ? d.on[s - 1] * radix[(size_t)s - 1] : 1;
         d.mdiv[s] = make_smalldiv((uint32_t)A);
-        d.odiv[s] = make_smalldiv((uint32_t)d.on[s]);
         d.rdiv[s] = make_smalldiv((uint32_t)R);
         d.twoff[s] = (int)tw.size();
         if (s + 1 < S)
@@ -471,8 +469,8 @@ static int64_t digit_layout(TableBuilder& tb, int prec, const std::vector<int>& 
                             }
                             pos += rem * (S >= 3 ? d.lst[S - 2] : a0);
                         } else {
-                            const int o = j / d.lst[s], m = j % d.lst[s];
-                            pos = (o / d.on[s]) * a0 + (o % d.on[s]) * radix[(size_t)s] * d.lst[s] + m;
+                            const int q = j / radix[0], o = q / d.lst[s], m = q % d.lst[s];
+                            pos = (j % radix[0]) * a0 + o * radix[(size_t)s] * d.lst[s] + m;
                         }
                         worst = std::max(worst, ++bank[(pos + c * pitch) % lanes]);
                     }
@@ -865,13 +863,15 @@ static bool build_pass(Plan* plan, TableBuilder& tb, const PassReq& q, std::stri
     // a pass whose output a later launch reads are put back by plan_create.
     // Lines of 4 KiB and more count as whole (one partial line in 32); one store
     // has to cover 128 bytes of a row (64-point complex64 lines, 32 bytes: 13 -> 19
-    // us), 256 of a column tile (128: 512^3 R2C's last pass 231 -> 234 us).
+    // us), 256 of a column tile (128: 512^3 R2C's last pass 231 -> 234 us) on
+    // data beyond half of the Infinity Cache, which a reader finds there no more.
     if (!(q.flags & kRealFlags) && q.out_role == Role::Out) {
         bool aligned = true;
         for (int k = out_col ? 1 : 0; k < 3; k++)
             if (ax[k].n > 1 && (ax[k].os * (int64_t)esize) % 128 != 0) aligned = false;
         const bool rows = !out_col && q.oes == 1 && TL * esize >= 128 && (aligned || (int64_t)d.nvalid_out * esize >= 4096);
-        const bool cols = out_col && aligned && (q.oes * esize) % 128 == 0 && C * esize >= 256 && n0 % C == 0;
+        const bool cols = out_col && aligned && (q.oes * esize) % 128 == 0 && C * esize >= 256 && n0 % C == 0 &&
+                          nl * q.L * esize >= ((int64_t)128 << 20);
         if (rows || cols) d.flags |= kNtStore;
     }
     // expand host-looped axes
