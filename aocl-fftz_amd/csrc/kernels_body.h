@@ -125,7 +125,7 @@ __device__ __forceinline__ void stage_sync(bool wave_local)
 
 // ---------------------------------------------------------------------------
 // LDS positions.  A line is kept as mixed-radix digits: position
-// d0 A0 + d1 A1 + ... + d(S-1), As = p.lst[s], where digit s holds the input
+// d0 A0 + d1 A1 + ... + d(S-1), As = p.st[s].lst, where digit s holds the input
 // digit n_s before stage s and the output digit k_s after it (input index
 // n0 L/R0 + n1 L/(R0 R1) + ..., output index k0 + R0 k1 + R0 R1 k2 + ...).
 // Stage s transforms digit s, so it reads and writes the same R_s positions.
@@ -138,11 +138,11 @@ __device__ __forceinline__ int last_base(const PassDesc& p, int j)
     const int S = p.nst;
     uint32_t rem = (uint32_t)j, base = 0;
     for (int s = 0; s + 2 < S; s++) {
-        const uint32_t q = sdiv(rem, p.rdiv[s]);
-        base += __umul24(rem - __umul24(q, (uint32_t)p.radix[s]), (uint32_t)p.lst[s]);
+        const uint32_t q = sdiv(rem, p.st[s].rdiv);
+        base += __umul24(rem - __umul24(q, (uint32_t)p.st[s].radix), (uint32_t)p.st[s].lst);
         rem = q;
     }
-    return (int)(base + __umul24(rem, (uint32_t)p.lst[S - 2]));
+    return (int)(base + __umul24(rem, (uint32_t)p.st[S - 2].lst));
 }
 
 // Leg 0 of butterfly j of a middle stage s; m is the index below digit s
@@ -151,11 +151,11 @@ __device__ __forceinline__ int last_base(const PassDesc& p, int j)
 // neighbouring lanes share a twiddle.
 __device__ __forceinline__ int mid_base(const PassDesc& p, int s, int j, uint32_t& m)
 {
-    const uint32_t q = sdiv((uint32_t)j, p.rdiv[0]);
-    const uint32_t d0 = (uint32_t)j - __umul24(q, (uint32_t)p.radix[0]);
-    const uint32_t o = sdiv(q, p.mdiv[s]);
-    m = q - __umul24(o, (uint32_t)p.lst[s]);
-    return (int)(__umul24(d0, (uint32_t)p.lst[0]) + __umul24(o, (uint32_t)(p.radix[s] * p.lst[s])) + m);
+    const uint32_t q = sdiv((uint32_t)j, p.st[0].rdiv);
+    const uint32_t d0 = (uint32_t)j - __umul24(q, (uint32_t)p.st[0].radix);
+    const uint32_t o = sdiv(q, p.st[s].mdiv);
+    m = q - __umul24(o, (uint32_t)p.st[s].lst);
+    return (int)(__umul24(d0, (uint32_t)p.st[0].lst) + __umul24(o, (uint32_t)(p.st[s].radix * p.st[s].lst)) + m);
 }
 
 // Stage twiddles, one row per output digit k >= 1 and one column per index m
@@ -163,7 +163,7 @@ __device__ __forceinline__ int mid_base(const PassDesc& p, int s, int j, uint32_
 template <typename R>
 __device__ __forceinline__ const cplx<R>* stage_tw(const PassDesc& p, int s)
 {
-    return reinterpret_cast<const cplx<R>*>(p.stw) + p.twoff[s];
+    return reinterpret_cast<const cplx<R>*>(p.stw) + p.st[s].twoff;
 }
 
 template <typename R, int RAD>
@@ -189,7 +189,7 @@ __device__ __forceinline__ void apply_twiddles(cplx<R> (&v)[RAD], const cplx<R> 
 template <typename R, int RAD, bool DIT>
 __device__ __forceinline__ void mid_stage(const PassDesc& p, cplx<R>* line, int t, int s, bool live, bool wave_local)
 {
-    const int nbl = live ? p.nbl[s] : 0, step = p.lst[s];
+    const int nbl = live ? p.st[s].nbl : 0, step = p.st[s].lst;
     const cplx<R>* tw = stage_tw<R>(p, s);
     int j = t, base = 0;
     cplx<R> w[RAD - 1];
@@ -322,7 +322,7 @@ template <typename R, int RAD, bool REAL>
 __device__ __forceinline__ void load_butterfly(const PassDesc& p, const cplx<R>* src, int j, int64_t gbase,
                                                cplx<R> (&v)[RAD])
 {
-    const int nbl = p.nbl[0];
+    const int nbl = p.st[0].nbl;
     if constexpr (REAL) {
         const R* s = reinterpret_cast<const R*>(src);
         if (p.flags & kRealIn) {
@@ -472,10 +472,10 @@ template <typename R, int RAD>
 __device__ __forceinline__ void first_to_lds(const PassDesc& p, cplx<R>* line, int j, cplx<R> (&v)[RAD])
 {
     cplx<R> w[RAD - 1];
-    load_twiddles<R, RAD>(stage_tw<R>(p, 0), (uint32_t)j, p.nbl[0], w);
+    load_twiddles<R, RAD>(stage_tw<R>(p, 0), (uint32_t)j, p.st[0].nbl, w);
     Dft<RAD, R>::run(v);
     apply_twiddles<R, RAD>(v, w);
-    const int step = p.lst[0];
+    const int step = p.st[0].lst;
 #pragma unroll
     for (int i = 0; i < RAD; i++) line[j + i * step] = v[i];
 }
@@ -483,7 +483,7 @@ __device__ __forceinline__ void first_to_lds(const PassDesc& p, cplx<R>* line, i
 template <typename R, int RAD, bool REAL>
 __device__ __forceinline__ void first_stage(const PassDesc& p, cplx<R>* line, int t, const cplx<R>* src, int64_t gbase)
 {
-    const int nbl = p.nbl[0];
+    const int nbl = p.st[0].nbl;
 #pragma unroll 1
     for (int j = t; j < nbl; j += p.TL) {
         cplx<R> v[RAD];
@@ -507,7 +507,7 @@ __device__ __forceinline__ void last_stage(const PassDesc& p, const cplx<R>* lin
 {
     // small radices: several butterflies at a time, for the LDS reads in flight
     constexpr int U = RAD <= 3 ? 4 : RAD <= 5 ? 2 : 1;
-    const int nbl = p.nbl[p.nst - 1];
+    const int nbl = p.st[p.nst - 1].nbl;
 #pragma unroll 1
     for (int j = t; j < nbl; j += U * p.TL) {
         cplx<R> v[U][RAD];
@@ -569,7 +569,7 @@ __device__ __forceinline__ void r2c_last_stage(const PassDesc& p, const cplx<R>*
                                                const cplx<R>* src)
 {
     using PS = PairSlots<RAD>;
-    const int nbl = p.nbl[p.nst - 1], L = p.L;
+    const int nbl = p.st[p.nst - 1].nbl, L = p.L;
     const bool even = (nbl & 1) == 0;
     const cplx<R>* rtw = reinterpret_cast<const cplx<R>*>(p.rtw);
     const R half = R(0.5);
@@ -647,7 +647,7 @@ __device__ __forceinline__ void c2r_first_stage(const PassDesc& p, cplx<R>* line
                                                 cplx<R>* dst)
 {
     using PS = PairSlots<RAD>;
-    const int nbl = p.nbl[0], L = p.L;
+    const int nbl = p.st[0].nbl, L = p.L;
     const bool even = (nbl & 1) == 0;
     const cplx<R>* rtw = reinterpret_cast<const cplx<R>*>(p.rtw);
 #pragma unroll 1
@@ -757,7 +757,7 @@ template <typename R, bool ALLRAD, bool DIT>
 __device__ __forceinline__ void mid_stage_any(const PassDesc& p, cplx<R>* line, int t, int s, bool live,
                                               bool wave_local)
 {
-    FFTZ_RADIX_SWITCH(p.radix[s], ALLRAD, (mid_stage<R, RAD, DIT>(p, line, t, s, live, wave_local)))
+    FFTZ_RADIX_SWITCH(p.st[s].radix, ALLRAD, (mid_stage<R, RAD, DIT>(p, line, t, s, live, wave_local)))
 }
 
 // Forms of the generic pass kernel: complex on both sides; a real side, with
@@ -805,15 +805,15 @@ __device__ __forceinline__ void pass_body(const PassDesc& p, const TileIo& io, c
         }
         if constexpr (REAL) {
             if (p.flags & kR2CPost) {
-                FFTZ_PAIR_SWITCH(p.radix[0], ALLRAD, REALK, (r2c_last_stage<R, RAD>(p, lds, 0, dst, src)))
+                FFTZ_PAIR_SWITCH(p.st[0].radix, ALLRAD, REALK, (r2c_last_stage<R, RAD>(p, lds, 0, dst, src)))
                 return;
             }
             if (p.flags & kC2RPre) {
-                FFTZ_PAIR_SWITCH(p.radix[0], ALLRAD, REALK, (c2r_first_stage<R, RAD>(p, lds, 0, src, dst)))
+                FFTZ_PAIR_SWITCH(p.st[0].radix, ALLRAD, REALK, (c2r_first_stage<R, RAD>(p, lds, 0, src, dst)))
                 return;
             }
         }
-        FFTZ_RADIX_SWITCH(p.radix[0], ALLRAD, (single_stage<R, RAD, REAL, NT>(p, src, dst, l0, gin, gout)))
+        FFTZ_RADIX_SWITCH(p.st[0].radix, ALLRAD, (single_stage<R, RAD, REAL, NT>(p, src, dst, l0, gin, gout)))
         return;
     }
     const bool wave_local = p.TL <= 64 && !in_col && !out_col;
@@ -823,11 +823,11 @@ __device__ __forceinline__ void pass_body(const PassDesc& p, const TileIo& io, c
         if constexpr (REAL) {
             packed = (p.flags & kC2RPre) != 0;
             if (packed) {
-                FFTZ_PAIR_SWITCH(p.radix[0], ALLRAD, REALK, (c2r_first_stage<R, RAD>(p, line, ti, src, dst)))
+                FFTZ_PAIR_SWITCH(p.st[0].radix, ALLRAD, REALK, (c2r_first_stage<R, RAD>(p, line, ti, src, dst)))
             }
         }
         if (!packed) {
-            FFTZ_RADIX_SWITCH(p.radix[0], ALLRAD, (first_stage<R, RAD, REAL>(p, line, ti, src, gin)))
+            FFTZ_RADIX_SWITCH(p.st[0].radix, ALLRAD, (first_stage<R, RAD, REAL>(p, line, ti, src, gin)))
         }
     }
     for (int s = 1; s + 1 < S; s++)
@@ -847,11 +847,11 @@ __device__ __forceinline__ void pass_body(const PassDesc& p, const TileIo& io, c
     const cplx<R>* line = lds + co * p.LP;
     if constexpr (REAL) {
         if (p.flags & kR2CPost) {
-            FFTZ_PAIR_SWITCH(p.radix[S - 1], ALLRAD, REALK, (r2c_last_stage<R, RAD>(p, line, to, dst, src)))
+            FFTZ_PAIR_SWITCH(p.st[S - 1].radix, ALLRAD, REALK, (r2c_last_stage<R, RAD>(p, line, to, dst, src)))
             return;
         }
     }
-    FFTZ_RADIX_SWITCH(p.radix[S - 1], ALLRAD, (last_stage<R, RAD, REAL, NT>(p, line, to, dst, l0, gout)))
+    FFTZ_RADIX_SWITCH(p.st[S - 1].radix, ALLRAD, (last_stage<R, RAD, REAL, NT>(p, line, to, dst, l0, gout)))
 }
 
 template <typename R, bool ALLRAD, int REALK, bool NT, int MAXT>
@@ -885,7 +885,7 @@ __global__ void __launch_bounds__(MAXT)
 template <typename R, int RAD>
 __device__ __forceinline__ void bs_first(const PassDesc& p, cplx<R>* line, int t, const cplx<R>* src)
 {
-    const int nbl = p.nbl[0];
+    const int nbl = p.st[0].nbl;
     const int n = p.nvalid_in;
     const cplx<R>* chirp = reinterpret_cast<const cplx<R>*>(p.chirp);
     const bool cj = (p.flags & kConjIn) != 0;
@@ -933,7 +933,7 @@ __device__ __forceinline__ void bs_first(const PassDesc& p, cplx<R>* line, int t
 template <typename R, int RAD>
 __device__ __forceinline__ void bs_center(const PassDesc& p, cplx<R>* line, int t, bool live, bool wave_local)
 {
-    const int full = p.nbl[p.nst - 1], nbl = live ? full : 0;
+    const int full = p.st[p.nst - 1].nbl, nbl = live ? full : 0;
     const cplx<R>* spec = reinterpret_cast<const cplx<R>*>(p.spec);
     int j = t, base = 0;
     cplx<R> w[RAD];
@@ -967,7 +967,7 @@ template <typename R, int RAD, bool NT>
 __device__ __forceinline__ void bs_final(const PassDesc& p, const cplx<R>* line, int t, cplx<R>* dst, bool live,
                                          bool wave_local)
 {
-    const int full = p.nbl[0], nbl = live ? full : 0, step = p.lst[0];
+    const int full = p.st[0].nbl, nbl = live ? full : 0, step = p.st[0].lst;
     const int n = p.nvalid_out;
     const cplx<R>* chirp = reinterpret_cast<const cplx<R>*>(p.chirp);
     const cplx<R>* tw = stage_tw<R>(p, 0);
@@ -1031,12 +1031,12 @@ __device__ __forceinline__ void bluestein_body(const PassDesc& p, const TileIo& 
     const bool wave_local = p.TL <= 64;
     cplx<R>* line = lds + c * p.LP;
     if (live) {
-        FFTZ_RADIX_SWITCH(p.radix[0], ALLRAD, (bs_first<R, RAD>(p, line, t, src)))
+        FFTZ_RADIX_SWITCH(p.st[0].radix, ALLRAD, (bs_first<R, RAD>(p, line, t, src)))
     }
     for (int s = 1; s + 1 < S; s++) mid_stage_any<R, ALLRAD, false>(p, line, t, s, live, wave_local);
-    FFTZ_RADIX_SWITCH(p.radix[S - 1], ALLRAD, (bs_center<R, RAD>(p, line, t, live, wave_local)))
+    FFTZ_RADIX_SWITCH(p.st[S - 1].radix, ALLRAD, (bs_center<R, RAD>(p, line, t, live, wave_local)))
     for (int s = S - 2; s >= 1; s--) mid_stage_any<R, ALLRAD, true>(p, line, t, s, live, wave_local);
-    FFTZ_RADIX_SWITCH(p.radix[0], ALLRAD, (bs_final<R, RAD, NT>(p, line, t, dst, live, wave_local)))
+    FFTZ_RADIX_SWITCH(p.st[0].radix, ALLRAD, (bs_final<R, RAD, NT>(p, line, t, dst, live, wave_local)))
 }
 
 template <typename R, bool ALLRAD, bool NT, int MAXT>

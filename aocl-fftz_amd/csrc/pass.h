@@ -97,6 +97,17 @@ inline SmallDiv make_smalldiv(uint32_t d)
     return f;
 }
 
+// Stage s of the generic kernels, which hold a line in LDS as mixed-radix
+// digits; together so that one scalar load fetches them.
+struct StageDesc {
+    int radix;
+    int nbl;        // butterflies: L / radix
+    int lst;        // LDS stride of digit s (that of stage 0 padded)
+    int twoff;      // twiddles in stw, in elements
+    SmallDiv mdiv;  // by lst (s >= 1)
+    SmallDiv rdiv;  // by radix
+};
+
 struct PassDesc {
     const void* in;
     void* out;
@@ -137,11 +148,7 @@ struct PassDesc {
     double scale_d;
     int radix[kMaxStages];
     int twoff[kMaxStages];     // stage s's twiddles in stw, in elements
-    // generic kernels (kernels_body.h): a line in LDS as mixed-radix digits
-    int nbl[kMaxStages];       // butterflies of stage s: L / radix[s]
-    int lst[kMaxStages];       // LDS stride of digit s (lst[0] padded)
-    SmallDiv mdiv[kMaxStages]; // by lst[s] (s >= 1)
-    SmallDiv rdiv[kMaxStages]; // by radix[s]
+    StageDesc st[kMaxStages];  // generic kernels (kernels_body.h)
 };
 
 // One tile of an uneven batch: `nlines` consecutive transforms of size class

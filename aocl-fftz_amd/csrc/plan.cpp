@@ -430,13 +430,13 @@ static int64_t digit_layout(TableBuilder& tb, int prec, const std::vector<int>& 
     int A = L;
     for (int s = 0; s < S; s++) {
         const int R = radix[(size_t)s];
-        d.radix[s] = R;
-        d.nbl[s] = L / R;
+        d.radix[s] = d.st[s].radix = R;
+        d.st[s].nbl = L / R;
         A /= R;
-        d.lst[s] = A;
-        d.mdiv[s] = make_smalldiv((uint32_t)A);
-        d.rdiv[s] = make_smalldiv((uint32_t)R);
-        d.twoff[s] = (int)tw.size();
+        d.st[s].lst = A;
+        d.st[s].mdiv = make_smalldiv((uint32_t)A);
+        d.st[s].rdiv = make_smalldiv((uint32_t)R);
+        d.st[s].twoff = (int)tw.size();
         if (s + 1 < S)
             for (int k = 1; k < R; k++)
                 for (int m = 0; m < A; m++) tw.push_back(root_fwd((int64_t)k * m, (int64_t)R * A));
@@ -444,7 +444,7 @@ static int64_t digit_layout(TableBuilder& tb, int prec, const std::vector<int>& 
     int LP = std::max(lp_min, L);
     if (S >= 2) {
         const int lanes = prec == 4 ? 16 : 8;  // lanes (and banks, in elements) per LDS cycle
-        const int A0 = d.lst[0];
+        const int A0 = d.st[0].lst;
         int best = 0;
         long best_cost = -1;
         for (int pad = 0; pad < 8; pad++) {
@@ -459,18 +459,18 @@ static int64_t digit_layout(TableBuilder& tb, int prec, const std::vector<int>& 
                     int worst = 0;
                     for (int l = l0; l < l0 + lanes; l++) {
                         const int c = l / std::min(TL, 64), j = l % std::min(TL, 64);
-                        if (j >= d.nbl[s]) continue;
+                        if (j >= d.st[s].nbl) continue;
                         int pos = 0;
                         if (s + 1 == S) {
                             int rem = j;
                             for (int i = 0; i + 2 < S; i++) {
-                                pos += (rem % radix[(size_t)i]) * (i ? d.lst[i] : a0);
+                                pos += (rem % radix[(size_t)i]) * (i ? d.st[i].lst : a0);
                                 rem /= radix[(size_t)i];
                             }
-                            pos += rem * (S >= 3 ? d.lst[S - 2] : a0);
+                            pos += rem * (S >= 3 ? d.st[S - 2].lst : a0);
                         } else {
-                            const int q = j / radix[0], o = q / d.lst[s], m = q % d.lst[s];
-                            pos = (j % radix[0]) * a0 + o * radix[(size_t)s] * d.lst[s] + m;
+                            const int q = j / radix[0], o = q / d.st[s].lst, m = q % d.st[s].lst;
+                            pos = (j % radix[0]) * a0 + o * radix[(size_t)s] * d.st[s].lst + m;
                         }
                         worst = std::max(worst, ++bank[(pos + c * pitch) % lanes]);
                     }
@@ -483,8 +483,8 @@ static int64_t digit_layout(TableBuilder& tb, int prec, const std::vector<int>& 
                 best = pad;
             }
         }
-        d.lst[0] = A0 + best;
-        LP = std::max(LP, radix[0] * d.lst[0]);
+        d.st[0].lst = A0 + best;
+        LP = std::max(LP, radix[0] * d.st[0].lst);
     }
     d.LP = LP | 1;
     if (tw.empty()) tw.push_back({1.0, 0.0});
