@@ -1790,12 +1790,20 @@ Plan* batch_plan_create(const std::vector<BatchItem>& items, int prec, int dir, 
     plan->out_extent_bytes = out_ext * esize;
     plan->flops = flops;
     // tiles per class, cost-sorted (largest first)
-    // a queue entry covers up to `rounds` rounds of C lines (about 128 KiB of
-    // input; 256 KiB in the large class, whose single-line rounds are up to
-    // 128 KiB each: measured 2.6% faster there, no gain in the others) so the
-    // per-entry cost (queue atomic, descriptor loads, barriers) is amortised
+    // A queue entry covers up to `rounds` rounds of C lines, so that the per-entry
+    // cost (queue atomic, descriptor loads, barriers) is amortised -- but its
+    // rounds run one after the other, and a workgroup's last entry is the
+    // launch's tail: an eighth of what a resident workgroup gets in all, between
+    // 16 KiB and 32 / 128 / 256 KiB.  Against 128 / 128 / 256 KiB throughout:
+    // 2000 items 2.18 -> 2.05 ms, 400 items 0.65 -> 0.48 ms, 100 items 0.43 ->
+    // 0.14 ms.
     const int64_t entry_env = env_int("FFTZ_BATCH_ENTRY_BYTES", 0);
-    const int64_t entry_cls[3] = {128 * 1024, 128 * 1024, 256 * 1024};
+    const int64_t entry_most[3] = {32 * 1024, 128 * 1024, 256 * 1024}, resident[3] = {4, 2, 1};
+    int64_t entry_cls[3] = {0, 0, 0};
+    for (const BatchItem& it : items)
+        if (it.batch) entry_cls[sizes[(size_t)size_index[it.n]].cls] += it.n * it.batch * esize;
+    for (int c = 0; c < 3; c++)
+        entry_cls[c] = std::max<int64_t>(16 * 1024, std::min(entry_most[c], entry_cls[c] / (8 * dev.cus * resident[c])));
     std::vector<std::vector<std::pair<double, BatchTile>>> tiles(3);
     for (const BatchItem& it : items) {
         if (it.batch == 0) continue;
