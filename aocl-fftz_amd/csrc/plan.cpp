@@ -704,7 +704,12 @@ static bool build_pass(Plan* plan, TableBuilder& tb, const PassReq& q, std::stri
         ln.stw_off = stage_twiddles(tb, prec, radix, d.twoff);
         d.LP = (lds_pad(need - 1) + 1) | 1;
     } else {
-        TL = line_threads(radix, q.L, q.want_in_col || q.want_out_col ? 4 : 64 / esize, tmax,
+        // column tiles: at most 64 threads per line (32 in complex128) while that
+        // leaves 20 elements per thread, see the tile's limit below
+        const bool cols = q.want_in_col || q.want_out_col;
+        int most = cols ? 256 / prec : tmax;
+        while (most < tmax && q.L > 20 * most) most *= 2;
+        TL = line_threads(radix, q.L, cols ? 4 : 64 / esize, most,
                           r2c ? (int)radix.size() - 1 : c2r ? 0 : -1, nl_total, prec);
         if (tuned_e == 8 || tuned_e == 16) TL = std::min(next_pow2((q.L + tuned_e - 1) / tuned_e), tmax);
         ln.E = std::max(tuned_e == 8 || tuned_e == 16 ? tuned_e : 1, (q.L + TL - 1) / TL);
@@ -763,10 +768,16 @@ static bool build_pass(Plan* plan, TableBuilder& tb, const PassReq& q, std::stri
         // points on: columns of 8 lines 35 us, of 4 lines 40 us (64 MiB each way)
         const bool whole = plan_match && prec == 8 && q.L >= 1024;
         const size_t budget = std::min(lds_cap, (size_t)env_int("FFTZ_COL_LDS", whole ? 160 * 1024 : 96 * 1024));
+        // Generic kernels: two workgroups per CU at their register counts, i.e.
+        // 512 threads (256 in complex128), so that one loads while the other
+        // computes: 1080-point columns of 961 x 13 images, 8 lines of 128
+        // threads 78 us, of 64 threads 63 us; complex128 600-point columns, 8
+        // lines of 64 threads 48 us, of 32 threads 38 us.
+        const int tcap = plan_match ? tmax : std::min(tmax, 2048 / prec);
         // a row of n0 lines that C does not divide is tiled raggedly (the
         // last tile of each row partly idle) rather than falling back to
         // element-strided row tiles
-        while (C * 2 <= cmax && (size_t)(C * 2) * line_bytes <= budget && C * 2 <= n0 && C * 2 * TL <= tmax)
+        while (C * 2 <= cmax && (size_t)(C * 2) * line_bytes <= budget && C * 2 <= n0 && C * 2 * TL <= tcap)
             C *= 2;
         // fewer than two tiles per CU: narrower ones, down to 16 lines (128- or
         // 256-byte segments); fewer than one for two CUs: down to four lines
