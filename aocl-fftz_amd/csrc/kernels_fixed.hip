@@ -101,6 +101,39 @@ __device__ __forceinline__ void stage_sync(bool wave_local)
     lds_barrier();
 }
 
+// Stage exchange through LDS: every thread writes W values and then reads N
+// values of its line.  at(i) / from(i): LDS slots of the i-th value written /
+// read.  Whole complex values, or (SPLIT) the real parts and then the
+// imaginary parts through an LDS of half the size: twice the barriers, but
+// half the LDS per workgroup where that is what limits the workgroups of a CU.
+// Ends with the reads issued; the caller puts a barrier before the next write.
+template <typename R, bool SPLIT, int TL, int W, int N, typename At, typename From>
+__device__ __forceinline__ void exchange(void* lds, const cplx<R>* v, cplx<R>* w, bool wave_local, At at, From from)
+{
+    if constexpr (SPLIT) {
+        R* l = reinterpret_cast<R*>(lds);
+#pragma unroll
+        for (int i = 0; i < W; i++) l[at(i)] = v[i].x;
+        stage_sync<TL>(wave_local);
+        R re[N];
+#pragma unroll
+        for (int i = 0; i < N; i++) re[i] = l[from(i)];
+        stage_sync<TL>(wave_local);
+#pragma unroll
+        for (int i = 0; i < W; i++) l[at(i)] = v[i].y;
+        stage_sync<TL>(wave_local);
+#pragma unroll
+        for (int i = 0; i < N; i++) w[i] = {re[i], l[from(i)]};
+    } else {
+        cplx<R>* l = reinterpret_cast<cplx<R>*>(lds);
+#pragma unroll
+        for (int i = 0; i < W; i++) l[at(i)] = v[i];
+        stage_sync<TL>(wave_local);
+#pragma unroll
+        for (int i = 0; i < N; i++) w[i] = l[from(i)];
+    }
+}
+
 template <typename R, int RAD>
 __device__ __forceinline__ void twiddle_legs(cplx<R>* v, const cplx<R>* w)
 {
@@ -110,52 +143,45 @@ __device__ __forceinline__ void twiddle_legs(cplx<R>* v, const cplx<R>* w)
 
 }  // namespace
 
-// One LDS stage s (not the first, not the last): read K butterflies, barrier,
-// twiddle + DFT, write, barrier.  (c, t) is this stage's thread mapping.
-template <typename R, int L, int s>
-__device__ __forceinline__ void fixed_mid_stage(const PassDesc& p, cplx<R>* lds, int c, int t, bool wave_local)
+// Pitch of a line in the LDS, in elements.
+template <int L>
+constexpr int kPitch = ((L - 1) + ((L - 1) >> 4) + 1) | 1;
+
+// Middle stages s .. S-2 and the exchange into the last one.  On entry v holds
+// the outputs of stage s-1, thread mapping (cw, tw) of that stage, 16/R0
+// butterflies of R0 legs at base + i * ls; on return w holds the operands of
+// the last stage under mapping (co, to).
+template <typename R, int L, int s, bool SPLIT>
+__device__ __forceinline__ void fixed_stages(const PassDesc& p, void* lds, int cw, int tw, int cm, int tm, int co,
+                                             int to, bool wave_local, const cplx<R>* v, cplx<R>* w)
 {
     using P = Plan2<L>;
-    constexpr int RAD = P::radix(s);
-    constexpr int ls = P::ls(s);
-    constexpr int K = 16 / RAD;
-    constexpr int TL = L / 16;
-    constexpr int nbl = L / RAD;
-    constexpr int LP = ((L - 1) + ((L - 1) >> 4) + 1) | 1;
-    cplx<R>* line = lds + c * LP;
-    cplx<R> v[K][RAD];
+    constexpr int S = P::S, TL = L / 16, LP = kPitch<L>;
+    constexpr int RP = P::radix(s - 1), lsP = P::ls(s - 1);  // the stage that wrote v
+    constexpr int RAD = P::radix(s), nbl = L / RAD;
+    // slot written for value i of v: butterfly j = tw + (i / RP) TL of stage s-1
+    auto at = [&](int i) {
+        const int j = tw + (i / RP) * TL, g = j / lsP, cc = j % lsP;
+        return cw * LP + pad_c<L>(g * RP * lsP + cc + (i % RP) * lsP);
+    };
+    const int c = s == S - 1 ? co : cm, t = s == S - 1 ? to : tm;
+    auto from = [&](int i) { return c * LP + pad_c<L>((i % RAD) * nbl + t + (i / RAD) * TL); };
+    if constexpr (s == S - 1) {
+        exchange<R, SPLIT, TL, 16, 16>(lds, v, w, wave_local, at, from);
+    } else {
+        cplx<R> u[16];
+        exchange<R, SPLIT, TL, 16, 16>(lds, v, u, wave_local, at, from);
+        stage_sync<TL>(wave_local);
+        const cplx<R>* twd = reinterpret_cast<const cplx<R>*>(p.stw) + p.twoff[s];
+        constexpr int ls = P::ls(s);
 #pragma unroll
-    for (int k = 0; k < K; k++) {
-        const int j = t + k * TL;
-#pragma unroll
-        for (int i = 0; i < RAD; i++) v[k][i] = line[pad_c<L>(i * nbl + j)];
-    }
-    stage_sync<TL>(wave_local);
-    const cplx<R>* tw = reinterpret_cast<const cplx<R>*>(p.stw) + p.twoff[s];
-#pragma unroll
-    for (int k = 0; k < K; k++) {
-        const int j = t + k * TL;
-        const int g = j / ls;
-        const int cc = j % ls;
-        twiddle_legs<R, RAD>(v[k], tw + cc * (RAD - 1));
-        Dft<RAD, R>::run(v[k]);
-        const int base = g * RAD * ls + cc;
-#pragma unroll
-        for (int i = 0; i < RAD; i++) line[pad_c<L>(base + i * ls)] = v[k][i];
-    }
-    stage_sync<TL>(wave_local);
-}
-
-template <typename R, int L, int s, int S>
-struct MidStages {
-    static __device__ __forceinline__ void run(const PassDesc& p, cplx<R>* lds, int c, int t, bool wave_local)
-    {
-        if constexpr (s < S - 1) {
-            fixed_mid_stage<R, L, s>(p, lds, c, t, wave_local);
-            MidStages<R, L, s + 1, S>::run(p, lds, c, t, wave_local);
+        for (int k = 0; k < 16 / RAD; k++) {
+            twiddle_legs<R, RAD>(u + k * RAD, twd + ((t + k * TL) % ls) * (RAD - 1));
+            Dft<RAD, R>::run(u + k * RAD);
         }
+        fixed_stages<R, L, s + 1, SPLIT>(p, lds, c, t, cm, tm, co, to, wave_local, u, w);
     }
-};
+}
 
 template <typename R, int L>
 __device__ __forceinline__ void fixed_load(const PassDesc& p, int64_t l_base, int c, int t, cplx<R>* v)
@@ -178,18 +204,16 @@ __device__ __forceinline__ void fixed_load(const PassDesc& p, int64_t l_base, in
 // threads (256, or 512 for wide column tiles).  A register prefetch of the
 // next tile was measured slower: the extra 16 live values per lane cut
 // occupancy from 5 to 2 waves/SIMD.
-template <typename R, int L, int MAXT>
+template <typename R, int L, int MAXT, bool SPLIT>
 __global__ void __launch_bounds__(MAXT) k_fixed_pass(const PassDesc p)
 {
     using P = Plan2<L>;
     constexpr int S = P::S;
     constexpr int TL = L / 16;
-    constexpr int LP = ((L - 1) + ((L - 1) >> 4) + 1) | 1;
     constexpr int R0 = P::radix(0);
     constexpr int RL = P::radix(S - 1);
     static_assert(R0 == 16, "first stage is radix 16");
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
-    cplx<R>* lds = reinterpret_cast<cplx<R>*>(smem_raw);
     const int tid = threadIdx.x;
     uint32_t tile = blockIdx.x;
     if (p.flags & kXcdRemap) {
@@ -199,9 +223,11 @@ __global__ void __launch_bounds__(MAXT) k_fixed_pass(const PassDesc p)
     const int64_t l_base = (int64_t)tile * p.C;
 
     // load (input-side mapping) + stage 1 in registers
-    const bool in_col = (p.flags & kInCol) != 0;
+    const bool in_col = (p.flags & kInCol) != 0, out_col = (p.flags & kOutCol) != 0;
     const int ci = in_col ? (tid & (p.C - 1)) : (tid / TL);
     const int ti = in_col ? (tid >> p.c_shift) : (tid % TL);
+    const int co = out_col ? (tid & (p.C - 1)) : (tid / TL);
+    const int to = out_col ? (tid >> p.c_shift) : (tid % TL);
     cplx<R> v[16];
     fixed_load<R, L>(p, l_base, ci, ti, v);
     if (p.flags & kConjIn) {
@@ -210,35 +236,15 @@ __global__ void __launch_bounds__(MAXT) k_fixed_pass(const PassDesc p)
     }
     // butterfly j = ti reads x[i*TL + ti]; writes y[ti*16 + i]
     Dft<16, R>::run(v);
-    {
-        cplx<R>* line = lds + ci * LP;
-#pragma unroll
-        for (int i = 0; i < 16; i++) line[pad_c<L>(ti * 16 + i)] = v[i];
-    }
     // lines held by one wavefront each (row mapping throughout, TL <= 64)
-    // exchange through LDS without workgroup barriers
-    const bool wave_local = !(p.flags & (kInCol | kOutCol));
-    stage_sync<TL>(wave_local);
-
-    // middle stages (row mapping)
-    MidStages<R, L, 1, S>::run(p, lds, tid / TL, tid % TL, wave_local);
-
-    // last stage (output-side mapping) + store
-    const bool out_col = (p.flags & kOutCol) != 0;
-    const int co = out_col ? (tid & (p.C - 1)) : (tid / TL);
-    const int to = out_col ? (tid >> p.c_shift) : (tid % TL);
+    // exchange through LDS without workgroup barriers; middle stages in row
+    // mapping, last stage in the output side's
+    const bool wave_local = !in_col && !out_col;
     constexpr int KL = 16 / RL;
     constexpr int lsL = L / RL;
-    cplx<R> w[KL][RL];
-    {
-        const cplx<R>* line = lds + co * LP;
-#pragma unroll
-        for (int k = 0; k < KL; k++) {
-            const int j = to + k * TL;
-#pragma unroll
-            for (int i = 0; i < RL; i++) w[k][i] = line[pad_c<L>(i * lsL + j)];
-        }
-    }
+    cplx<R> wv[16];
+    fixed_stages<R, L, 1, SPLIT>(p, smem_raw, ci, ti, tid / TL, tid % TL, co, to, wave_local, v, wv);
+    cplx<R>(&w)[KL][RL] = *reinterpret_cast<cplx<R>(*)[KL][RL]>(wv);
     uint32_t l_out;
     if (!slot_line_f(p, l_base, co, l_out)) return;
     LineOff lo = line_off(p, l_out);
@@ -293,20 +299,29 @@ template <typename R, int MAXT>
 static const void* fixed_sym(int L)
 {
     switch (L) {
-        case 64: return MAXT == 256 ? (const void*)&k_fixed_pass<R, 64, 256> : nullptr;
-        case 128: return MAXT == 256 ? (const void*)&k_fixed_pass<R, 128, 256> : nullptr;
-        case 256: return (const void*)&k_fixed_pass<R, 256, MAXT>;
-        case 512: return (const void*)&k_fixed_pass<R, 512, MAXT>;
-        case 1024: return (const void*)&k_fixed_pass<R, 1024, MAXT>;
-        case 2048: return (const void*)&k_fixed_pass<R, 2048, MAXT>;
-        case 4096: return (const void*)&k_fixed_pass<R, 4096, MAXT>;
+        case 64: return MAXT == 256 ? (const void*)&k_fixed_pass<R, 64, 256, false> : nullptr;
+        case 128: return MAXT == 256 ? (const void*)&k_fixed_pass<R, 128, 256, false> : nullptr;
+        case 256: return (const void*)&k_fixed_pass<R, 256, MAXT, false>;
+        case 512: return (const void*)&k_fixed_pass<R, 512, MAXT, false>;
+        case 1024: return (const void*)&k_fixed_pass<R, 1024, MAXT, false>;
+        case 2048: return (const void*)&k_fixed_pass<R, 2048, MAXT, false>;
+        case 4096: return (const void*)&k_fixed_pass<R, 4096, MAXT, false>;
         default: return nullptr;
     }
 }
 
-const void* kernel_symbol_fixed(int prec_bytes, int L, int maxt)
+const void* kernel_symbol_fixed(int prec_bytes, int L, int maxt, bool split)
 {
     if (maxt != 256 && maxt != 512) return nullptr;
+    if (split) {
+        if (prec_bytes == 4 && L == 512)
+            return maxt == 256 ? (const void*)&k_fixed_pass<float, 512, 256, true>
+                               : (const void*)&k_fixed_pass<float, 512, 512, true>;
+        if (prec_bytes == 8 && L == 256)
+            return maxt == 256 ? (const void*)&k_fixed_pass<double, 256, 256, true>
+                               : (const void*)&k_fixed_pass<double, 256, 512, true>;
+        return nullptr;
+    }
     if (prec_bytes == 4) return maxt == 256 ? fixed_sym<float, 256>(L) : fixed_sym<float, 512>(L);
     return maxt == 256 ? fixed_sym<double, 256>(L) : fixed_sym<double, 512>(L);
 }

@@ -61,9 +61,10 @@ const DeviceInfo& device_info()
         for (int prec : {4, 8})
             for (int L = 64; L <= 4096; L *= 2)
                 for (int t : {256, 512})
-                    if (const void* f = kernel_symbol_fixed(prec, L, t))
-                        (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                  (int)info.lds_per_block);
+                    for (bool split : {false, true})
+                        if (const void* f = kernel_symbol_fixed(prec, L, t, split))
+                            (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                      (int)info.lds_per_block);
         for (int m : {kMfmaF32, kMfmaBf16x3, kMfmaF16x2})
             for (int L : {256, 4096})
                 for (int nb : {2, 4})
@@ -860,6 +861,7 @@ static bool build_pass(Plan* plan, TableBuilder& tb, const PassReq& q, std::stri
     }
     ln.grid = (uint32_t)tiles;
     ln.lds_bytes = (uint32_t)((size_t)C * line_bytes);
+    ln.split = ln.fixed && (in_col || out_col) && q.L == (prec == 4 ? 512 : 256);
     if (use_mfma) ln.lds_bytes += 64;  // per-wavefront maxima of the fp16 line scale
     // XCD-contiguous tile order: measured to help passes that read rows and
     // store columns (the four-step's transposing last pass) and to cost ~5%
@@ -2412,11 +2414,11 @@ static hipError_t launch_all(Plan* p, void* work, unsigned* counters, const void
         const float* frag = ln.frag;
         void* args[] = {&d, &frag};
         const void* fn = ln.mfma ? kernel_symbol_mfma(ln.mfma, ln.d.L, ln.mfma_nb)
-                         : ln.fixed ? kernel_symbol_fixed(p->spec.prec_bytes, ln.d.L, ln.maxt)
+                         : ln.fixed ? kernel_symbol_fixed(p->spec.prec_bytes, ln.d.L, ln.maxt, ln.split)
                                     : kernel_symbol(pass_kind(ln), p->spec.prec_bytes, ln.all_radix,
                                                     (d.flags & kNtStore) != 0, ln.maxt);
-        hipError_t e = hipLaunchKernel(fn, dim3(ln.grid),
-                                       dim3(ln.block), args, ln.lds_bytes, stream);
+        hipError_t e = hipLaunchKernel(fn, dim3(ln.grid), dim3(ln.block), args,
+                                       ln.split ? ln.lds_bytes / 2 : ln.lds_bytes, stream);
         if (e != hipSuccess) return e;
         if (prof) {
             e = record_prof(p, stream);

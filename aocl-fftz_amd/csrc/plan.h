@@ -80,6 +80,7 @@ struct Launch {
     int E = 16;        // complex values of a line per thread
     int maxt = 256;    // block-size bound of the kernel variant
     bool fixed = false;  // fixed-length kernel (kernels_fixed.hip)
+    bool split = false;  // its exchanges run through half of lds_bytes
     int mfma = 0;        // MfmaMode of a matrix-core pass (kernels_mfma.hip)
     int mfma_nb = 4;     // its column blocks per wavefront
     PassDesc d{};
