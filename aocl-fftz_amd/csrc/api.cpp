@@ -325,8 +325,11 @@ aoclfftz_error_type run(Handle* h, void* in, void* out, const char* fname)
                     s->stage_out_bytes = need_out;
                 }
                 dout = s->stage_out;
-                // strided outputs: keep the caller's untouched elements
-                if (hipMemcpyAsync(dout, out, need_out, hipMemcpyHostToDevice, s->stream) != hipSuccess) {
+                // outputs with gaps: keep the caller's untouched elements (a
+                // dense output is overwritten whole: 16 MiB each way 2.18 ->
+                // 1.59 ms without this copy)
+                if (!p->dense_out &&
+                    hipMemcpyAsync(dout, out, need_out, hipMemcpyHostToDevice, s->stream) != hipSuccess) {
                     rc = AOCLFFTZ_EXECUTION_FAILURE;
                     break;
                 }

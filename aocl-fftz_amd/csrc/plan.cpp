@@ -1088,6 +1088,24 @@ static int64_t extent(const std::vector<AxisSpec>& dims, const std::vector<AxisS
     return e + 1;
 }
 
+// Whether the output side is one gapless run: its axes, by stride, each continue
+// where the one before ends (no zero, negative or overlapping strides).
+static bool dense(const std::vector<AxisSpec>& dims, const std::vector<AxisSpec>& vecs, int64_t n0_override)
+{
+    std::vector<std::pair<int64_t, int64_t>> ax;  // stride, length
+    for (size_t i = 0; i < dims.size(); i++)
+        ax.push_back({dims[i].os, i == 0 && n0_override > 0 ? n0_override : dims[i].n});
+    for (auto& v : vecs) ax.push_back({v.os, v.n});
+    ax.erase(std::remove_if(ax.begin(), ax.end(), [](const auto& a) { return a.second == 1; }), ax.end());
+    std::sort(ax.begin(), ax.end());
+    int64_t next = 1;
+    for (const auto& a : ax) {
+        if (a.first != next) return false;
+        next *= a.second;
+    }
+    return true;
+}
+
 // Balanced factorisation of a large 1-D length into p factors, each <= fmax
 // and a product of radices.
 static bool split_factors(int64_t N, int64_t fmax, std::vector<int64_t>& f)
@@ -2160,6 +2178,7 @@ Plan* plan_create(const ProblemSpec& spec_in, std::string& err, bool dry_run)
         plan->in_extent_bytes = extent(spec.dims, spec.vecs, true, spec.dims[0].n / 2 + 1) * 2 * spec.prec_bytes;
         plan->out_extent_bytes = extent(spec.dims, spec.vecs, false, -1) * spec.prec_bytes;
     }
+    plan->dense_out = dense(spec.dims, spec.vecs, spec.type == FftType::R2C ? spec.dims[0].n / 2 + 1 : -1);
     if (plan->noop) return plan;
 
     // algorithmic flop count (5 N log2 N for C2C, 2.5 N log2 N for real)

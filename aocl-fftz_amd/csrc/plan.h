@@ -120,6 +120,7 @@ struct Plan {
     std::vector<Launch> launches;
     size_t work_bytes = 0;
     int64_t in_extent_bytes = 0, out_extent_bytes = 0;
+    bool dense_out = false;  // the transform writes every element of the output extent
     std::vector<unsigned char> host_tables;
     void* tables = nullptr;
     void* setup_in = nullptr;
