@@ -7,16 +7,21 @@ namespace fftz {
 
 enum class KernelKind { Pass, Real, RealWide, Bluestein };
 
-// Device function symbol for hipLaunchKernel / hipFuncSetAttribute.
-// prec_bytes: 4 (complex64) or 8 (complex128).  all_radix: the variant that
-// carries the 3/5/6/7/9/10/11/12/13 stages (the power-of-two variant carries
-// only 2/4/8/16 and therefore needs fewer VGPRs).  nt: the variant whose
-// complex results bypass the L2's write-back (kNtStore).  maxt: block-size bound of
-// the variant, 256 or more (then 1024 threads in complex64, 512 in
-// complex128); the 256 variants get a larger VGPR budget.  Real: passes with a
-// real side (kRealFlags); RealWide: real-packed ones whose pair stage (last for
-// R2C, first for C2R) has radix 11 or 13.
-const void* kernel_symbol(KernelKind kind, int prec_bytes, bool all_radix, bool nt, int maxt);
+// Radices a generic kernel carries: 2, 4, 8, 16; all of 2 .. 13 and 16; or all
+// but 11, 13 and 16 (complex64 plain passes only).  The registers of the widest
+// butterfly set the wavefronts of every launch: 112 with all radices (four
+// wavefronts per SIMD), 88 without those three (five).
+enum RadixSet : int { kRadPow2 = 0, kRadAll = 1, kRadLight = 2 };
+
+// Device function symbol for hipLaunchKernel / hipFuncSetAttribute; nullptr
+// where there is no such kernel.  prec_bytes: 4 (complex64) or 8 (complex128).
+// rad: a RadixSet.  nt: the variant whose complex results bypass the L2's
+// write-back (kNtStore).  maxt: block-size bound of the variant, 256 or more
+// (then 1024 threads in complex64, 512 in complex128); the 256 variants get a
+// larger VGPR budget.  Real: passes with a real side (kRealFlags); RealWide:
+// real-packed ones whose pair stage (last for R2C, first for C2R) has radix 11
+// or 13.
+const void* kernel_symbol(KernelKind kind, int prec_bytes, int rad, bool nt, int maxt);
 
 // Uneven-batch persistent kernel (k_batch) of a tile class (0 small: 256
 // threads, 1 medium: 512, 2 large: 1024 in complex64, 512 in complex128) and
@@ -30,6 +35,7 @@ const void* kernel_symbol_pass_f32_mixed(KernelKind kind, bool nt, int maxt);
 const void* kernel_symbol_pass_f32_pow2(KernelKind kind, bool nt, int maxt);
 const void* kernel_symbol_pass_f64_mixed(KernelKind kind, bool nt, int maxt);
 const void* kernel_symbol_pass_f64_pow2(KernelKind kind, bool nt, int maxt);
+const void* kernel_symbol_pass_f32_light(bool nt, int maxt);
 const void* kernel_symbol_batch_f32_small();
 const void* kernel_symbol_batch_f32_medium();
 const void* kernel_symbol_batch_f32_large();

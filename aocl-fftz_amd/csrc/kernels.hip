@@ -16,11 +16,16 @@ __global__ void k_reset_counters(unsigned* c, int n)
     if ((int)threadIdx.x < n) c[threadIdx.x] = 0u;
 }
 
-const void* kernel_symbol(KernelKind kind, int prec_bytes, bool all_radix, bool nt, int maxt)
+const void* kernel_symbol(KernelKind kind, int prec_bytes, int rad, bool nt, int maxt)
 {
+    if (rad == kRadLight) {
+        if (kind != KernelKind::Pass || prec_bytes != 4) return nullptr;
+        return kernel_symbol_pass_f32_light(nt, maxt);
+    }
     if (prec_bytes == 4)
-        return all_radix ? kernel_symbol_pass_f32_mixed(kind, nt, maxt) : kernel_symbol_pass_f32_pow2(kind, nt, maxt);
-    return all_radix ? kernel_symbol_pass_f64_mixed(kind, nt, maxt) : kernel_symbol_pass_f64_pow2(kind, nt, maxt);
+        return rad == kRadAll ? kernel_symbol_pass_f32_mixed(kind, nt, maxt)
+                              : kernel_symbol_pass_f32_pow2(kind, nt, maxt);
+    return rad == kRadAll ? kernel_symbol_pass_f64_mixed(kind, nt, maxt) : kernel_symbol_pass_f64_pow2(kind, nt, maxt);
 }
 
 const void* kernel_symbol_batch(int prec_bytes, int cls)

@@ -224,14 +224,19 @@ __device__ __forceinline__ void mid_stage(const PassDesc& p, cplx<R>* line, int 
         CALL;                    \
     } break;
 
-#define FFTZ_RADIX_SWITCH(rad, ALLRAD, CALL)       \
+#define FFTZ_RADIX_SWITCH(rad, RADSET, CALL)       \
     switch (rad) {                                 \
         FFTZ_RADIX_CASE(2, CALL)                   \
         FFTZ_RADIX_CASE(4, CALL)                   \
         FFTZ_RADIX_CASE(8, CALL)                   \
-        FFTZ_RADIX_CASE(16, CALL)                  \
+        case 16:                                   \
+            if constexpr (RADSET != kRadLight) {   \
+                constexpr int RAD = 16;            \
+                CALL;                              \
+            }                                      \
+            break;                                 \
         default:                                   \
-            if constexpr (ALLRAD) {                \
+            if constexpr (RADSET != kRadPow2) {    \
                 switch (rad) {                     \
                     FFTZ_RADIX_CASE(3, CALL)       \
                     FFTZ_RADIX_CASE(5, CALL)       \
@@ -239,10 +244,15 @@ __device__ __forceinline__ void mid_stage(const PassDesc& p, cplx<R>* line, int 
                     FFTZ_RADIX_CASE(7, CALL)       \
                     FFTZ_RADIX_CASE(9, CALL)       \
                     FFTZ_RADIX_CASE(10, CALL)      \
-                    FFTZ_RADIX_CASE(11, CALL)      \
                     FFTZ_RADIX_CASE(12, CALL)      \
-                    FFTZ_RADIX_CASE(13, CALL)      \
                     default: break;                \
+                }                                  \
+                if constexpr (RADSET == kRadAll) { \
+                    switch (rad) {                 \
+                        FFTZ_RADIX_CASE(11, CALL)  \
+                        FFTZ_RADIX_CASE(13, CALL)  \
+                        default: break;            \
+                    }                              \
                 }                                  \
             }                                      \
             break;                                 \
@@ -250,7 +260,7 @@ __device__ __forceinline__ void mid_stage(const PassDesc& p, cplx<R>* line, int 
 
 // Radices of the stage that holds mirrored butterfly pairs (kRealPair: up to
 // 10, kRealWide: 11 and 13).
-#define FFTZ_PAIR_SWITCH(rad, ALLRAD, REAL, CALL)  \
+#define FFTZ_PAIR_SWITCH(rad, RADSET, REAL, CALL)  \
     if constexpr (REAL == kRealWide) {             \
         switch (rad) {                             \
             FFTZ_RADIX_CASE(11, CALL)              \
@@ -263,7 +273,7 @@ __device__ __forceinline__ void mid_stage(const PassDesc& p, cplx<R>* line, int 
             FFTZ_RADIX_CASE(4, CALL)               \
             FFTZ_RADIX_CASE(8, CALL)               \
             default:                               \
-                if constexpr (ALLRAD) {            \
+                if constexpr (RADSET != kRadPow2) { \
                     switch (rad) {                 \
                         FFTZ_RADIX_CASE(3, CALL)   \
                         FFTZ_RADIX_CASE(5, CALL)   \
@@ -753,11 +763,11 @@ __device__ __forceinline__ void identity_line(const PassDesc& p, const cplx<R>* 
 }
 
 // Every middle stage begins with the barrier that ends the stage before it.
-template <typename R, bool ALLRAD, bool DIT>
+template <typename R, int RADSET, bool DIT>
 __device__ __forceinline__ void mid_stage_any(const PassDesc& p, cplx<R>* line, int t, int s, bool live,
                                               bool wave_local)
 {
-    FFTZ_RADIX_SWITCH(p.st[s].radix, ALLRAD, (mid_stage<R, RAD, DIT>(p, line, t, s, live, wave_local)))
+    FFTZ_RADIX_SWITCH(p.st[s].radix, RADSET, (mid_stage<R, RAD, DIT>(p, line, t, s, live, wave_local)))
 }
 
 // Forms of the generic pass kernel: complex on both sides; a real side, with
@@ -767,7 +777,7 @@ enum RealForm : int { kRealNone = 0, kRealPair = 1, kRealWide = 2 };
 // One tile: C lines, threads (c, t) per side's mapping -- row (a wavefront
 // walks along a line) or column (it walks the same element of adjacent lines).
 // REAL passes carry the real-packed and promoted forms and are row-mapped.
-template <typename R, bool ALLRAD, int REALK, bool NT>
+template <typename R, int RADSET, int REALK, bool NT>
 __device__ __forceinline__ void pass_body(const PassDesc& p, const TileIo& io, cplx<R>* lds, int64_t l_base, int tid)
 {
     constexpr bool REAL = REALK != kRealNone;
@@ -805,15 +815,15 @@ __device__ __forceinline__ void pass_body(const PassDesc& p, const TileIo& io, c
         }
         if constexpr (REAL) {
             if (p.flags & kR2CPost) {
-                FFTZ_PAIR_SWITCH(p.st[0].radix, ALLRAD, REALK, (r2c_last_stage<R, RAD>(p, lds, 0, dst, src)))
+                FFTZ_PAIR_SWITCH(p.st[0].radix, RADSET, REALK, (r2c_last_stage<R, RAD>(p, lds, 0, dst, src)))
                 return;
             }
             if (p.flags & kC2RPre) {
-                FFTZ_PAIR_SWITCH(p.st[0].radix, ALLRAD, REALK, (c2r_first_stage<R, RAD>(p, lds, 0, src, dst)))
+                FFTZ_PAIR_SWITCH(p.st[0].radix, RADSET, REALK, (c2r_first_stage<R, RAD>(p, lds, 0, src, dst)))
                 return;
             }
         }
-        FFTZ_RADIX_SWITCH(p.st[0].radix, ALLRAD, (single_stage<R, RAD, REAL, NT>(p, src, dst, l0, gin, gout)))
+        FFTZ_RADIX_SWITCH(p.st[0].radix, RADSET, (single_stage<R, RAD, REAL, NT>(p, src, dst, l0, gin, gout)))
         return;
     }
     const bool wave_local = p.TL <= 64 && !in_col && !out_col;
@@ -823,15 +833,15 @@ __device__ __forceinline__ void pass_body(const PassDesc& p, const TileIo& io, c
         if constexpr (REAL) {
             packed = (p.flags & kC2RPre) != 0;
             if (packed) {
-                FFTZ_PAIR_SWITCH(p.st[0].radix, ALLRAD, REALK, (c2r_first_stage<R, RAD>(p, line, ti, src, dst)))
+                FFTZ_PAIR_SWITCH(p.st[0].radix, RADSET, REALK, (c2r_first_stage<R, RAD>(p, line, ti, src, dst)))
             }
         }
         if (!packed) {
-            FFTZ_RADIX_SWITCH(p.st[0].radix, ALLRAD, (first_stage<R, RAD, REAL>(p, line, ti, src, gin)))
+            FFTZ_RADIX_SWITCH(p.st[0].radix, RADSET, (first_stage<R, RAD, REAL>(p, line, ti, src, gin)))
         }
     }
     for (int s = 1; s + 1 < S; s++)
-        mid_stage_any<R, ALLRAD, false>(p, lds + cr * p.LP, tr, s, cr < p.C, wave_local);
+        mid_stage_any<R, RADSET, false>(p, lds + cr * p.LP, tr, s, cr < p.C, wave_local);
     stage_sync(wave_local);
     if (in_col != out_col) {
         const SlotLine slo = slot_line(p, io, l_base, co);
@@ -847,14 +857,14 @@ __device__ __forceinline__ void pass_body(const PassDesc& p, const TileIo& io, c
     const cplx<R>* line = lds + co * p.LP;
     if constexpr (REAL) {
         if (p.flags & kR2CPost) {
-            FFTZ_PAIR_SWITCH(p.st[S - 1].radix, ALLRAD, REALK, (r2c_last_stage<R, RAD>(p, line, to, dst, src)))
+            FFTZ_PAIR_SWITCH(p.st[S - 1].radix, RADSET, REALK, (r2c_last_stage<R, RAD>(p, line, to, dst, src)))
             return;
         }
     }
-    FFTZ_RADIX_SWITCH(p.st[S - 1].radix, ALLRAD, (last_stage<R, RAD, REAL, NT>(p, line, to, dst, l0, gout)))
+    FFTZ_RADIX_SWITCH(p.st[S - 1].radix, RADSET, (last_stage<R, RAD, REAL, NT>(p, line, to, dst, l0, gout)))
 }
 
-template <typename R, bool ALLRAD, int REALK, bool NT, int MAXT>
+template <typename R, int RADSET, int REALK, bool NT, int MAXT>
 __global__ void __launch_bounds__(MAXT)
     __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 && REALK == kRealPair ? 4 : 1))) k_fft_pass(const PassDesc p_arg)
 {
@@ -863,7 +873,7 @@ __global__ void __launch_bounds__(MAXT)
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
     cplx<R>* lds = reinterpret_cast<cplx<R>*>(smem_raw);
     const int64_t l_base = (int64_t)tile_of_block(p) * p.C;
-    pass_body<R, ALLRAD, REALK, NT>(p, io_of(p), lds, l_base, threadIdx.x);
+    pass_body<R, RADSET, REALK, NT>(p, io_of(p), lds, l_base, threadIdx.x);
 }
 
 // ---------------------------------------------------------------------------
@@ -1008,7 +1018,7 @@ __device__ __forceinline__ void bs_final(const PassDesc& p, const cplx<R>* line,
     }
 }
 
-template <typename R, bool ALLRAD, bool NT>
+template <typename R, int RADSET, bool NT>
 __device__ __forceinline__ void bluestein_body(const PassDesc& p, const TileIo& io, cplx<R>* lds, int64_t l_base, int tid)
 {
     const int c = tid >> p.tl_shift;
@@ -1031,22 +1041,22 @@ __device__ __forceinline__ void bluestein_body(const PassDesc& p, const TileIo& 
     const bool wave_local = p.TL <= 64;
     cplx<R>* line = lds + c * p.LP;
     if (live) {
-        FFTZ_RADIX_SWITCH(p.st[0].radix, ALLRAD, (bs_first<R, RAD>(p, line, t, src)))
+        FFTZ_RADIX_SWITCH(p.st[0].radix, RADSET, (bs_first<R, RAD>(p, line, t, src)))
     }
-    for (int s = 1; s + 1 < S; s++) mid_stage_any<R, ALLRAD, false>(p, line, t, s, live, wave_local);
-    FFTZ_RADIX_SWITCH(p.st[S - 1].radix, ALLRAD, (bs_center<R, RAD>(p, line, t, live, wave_local)))
-    for (int s = S - 2; s >= 1; s--) mid_stage_any<R, ALLRAD, true>(p, line, t, s, live, wave_local);
-    FFTZ_RADIX_SWITCH(p.st[0].radix, ALLRAD, (bs_final<R, RAD, NT>(p, line, t, dst, live, wave_local)))
+    for (int s = 1; s + 1 < S; s++) mid_stage_any<R, RADSET, false>(p, line, t, s, live, wave_local);
+    FFTZ_RADIX_SWITCH(p.st[S - 1].radix, RADSET, (bs_center<R, RAD>(p, line, t, live, wave_local)))
+    for (int s = S - 2; s >= 1; s--) mid_stage_any<R, RADSET, true>(p, line, t, s, live, wave_local);
+    FFTZ_RADIX_SWITCH(p.st[0].radix, RADSET, (bs_final<R, RAD, NT>(p, line, t, dst, live, wave_local)))
 }
 
-template <typename R, bool ALLRAD, bool NT, int MAXT>
+template <typename R, int RADSET, bool NT, int MAXT>
 __global__ void __launch_bounds__(MAXT) k_bluestein(const PassDesc p_arg)
 {
     (void)p_arg;
     const PassDesc& p = kernarg_desc();
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
     cplx<R>* lds = reinterpret_cast<cplx<R>*>(smem_raw);
-    bluestein_body<R, ALLRAD, NT>(p, io_of(p), lds, (int64_t)blockIdx.x * p.C, threadIdx.x);
+    bluestein_body<R, RADSET, NT>(p, io_of(p), lds, (int64_t)blockIdx.x * p.C, threadIdx.x);
 }
 
 // ---------------------------------------------------------------------------
@@ -1088,9 +1098,9 @@ __global__ void __launch_bounds__(MAXT) k_batch(const BatchArgs a)
         // a queue entry covers one or more rounds of C lines
         for (int64_t lb = 0; lb < io.nlines; lb += C) {
             if (blue)
-                bluestein_body<R, true, true>(p, io, lds, lb, tid);
+                bluestein_body<R, kRadAll, true>(p, io, lds, lb, tid);
             else
-                pass_body<R, true, kRealNone, true>(p, io, lds, lb, tid);
+                pass_body<R, kRadAll, kRealNone, true>(p, io, lds, lb, tid);
             __syncthreads();
         }
         if (tid == 0) s_tile = nxt;
@@ -1106,23 +1116,31 @@ __global__ void __launch_bounds__(MAXT) k_batch(const BatchArgs a)
 template <typename R>
 constexpr int kBigBlock = sizeof(R) == 4 ? 1024 : 512;
 
-template <typename R, bool A, int T>
+template <typename R, int A>
+inline const void* sym_pass(bool nt, int maxt)
+{
+    if (maxt <= 256)
+        return nt ? (const void*)&k_fft_pass<R, A, kRealNone, true, 256>
+                  : (const void*)&k_fft_pass<R, A, kRealNone, false, 256>;
+    return nt ? (const void*)&k_fft_pass<R, A, kRealNone, true, kBigBlock<R>>
+              : (const void*)&k_fft_pass<R, A, kRealNone, false, kBigBlock<R>>;
+}
+
+template <typename R, int A, int T>
 inline const void* sym(KernelKind kind, bool nt)
 {
     constexpr int TR = T > kBigBlock<R> / 2 ? kBigBlock<R> / 2 : T;
     switch (kind) {
-        case KernelKind::Pass:
-            return nt ? (const void*)&k_fft_pass<R, A, kRealNone, true, T>
-                      : (const void*)&k_fft_pass<R, A, kRealNone, false, T>;
+        case KernelKind::Pass: return sym_pass<R, A>(nt, T);
         case KernelKind::Real: return (const void*)&k_fft_pass<R, A, kRealPair, false, TR>;
         case KernelKind::RealWide:
-            if constexpr (A) return (const void*)&k_fft_pass<R, A, kRealWide, false, TR>;
+            if constexpr (A == kRadAll) return (const void*)&k_fft_pass<R, A, kRealWide, false, TR>;
             return nullptr;
         default: return nt ? (const void*)&k_bluestein<R, A, true, T> : (const void*)&k_bluestein<R, A, false, T>;
     }
 }
 
-template <typename R, bool A>
+template <typename R, int A>
 inline const void* sym_t(KernelKind kind, bool nt, int maxt)
 {
     return maxt <= 256 ? sym<R, A, 256>(kind, nt) : sym<R, A, kBigBlock<R>>(kind, nt);

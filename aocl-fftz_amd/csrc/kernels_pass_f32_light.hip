@@ -1,0 +1,9 @@
+// Instantiation unit: single-size pass kernels with the radices of kRadLight,
+// complex64; 256- or 1024-thread bound.
+#include "kernels_body.h"
+
+namespace fftz {
+
+const void* kernel_symbol_pass_f32_light(bool nt, int maxt) { return sym_pass<float, kRadLight>(nt, maxt); }
+
+}  // namespace fftz

@@ -6,7 +6,7 @@ namespace fftz {
 
 const void* kernel_symbol_pass_f32_mixed(KernelKind kind, bool nt, int maxt)
 {
-    return sym_t<float, true>(kind, nt, maxt);
+    return sym_t<float, kRadAll>(kind, nt, maxt);
 }
 
 }  // namespace fftz

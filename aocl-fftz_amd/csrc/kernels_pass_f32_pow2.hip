@@ -6,7 +6,7 @@ namespace fftz {
 
 const void* kernel_symbol_pass_f32_pow2(KernelKind kind, bool nt, int maxt)
 {
-    return sym_t<float, false>(kind, nt, maxt);
+    return sym_t<float, kRadPow2>(kind, nt, maxt);
 }
 
 }  // namespace fftz

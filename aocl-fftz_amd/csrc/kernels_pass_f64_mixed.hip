@@ -6,7 +6,7 @@ namespace fftz {
 
 const void* kernel_symbol_pass_f64_mixed(KernelKind kind, bool nt, int maxt)
 {
-    return sym_t<double, true>(kind, nt, maxt);
+    return sym_t<double, kRadAll>(kind, nt, maxt);
 }
 
 }  // namespace fftz

@@ -51,11 +51,11 @@ const DeviceInfo& device_info()
         info.warp = prop.warpSize;
         // Allow every kernel to use the full LDS of a workgroup.
         for (int prec : {4, 8})
-            for (bool all : {false, true})
+            for (int rad : {kRadPow2, kRadAll, kRadLight})
                 for (KernelKind k : {KernelKind::Pass, KernelKind::Real, KernelKind::RealWide, KernelKind::Bluestein})
                     for (bool nt : {false, true})
                         for (int t : {256, 1024})
-                            if (const void* f = kernel_symbol(k, prec, all, nt, t))
+                            if (const void* f = kernel_symbol(k, prec, rad, nt, t))
                                 (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize,
                                                           (int)info.lds_per_block);
         for (int prec : {4, 8})
@@ -665,11 +665,18 @@ static bool build_pass(Plan* plan, TableBuilder& tb, const PassReq& q, std::stri
             !(r2c && tr->back() > 10) && !(c2r && tr->front() > 10))
             radix = *tr;
     d.nst = (int)radix.size();
-    ln.all_radix = false;
+    // Plain complex64 lines without 11, 13 and 16 take the kernel that does not
+    // carry them: five wavefronts per SIMD in place of four.  3001 x 1200 points
+    // 16.2 -> 15.4 us, 1080x1920 grids 266 -> 259.  Complex128 would go from two
+    // to three (208 -> 168 VGPRs), but its 120- and 100-point columns measured
+    // no gain (100x120x144 91.7 -> 92.7), so it has no such kernel.
+    bool pow2_only = true, light = prec == 4 && q.kind == KernelKind::Pass && !(q.flags & kRealFlags);
     for (size_t s = 0; s < radix.size(); s++) {
         d.radix[s] = radix[s];
-        if (radix[s] != 2 && radix[s] != 4 && radix[s] != 8 && radix[s] != 16) ln.all_radix = true;
+        if (radix[s] != 2 && radix[s] != 4 && radix[s] != 8 && radix[s] != 16) pow2_only = false;
+        if (radix[s] == 11 || radix[s] == 13 || radix[s] == 16) light = false;
     }
+    ln.rad = light ? kRadLight : pow2_only ? kRadPow2 : kRadAll;
     // a tuned number of values per thread
     const int tuned_e = plan->spec.tune.elems ? plan->spec.tune.elems : env_int("FFTZ_E", 0);
     const int need = q.L + q.extra_lds_elems;
@@ -2436,7 +2443,7 @@ static hipError_t launch_all(Plan* p, void* work, unsigned* counters, const void
         void* args[] = {&d, &frag};
         const void* fn = ln.mfma ? kernel_symbol_mfma(ln.mfma, ln.d.L, ln.mfma_nb)
                          : ln.fixed ? kernel_symbol_fixed(p->spec.prec_bytes, ln.d.L, ln.maxt, ln.split)
-                                    : kernel_symbol(pass_kind(ln), p->spec.prec_bytes, ln.all_radix,
+                                    : kernel_symbol(pass_kind(ln), p->spec.prec_bytes, ln.rad,
                                                     (d.flags & kNtStore) != 0, ln.maxt);
         hipError_t e = hipLaunchKernel(fn, dim3(ln.grid), dim3(ln.block), args,
                                        ln.split ? ln.lds_bytes / 2 : ln.lds_bytes, stream);

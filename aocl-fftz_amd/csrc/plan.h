@@ -76,7 +76,7 @@ struct BatchClass {
 
 struct Launch {
     KernelKind kind = KernelKind::Pass;
-    bool all_radix = false;
+    int rad = kRadPow2;  // RadixSet of a generic kernel
     int E = 16;        // complex values of a line per thread
     int maxt = 256;    // block-size bound of the kernel variant
     bool fixed = false;  // fixed-length kernel (kernels_fixed.hip)
