@@ -7,11 +7,28 @@ namespace fftz {
 
 enum class KernelKind { Pass, Real, RealWide, Bluestein };
 
-// Radices a generic kernel carries: 2, 4, 8, 16; all of 2 .. 13 and 16; or all
-// but 11, 13 and 16 (complex64 plain passes only).  The registers of the widest
-// butterfly set the wavefronts of every launch: 112 with all radices (four
-// wavefronts per SIMD), 88 without those three (five).
-enum RadixSet : int { kRadPow2 = 0, kRadAll = 1, kRadLight = 2 };
+// Radices a generic kernel carries.  The widest butterfly it carries sets the
+// registers, and with them the wavefronts, of every launch; wavefronts per SIMD
+// of the plain pass and of Bluestein in complex64 / complex128: kRadAll 4 / 2,
+// kRadLight 5 / 3, kRadTo8 - / 4.
+enum RadixSet : int {
+    kRadPow2 = 0,   // 2, 4, 8, 16
+    kRadAll = 1,    // 2 .. 13, 16
+    kRadLight = 2,  // 2 .. 12; no real passes
+    kRadTo8 = 3,    // 2 .. 8, complex128 only; mirrored pairs of radix 2 .. 6
+};
+
+constexpr bool rad_in_set(int set, int r)
+{
+    return set == kRadPow2    ? (r & (r - 1)) == 0
+           : set == kRadLight ? r <= 12
+           : set == kRadTo8   ? r <= 8
+                              : true;
+}
+
+// Radices of the stage that holds mirrored butterfly pairs (two butterflies'
+// registers at once).
+constexpr bool rad_in_pairs(int set, int r) { return r <= (set == kRadTo8 ? 6 : 10) && rad_in_set(set, r); }
 
 // Device function symbol for hipLaunchKernel / hipFuncSetAttribute; nullptr
 // where there is no such kernel.  prec_bytes: 4 (complex64) or 8 (complex128).
@@ -35,7 +52,9 @@ const void* kernel_symbol_pass_f32_mixed(KernelKind kind, bool nt, int maxt);
 const void* kernel_symbol_pass_f32_pow2(KernelKind kind, bool nt, int maxt);
 const void* kernel_symbol_pass_f64_mixed(KernelKind kind, bool nt, int maxt);
 const void* kernel_symbol_pass_f64_pow2(KernelKind kind, bool nt, int maxt);
-const void* kernel_symbol_pass_f32_light(bool nt, int maxt);
+const void* kernel_symbol_pass_f32_light(KernelKind kind, bool nt, int maxt);
+const void* kernel_symbol_pass_f64_light(KernelKind kind, bool nt, int maxt);
+const void* kernel_symbol_pass_f64_to8(KernelKind kind, bool nt, int maxt);
 const void* kernel_symbol_batch_f32_small();
 const void* kernel_symbol_batch_f32_medium();
 const void* kernel_symbol_batch_f32_large();

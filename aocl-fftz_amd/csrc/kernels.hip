@@ -18,14 +18,19 @@ __global__ void k_reset_counters(unsigned* c, int n)
 
 const void* kernel_symbol(KernelKind kind, int prec_bytes, int rad, bool nt, int maxt)
 {
-    if (rad == kRadLight) {
-        if (kind != KernelKind::Pass || prec_bytes != 4) return nullptr;
-        return kernel_symbol_pass_f32_light(nt, maxt);
+    if (prec_bytes == 4) switch (rad) {
+            case kRadPow2: return kernel_symbol_pass_f32_pow2(kind, nt, maxt);
+            case kRadAll: return kernel_symbol_pass_f32_mixed(kind, nt, maxt);
+            case kRadLight: return kernel_symbol_pass_f32_light(kind, nt, maxt);
+            default: return nullptr;
+        }
+    switch (rad) {
+        case kRadPow2: return kernel_symbol_pass_f64_pow2(kind, nt, maxt);
+        case kRadAll: return kernel_symbol_pass_f64_mixed(kind, nt, maxt);
+        case kRadLight: return kernel_symbol_pass_f64_light(kind, nt, maxt);
+        case kRadTo8: return kernel_symbol_pass_f64_to8(kind, nt, maxt);
+        default: return nullptr;
     }
-    if (prec_bytes == 4)
-        return rad == kRadAll ? kernel_symbol_pass_f32_mixed(kind, nt, maxt)
-                              : kernel_symbol_pass_f32_pow2(kind, nt, maxt);
-    return rad == kRadAll ? kernel_symbol_pass_f64_mixed(kind, nt, maxt) : kernel_symbol_pass_f64_pow2(kind, nt, maxt);
 }
 
 const void* kernel_symbol_batch(int prec_bytes, int cls)

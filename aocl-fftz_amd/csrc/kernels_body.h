@@ -24,8 +24,8 @@
 // self-sorting geometry, core/solvers/complex/pow2_iterative_solver_dft.c:27-78,
 // moves every stage's results instead.)
 //
-// Included by the instantiation units kernels_pass_{f32,f64}_{mixed,pow2}.hip
-// and kernels_batch_{f32,f64}_{small,medium,large}.hip (compiled in
+// Included by the instantiation units kernels_pass_{f32,f64}_{mixed,pow2,light}.hip,
+// kernels_pass_f64_to8.hip and kernels_batch_{f32,f64}_{small,medium,large}.hip (compiled in
 // parallel); kernels.hip holds the launch-table dispatch.
 #pragma once
 
@@ -218,74 +218,62 @@ __device__ __forceinline__ void mid_stage(const PassDesc& p, cplx<R>* line, int 
     }
 }
 
-#define FFTZ_RADIX_CASE(r, CALL) \
-    case r: {                    \
-        constexpr int RAD = r;   \
-        CALL;                    \
-    } break;
+#define FFTZ_RADIX_CASE(RADSET, r, CALL)            \
+    case r:                                         \
+        if constexpr (rad_in_set((RADSET), r)) {    \
+            constexpr int RAD = r;                  \
+            CALL;                                   \
+        }                                           \
+        break;
 
-#define FFTZ_RADIX_SWITCH(rad, RADSET, CALL)       \
-    switch (rad) {                                 \
-        FFTZ_RADIX_CASE(2, CALL)                   \
-        FFTZ_RADIX_CASE(4, CALL)                   \
-        FFTZ_RADIX_CASE(8, CALL)                   \
-        case 16:                                   \
-            if constexpr (RADSET != kRadLight) {   \
-                constexpr int RAD = 16;            \
-                CALL;                              \
-            }                                      \
-            break;                                 \
-        default:                                   \
-            if constexpr (RADSET != kRadPow2) {    \
-                switch (rad) {                     \
-                    FFTZ_RADIX_CASE(3, CALL)       \
-                    FFTZ_RADIX_CASE(5, CALL)       \
-                    FFTZ_RADIX_CASE(6, CALL)       \
-                    FFTZ_RADIX_CASE(7, CALL)       \
-                    FFTZ_RADIX_CASE(9, CALL)       \
-                    FFTZ_RADIX_CASE(10, CALL)      \
-                    FFTZ_RADIX_CASE(12, CALL)      \
-                    default: break;                \
-                }                                  \
-                if constexpr (RADSET == kRadAll) { \
-                    switch (rad) {                 \
-                        FFTZ_RADIX_CASE(11, CALL)  \
-                        FFTZ_RADIX_CASE(13, CALL)  \
-                        default: break;            \
-                    }                              \
-                }                                  \
-            }                                      \
-            break;                                 \
+#define FFTZ_RADIX_SWITCH(rad, RADSET, CALL)        \
+    switch (rad) {                                  \
+        FFTZ_RADIX_CASE(RADSET, 2, CALL)            \
+        FFTZ_RADIX_CASE(RADSET, 3, CALL)            \
+        FFTZ_RADIX_CASE(RADSET, 4, CALL)            \
+        FFTZ_RADIX_CASE(RADSET, 5, CALL)            \
+        FFTZ_RADIX_CASE(RADSET, 6, CALL)            \
+        FFTZ_RADIX_CASE(RADSET, 7, CALL)            \
+        FFTZ_RADIX_CASE(RADSET, 8, CALL)            \
+        FFTZ_RADIX_CASE(RADSET, 9, CALL)            \
+        FFTZ_RADIX_CASE(RADSET, 10, CALL)           \
+        FFTZ_RADIX_CASE(RADSET, 11, CALL)           \
+        FFTZ_RADIX_CASE(RADSET, 12, CALL)           \
+        FFTZ_RADIX_CASE(RADSET, 13, CALL)           \
+        FFTZ_RADIX_CASE(RADSET, 16, CALL)           \
+        default: break;                             \
     }
 
 // Radices of the stage that holds mirrored butterfly pairs (kRealPair: up to
 // 10, kRealWide: 11 and 13).
-#define FFTZ_PAIR_SWITCH(rad, RADSET, REAL, CALL)  \
-    if constexpr (REAL == kRealWide) {             \
-        switch (rad) {                             \
-            FFTZ_RADIX_CASE(11, CALL)              \
-            FFTZ_RADIX_CASE(13, CALL)              \
-            default: break;                        \
-        }                                          \
-    } else {                                       \
-        switch (rad) {                             \
-            FFTZ_RADIX_CASE(2, CALL)               \
-            FFTZ_RADIX_CASE(4, CALL)               \
-            FFTZ_RADIX_CASE(8, CALL)               \
-            default:                               \
-                if constexpr (RADSET != kRadPow2) { \
-                    switch (rad) {                 \
-                        FFTZ_RADIX_CASE(3, CALL)   \
-                        FFTZ_RADIX_CASE(5, CALL)   \
-                        FFTZ_RADIX_CASE(6, CALL)   \
-                        FFTZ_RADIX_CASE(7, CALL)   \
-                        FFTZ_RADIX_CASE(9, CALL)   \
-                        FFTZ_RADIX_CASE(10, CALL)  \
-                        default: break;            \
-                    }                              \
-                }                                  \
-                break;                             \
-        }                                          \
+#define FFTZ_PAIR_CASE(RADSET, r, CALL)             \
+    case r:                                         \
+        if constexpr (rad_in_pairs((RADSET), r)) {  \
+            constexpr int RAD = r;                  \
+            CALL;                                   \
+        }                                           \
+        break;
+
+#define FFTZ_PAIR_SWITCH(rad, RADSET, REAL, CALL)   \
+    if constexpr (REAL == kRealWide) {              \
+        switch (rad) {                              \
+            FFTZ_RADIX_CASE(kRadAll, 11, CALL)      \
+            FFTZ_RADIX_CASE(kRadAll, 13, CALL)      \
+            default: break;                         \
+        }                                           \
+    } else {                                        \
+        switch (rad) {                              \
+            FFTZ_PAIR_CASE(RADSET, 2, CALL)         \
+            FFTZ_PAIR_CASE(RADSET, 3, CALL)         \
+            FFTZ_PAIR_CASE(RADSET, 4, CALL)         \
+            FFTZ_PAIR_CASE(RADSET, 5, CALL)         \
+            FFTZ_PAIR_CASE(RADSET, 6, CALL)         \
+            FFTZ_PAIR_CASE(RADSET, 7, CALL)         \
+            FFTZ_PAIR_CASE(RADSET, 8, CALL)         \
+            FFTZ_PAIR_CASE(RADSET, 9, CALL)         \
+            FFTZ_PAIR_CASE(RADSET, 10, CALL)        \
+            default: break;                         \
+        }                                           \
     }
 
 // ---------------------------------------------------------------------------
@@ -866,7 +854,7 @@ __device__ __forceinline__ void pass_body(const PassDesc& p, const TileIo& io, c
 
 template <typename R, int RADSET, int REALK, bool NT, int MAXT>
 __global__ void __launch_bounds__(MAXT)
-    __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 && REALK == kRealPair ? 4 : 1))) k_fft_pass(const PassDesc p_arg)
+    __attribute__((amdgpu_waves_per_eu(REALK == kRealNone ? (RADSET == kRadLight && sizeof(R) == 8 ? 3 : 1) : REALK == kRealWide ? 1 : sizeof(R) == 4 ? 4 : RADSET == kRadTo8 ? 3 : 2))) k_fft_pass(const PassDesc p_arg)
 {
     (void)p_arg;
     const PassDesc& p = kernarg_desc();
@@ -1116,23 +1104,17 @@ __global__ void __launch_bounds__(MAXT) k_batch(const BatchArgs a)
 template <typename R>
 constexpr int kBigBlock = sizeof(R) == 4 ? 1024 : 512;
 
-template <typename R, int A>
-inline const void* sym_pass(bool nt, int maxt)
-{
-    if (maxt <= 256)
-        return nt ? (const void*)&k_fft_pass<R, A, kRealNone, true, 256>
-                  : (const void*)&k_fft_pass<R, A, kRealNone, false, 256>;
-    return nt ? (const void*)&k_fft_pass<R, A, kRealNone, true, kBigBlock<R>>
-              : (const void*)&k_fft_pass<R, A, kRealNone, false, kBigBlock<R>>;
-}
-
 template <typename R, int A, int T>
 inline const void* sym(KernelKind kind, bool nt)
 {
     constexpr int TR = T > kBigBlock<R> / 2 ? kBigBlock<R> / 2 : T;
     switch (kind) {
-        case KernelKind::Pass: return sym_pass<R, A>(nt, T);
-        case KernelKind::Real: return (const void*)&k_fft_pass<R, A, kRealPair, false, TR>;
+        case KernelKind::Pass:
+            return nt ? (const void*)&k_fft_pass<R, A, kRealNone, true, T>
+                      : (const void*)&k_fft_pass<R, A, kRealNone, false, T>;
+        case KernelKind::Real:
+            if constexpr (A != kRadLight) return (const void*)&k_fft_pass<R, A, kRealPair, false, TR>;
+            return nullptr;
         case KernelKind::RealWide:
             if constexpr (A == kRadAll) return (const void*)&k_fft_pass<R, A, kRealWide, false, TR>;
             return nullptr;

@@ -4,6 +4,9 @@
 
 namespace fftz {
 
-const void* kernel_symbol_pass_f32_light(bool nt, int maxt) { return sym_pass<float, kRadLight>(nt, maxt); }
+const void* kernel_symbol_pass_f32_light(KernelKind kind, bool nt, int maxt)
+{
+    return sym_t<float, kRadLight>(kind, nt, maxt);
+}
 
 }  // namespace fftz

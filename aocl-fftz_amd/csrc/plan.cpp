@@ -51,7 +51,7 @@ const DeviceInfo& device_info()
         info.warp = prop.warpSize;
         // Allow every kernel to use the full LDS of a workgroup.
         for (int prec : {4, 8})
-            for (int rad : {kRadPow2, kRadAll, kRadLight})
+            for (int rad : {kRadPow2, kRadAll, kRadLight, kRadTo8})
                 for (KernelKind k : {KernelKind::Pass, KernelKind::Real, KernelKind::RealWide, KernelKind::Bluestein})
                     for (bool nt : {false, true})
                         for (int t : {256, 1024})
@@ -368,15 +368,13 @@ static int64_t stage_twiddles(TableBuilder& tb, int prec, const std::vector<int>
 //     column tile fills a wavefront (mint).
 //   * At most 16 elements per thread: beyond that too few wavefronts fit next
 //     to the lines' LDS (1,000,000-point complex64, passes of 100: 12 per
-//     thread 97 us, 25 per thread 104 us).  Short complex128 lines may take up
-//     to 32, for at least 15% less work: their registers allow no more than
-//     eight wavefronts per CU in any case (100 x 120 x 144 grid, pass of 100:
-//     25 per thread 16.6 us, 12 per thread 18.7 us).
+//     thread 97 us, 25 per thread 104 us; 100 x 120 x 144 complex128 grid, 12
+//     and 16 per thread 84.7 us, 25 to 32 per thread 87.1 us).
 //   * Among the widths within 8% of the least work, short lines take the
 //     narrowest (room for more lines) and long ones and pair stages the widest
 //     (more loads in flight per line).
 //   * Where the lines are too few for eight wavefronts per CU (two in
-//     complex128, which holds eight at most), wider, up to 1.6 times the least
+//     complex128), wider, up to 1.6 times the least
 //     work: the launch is latency-bound.
 // lines: how many there are; pair: the stage whose threads take two
 // butterflies at a time, or -1.
@@ -394,9 +392,8 @@ static int line_threads(const std::vector<int>& radix, int L, int mint, int maxt
         }
         return tl * 16 < L ? 1.15 * w : w;
     };
-    const int most = prec == 8 && L <= 128 ? 32 : 16;
     int first = 1;
-    while (first < widest && (first * most < L || first < mint)) first *= 2;
+    while (first < widest && (first * 16 < L || first < mint)) first *= 2;
     double least = 1e300;
     for (int tl = first; tl <= widest; tl *= 2) least = std::min(least, work(tl));
     int tl = first;
@@ -665,18 +662,21 @@ static bool build_pass(Plan* plan, TableBuilder& tb, const PassReq& q, std::stri
             !(r2c && tr->back() > 10) && !(c2r && tr->front() > 10))
             radix = *tr;
     d.nst = (int)radix.size();
-    // Plain complex64 lines without 11, 13 and 16 take the kernel that does not
-    // carry them: five wavefronts per SIMD in place of four.  3001 x 1200 points
-    // 16.2 -> 15.4 us, 1080x1920 grids 266 -> 259.  Complex128 would go from two
-    // to three (208 -> 168 VGPRs), but its 120- and 100-point columns measured
-    // no gain (100x120x144 91.7 -> 92.7), so it has no such kernel.
-    bool pow2_only = true, light = prec == 4 && q.kind == KernelKind::Pass && !(q.flags & kRealFlags);
-    for (size_t s = 0; s < radix.size(); s++) {
-        d.radix[s] = radix[s];
-        if (radix[s] != 2 && radix[s] != 4 && radix[s] != 8 && radix[s] != 16) pow2_only = false;
-        if (radix[s] == 11 || radix[s] == 13 || radix[s] == 16) light = false;
+    // The narrowest radix set that holds the line's radices: its kernel has the
+    // fewest registers.  Complex128, all radices -> set: 100 x 120 x 144 grid
+    // 91 -> 85 us (kRadLight), 2048 x 675 real batch of 4 214 -> 155 us
+    // (kRadTo8), 2894 lines of 1372 47.7 -> 41 us; complex64: 3001 lines of 1200
+    // 14.9 -> 14.1 us.  A complex64 set of radices up to 8 would save no
+    // wavefront worth having over kRadLight (78 against 92 VGPRs).
+    const bool real = q.kind == KernelKind::Pass && (q.flags & kRealFlags);
+    for (int set : {kRadAll, kRadPow2, kRadLight, kRadTo8}) {
+        if ((set == kRadLight && real) || (set == kRadTo8 && prec == 4)) continue;
+        const int pair = radix.empty() ? 1 : r2c ? radix.back() : c2r ? radix.front() : 1;  // one point: no stage
+        bool fits = rad_in_pairs(set, pair);
+        for (int r : radix) fits = fits && rad_in_set(set, r);
+        if (fits || set == kRadAll) ln.rad = set;
     }
-    ln.rad = light ? kRadLight : pow2_only ? kRadPow2 : kRadAll;
+    for (size_t s = 0; s < radix.size(); s++) d.radix[s] = radix[s];
     // a tuned number of values per thread
     const int tuned_e = plan->spec.tune.elems ? plan->spec.tune.elems : env_int("FFTZ_E", 0);
     const int need = q.L + q.extra_lds_elems;
