@@ -869,7 +869,10 @@ static bool build_pass(Plan* plan, TableBuilder& tb, const PassReq& q, std::stri
     }
     ln.grid = (uint32_t)tiles;
     ln.lds_bytes = (uint32_t)((size_t)C * line_bytes);
-    ln.split = ln.fixed && (in_col || out_col) && q.L == (prec == 4 ? 512 : 256);
+    // Exchange in halves only where more tiles than the two per CU that the
+    // full exchange holds are waiting: 28 x 65536 complex128 (448 tiles a pass)
+    // 27.9 us with it, 26.9 us without.
+    ln.split = ln.fixed && (in_col || out_col) && q.L == (prec == 4 ? 512 : 256) && tiles > 2 * dev.cus;
     if (use_mfma) ln.lds_bytes += 64;  // per-wavefront maxima of the fp16 line scale
     // XCD-contiguous tile order: measured to help passes that read rows and
     // store columns (the four-step's transposing last pass) and to cost ~5%
