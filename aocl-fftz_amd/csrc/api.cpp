@@ -652,7 +652,7 @@ const FFTZ_CHAR* aoclfftz_gpu_plan_info(FFTZ_VOID* handle)
            << " L=" << ln.d.L << " r=";
         for (int s = 0; s < ln.d.nst; s++) os << (s ? "x" : "") << ln.d.radix[s];
         os << " C=" << ln.d.C << " TL=" << ln.d.TL << " grid=" << ln.grid << " block=" << ln.block
-           << " lds=" << ln.lds_bytes << ((ln.d.flags & fftz::kInCol) ? " incol" : "")
+           << " lds=" << ln.launched_lds() << (ln.split ? " split" : "") << ((ln.d.flags & fftz::kNtStore) ? " nt" : "") << ((ln.d.flags & fftz::kInCol) ? " incol" : "")
            << ((ln.d.flags & fftz::kOutCol) ? " outcol" : "") << ((ln.d.flags & fftz::kTw4) ? " tw4" : "") << "]";
     }
     os << " work=" << p->work_bytes;

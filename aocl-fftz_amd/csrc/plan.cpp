@@ -2262,16 +2262,38 @@ static std::string batch_json(const Plan* p)
     os << "],\"classes\":[";
     for (size_t c = 0; c < p->bclasses.size(); c++) {
         const BatchClass& bc = p->bclasses[c];
-        os << (c ? "," : "") << "{\"maxt\":" << bc.maxt << ",\"lds\":" << bc.lds_bytes
+        // complex values of a line per thread: the most in this class
+        const BatchTile* q = hd ? reinterpret_cast<const BatchTile*>(p->host_tables.data() + bc.tiles_off) : nullptr;
+        int E = 0;
+        for (int i = 0; q && i < bc.ntiles; i++) {
+            const PassDesc& d = hd[q[i].desc];
+            E = std::max(E, (d.L + d.TL - 1) / d.TL);
+        }
+        os << (c ? "," : "") << "{\"E\":" << E << ",\"maxt\":" << bc.maxt << ",\"lds\":" << bc.lds_bytes
            << ",\"grid\":" << bc.grid << ",\"tiles\":[";
-        const BatchTile* t = hd ? reinterpret_cast<const BatchTile*>(p->host_tables.data() + bc.tiles_off) : nullptr;
-        for (int i = 0; t && i < bc.ntiles; i++)
-            os << (i ? "," : "") << "[" << t[i].desc << "," << t[i].nlines << "," << t[i].bluestein << ","
-               << t[i].in_off << "," << t[i].out_off << "," << t[i].dist << "]";
+        for (int i = 0; q && i < bc.ntiles; i++)
+            os << (i ? "," : "") << "[" << q[i].desc << "," << q[i].nlines << "," << q[i].bluestein << ","
+               << q[i].in_off << "," << q[i].out_off << "," << q[i].dist << "]";
         os << "]}";
     }
     os << "]}";
     return os.str();
+}
+
+static KernelKind pass_kind(const Launch& ln);
+
+// Kernel form of a launch: the fixed-length and matrix-core kernels, or the generic
+// kernel's (KernelKind).
+static const char* form_name(const Launch& ln)
+{
+    if (ln.mfma) return "mfma";
+    if (ln.fixed) return "fixed";
+    switch (pass_kind(ln)) {
+        case KernelKind::Bluestein: return "bluestein";
+        case KernelKind::Real: return "real";
+        case KernelKind::RealWide: return "real_wide";
+        default: return "pass";
+    }
 }
 
 std::string plan_json(const Plan* p)
@@ -2292,13 +2314,17 @@ std::string plan_json(const Plan* p)
            << ",\"flags\":" << d.flags << ",\"C\":" << d.C << ",\"TL\":" << d.TL << ",\"LP\":" << d.LP
            << ",\"vrow\":" << d.vrow.d << ",\"maxt\":" << ln.maxt
            << ",\"E\":" << ln.E << ",\"fixed\":" << (ln.fixed ? 1 : 0) << ",\"mfma\":" << ln.mfma << ",\"grid\":" << ln.grid << ",\"block\":" << ln.block
-           << ",\"lds\":" << ln.lds_bytes << ",\"in_role\":" << (int)ln.in_role
+           << ",\"rad\":" << ln.rad << ",\"form\":\"" << form_name(ln) << "\",\"split\":" << (ln.split ? 1 : 0)
+           << ",\"nt\":" << ((d.flags & kNtStore) ? 1 : 0) << ",\"lds\":" << ln.lds_bytes
+           << ",\"lds_launched\":" << ln.launched_lds() << ",\"in_role\":" << (int)ln.in_role
            << ",\"out_role\":" << (int)ln.out_role << ",\"in_off\":" << ln.in_off_bytes
            << ",\"out_off\":" << ln.out_off_bytes << ",\"tw4_n\":" << d.tw4_n << ",\"nchirp\":" << d.nchirp
            << ",\"gin\":[" << d.gin[0] << "," << d.gin[1] << "," << d.gin[2] << "," << d.gin[3] << "],\"gout\":["
            << d.gout[0] << "," << d.gout[1] << "," << d.gout[2] << "," << d.gout[3] << "],\"gin_base\":" << d.gin_base
            << ",\"gout_base\":" << d.gout_base << ",\"radix\":[";
         for (int s = 0; s < d.nst; s++) os << (s ? "," : "") << d.radix[s];
+        os << "],\"ls\":[";
+        for (int s = 0, ls = 1; s < d.nst; ls *= d.radix[s++]) os << (s ? "," : "") << ls;
         os << "]}";
         first = false;
     }
@@ -2449,7 +2475,7 @@ static hipError_t launch_all(Plan* p, void* work, unsigned* counters, const void
                                     : kernel_symbol(pass_kind(ln), p->spec.prec_bytes, ln.rad,
                                                     (d.flags & kNtStore) != 0, ln.maxt);
         hipError_t e = hipLaunchKernel(fn, dim3(ln.grid), dim3(ln.block), args,
-                                       ln.split ? ln.lds_bytes / 2 : ln.lds_bytes, stream);
+                                       ln.launched_lds(), stream);
         if (e != hipSuccess) return e;
         if (prof) {
             e = record_prof(p, stream);

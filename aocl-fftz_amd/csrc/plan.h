@@ -86,7 +86,8 @@ struct Launch {
     PassDesc d{};
     Role in_role = Role::In, out_role = Role::Out;
     int64_t in_off_bytes = 0, out_off_bytes = 0;
-    uint32_t grid = 0, block = 0, lds_bytes = 0;
+    uint32_t grid = 0, block = 0, lds_bytes = 0;  // lds_bytes: the whole tile
+    uint32_t launched_lds() const { return split ? lds_bytes / 2 : lds_bytes; }
     // table offsets in the plan arena (-1: none), resolved after upload
     int64_t stw_off = -1, tw4_off = -1, chirp_off = -1, spec_off = -1, rtw_off = -1;
     int64_t frag_off = -1;  // MFMA DFT-16 operand fragments (64 lanes x 32 floats)
