@@ -36,8 +36,8 @@ constexpr bool rad_in_pairs(int set, int r) { return r <= (set == kRadTo8 ? 6 : 
 // write-back (kNtStore).  maxt: block-size bound of the variant, 256 or more
 // (then 1024 threads in complex64, 512 in complex128); the 256 variants get a
 // larger VGPR budget.  Real: passes with a real side (kRealFlags); RealWide:
-// real-packed ones whose pair stage (last for R2C, first for C2R) has radix 11
-// or 13.
+// real-packed ones whose pair stage (last for R2C, first for C2R) has a radix
+// above 10: 11 or 13 where the length has no other, any in a tuned order.
 const void* kernel_symbol(KernelKind kind, int prec_bytes, int rad, bool nt, int maxt);
 
 // Uneven-batch persistent kernel (k_batch) of a tile class (0 small: 256

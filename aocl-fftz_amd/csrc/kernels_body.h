@@ -245,7 +245,7 @@ __device__ __forceinline__ void mid_stage(const PassDesc& p, cplx<R>* line, int 
     }
 
 // Radices of the stage that holds mirrored butterfly pairs (kRealPair: up to
-// 10, kRealWide: 11 and 13).
+// 10, kRealWide: 11 and 13, and 12 and 16 where a tuned order asks for them).
 #define FFTZ_PAIR_CASE(RADSET, r, CALL)             \
     case r:                                         \
         if constexpr (rad_in_pairs((RADSET), r)) {  \
@@ -258,7 +258,9 @@ __device__ __forceinline__ void mid_stage(const PassDesc& p, cplx<R>* line, int 
     if constexpr (REAL == kRealWide) {              \
         switch (rad) {                              \
             FFTZ_RADIX_CASE(kRadAll, 11, CALL)      \
+            FFTZ_RADIX_CASE(kRadAll, 12, CALL)      \
             FFTZ_RADIX_CASE(kRadAll, 13, CALL)      \
+            FFTZ_RADIX_CASE(kRadAll, 16, CALL)      \
             default: break;                         \
         }                                           \
     } else {                                        \
@@ -759,7 +761,7 @@ __device__ __forceinline__ void mid_stage_any(const PassDesc& p, cplx<R>* line, 
 }
 
 // Forms of the generic pass kernel: complex on both sides; a real side, with
-// pair stages of radix <= 10; the same with pair stages of radix 11 or 13.
+// pair stages of radix <= 10; the same with wider pair stages.
 enum RealForm : int { kRealNone = 0, kRealPair = 1, kRealWide = 2 };
 
 // One tile: C lines, threads (c, t) per side's mapping -- row (a wavefront

@@ -658,9 +658,7 @@ static bool build_pass(Plan* plan, TableBuilder& tb, const PassReq& q, std::stri
     const bool r2c = (q.flags & kR2CPost) != 0, c2r = (q.flags & kC2RPre) != 0;
     if (r2c || c2r) radix = packed_radices(q.L, radix, c2r);
     if (const std::vector<int>* tr = plan->spec.tune.radices(q.L))
-        if (q.kind == KernelKind::Pass && plan->spec.mfma_mode == kMfmaNone && radix_order_ok(q.L, *tr) &&
-            !(r2c && tr->back() > 10) && !(c2r && tr->front() > 10))
-            radix = *tr;
+        if (q.kind == KernelKind::Pass && plan->spec.mfma_mode == kMfmaNone && radix_order_ok(q.L, *tr)) radix = *tr;
     d.nst = (int)radix.size();
     // The narrowest radix set that holds the line's radices: its kernel has the
     // fewest registers.  Complex128, all radices -> set: 100 x 120 x 144 grid
