@@ -73,10 +73,6 @@ __device__ __forceinline__ void store_nt(cplx<R>* p, cplx<R> v)
     __builtin_nontemporal_store(w, reinterpret_cast<vec*>(p));
 }
 
-// Around the stores of a branch that differs from its sibling only in store_nt:
-// without it the optimiser merges the two branches into ordinary stores.
-__device__ __forceinline__ void keep_branch() { asm volatile("" ::: "memory"); }
-
 template <int R_, typename R>
 struct Dft;
 

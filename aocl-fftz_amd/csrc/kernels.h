@@ -66,8 +66,8 @@ const void* kernel_symbol_batch_f64_large();
 // then remainder, 16 elements per thread), block <= maxt (256, or 512 for
 // L >= 256); nullptr otherwise.  split (complex64 L = 512, complex128 L = 256):
 // stage exchanges of the real and the imaginary parts in turn, through half
-// the LDS.
-const void* kernel_symbol_fixed(int prec_bytes, int L, int maxt, bool split);
+// the LDS.  nt: results bypass the L2's write-back.
+const void* kernel_symbol_fixed(int prec_bytes, int L, int maxt, bool split, bool nt);
 
 // Matrix-core pass (kernels_mfma.hip) for complex64, L = 256 or 4096, with
 // operand precision `mode` (MfmaMode) and nb (2 or 4) column blocks per

@@ -62,9 +62,10 @@ const DeviceInfo& device_info()
             for (int L = 64; L <= 4096; L *= 2)
                 for (int t : {256, 512})
                     for (bool split : {false, true})
-                        if (const void* f = kernel_symbol_fixed(prec, L, t, split))
-                            (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                      (int)info.lds_per_block);
+                        for (bool nt : {false, true})
+                            if (const void* f = kernel_symbol_fixed(prec, L, t, split, nt))
+                                (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                          (int)info.lds_per_block);
         for (int m : {kMfmaF32, kMfmaBf16x3, kMfmaF16x2})
             for (int L : {256, 4096})
                 for (int nb : {2, 4})
@@ -2469,7 +2470,8 @@ static hipError_t launch_all(Plan* p, void* work, unsigned* counters, const void
         const float* frag = ln.frag;
         void* args[] = {&d, &frag};
         const void* fn = ln.mfma ? kernel_symbol_mfma(ln.mfma, ln.d.L, ln.mfma_nb)
-                         : ln.fixed ? kernel_symbol_fixed(p->spec.prec_bytes, ln.d.L, ln.maxt, ln.split)
+                         : ln.fixed ? kernel_symbol_fixed(p->spec.prec_bytes, ln.d.L, ln.maxt, ln.split,
+                                                          (d.flags & kNtStore) != 0)
                                     : kernel_symbol(pass_kind(ln), p->spec.prec_bytes, ln.rad,
                                                     (d.flags & kNtStore) != 0, ln.maxt);
         hipError_t e = hipLaunchKernel(fn, dim3(ln.grid), dim3(ln.block), args,
