@@ -705,6 +705,7 @@ static bool build_pass(Plan* plan, TableBuilder& tb, const PassReq& q, std::stri
     for (auto& a : q.lines) nl_total *= a.n;
     // threads per line, and the table and layout that go with the kernel
     int TL;
+    bool few = false;  // few lines for column tiles
     if (plan_match) {
         TL = q.L / 16;
         ln.E = 16;
@@ -712,10 +713,15 @@ static bool build_pass(Plan* plan, TableBuilder& tb, const PassReq& q, std::stri
         d.LP = (lds_pad(need - 1) + 1) | 1;
     } else {
         // column tiles: at most 64 threads per line (32 in complex128) while that
-        // leaves 20 elements per thread, see the tile's limit below
+        // leaves 20 elements per thread, see the tile's limit below -- but not
+        // where the lines are too few for one such tile's threads on every CU
+        // (complex64, 64 or 128 threads against none of these limits: 8 lines of
+        // 2800 12.7 -> 9.4 us, 514 of 1125 11.2 -> 9.5, 300 of 2800 15.0 -> 13.1)
         const bool cols = q.want_in_col || q.want_out_col;
         int most = cols ? 256 / prec : tmax;
         while (most < tmax && q.L > 20 * most) most *= 2;
+        few = cols && nl_total * most < (int64_t)dev.cus * (2048 / prec);
+        if (few) most = tmax;
         TL = line_threads(radix, q.L, cols ? 4 : 64 / esize, most,
                           r2c ? (int)radix.size() - 1 : c2r ? 0 : -1, nl_total, prec);
         if (tuned_e == 8 || tuned_e == 16) TL = std::min(next_pow2((q.L + tuned_e - 1) / tuned_e), tmax);
@@ -772,25 +778,52 @@ static bool build_pass(Plan* plan, TableBuilder& tb, const PassReq& q, std::stri
         d.tl_shift = 4;
     } else if (in_col || out_col) {
         const int cmax = plan->spec.tune.col_c ? plan->spec.tune.col_c : env_int("FFTZ_COL_C", prec == 8 ? 16 : 32);
-        // complex128 tiles of the fixed kernels take the whole LDS from 1024
-        // points on: columns of 8 lines 35 us, of 4 lines 40 us (64 MiB each way)
-        const bool whole = plan_match && prec == 8 && q.L >= 1024;
-        const size_t budget = std::min(lds_cap, (size_t)env_int("FFTZ_COL_LDS", whole ? 160 * 1024 : 96 * 1024));
+        const size_t budget = std::min(lds_cap, (size_t)env_int("FFTZ_COL_LDS", 96 * 1024));
         // Generic kernels: two workgroups per CU at their register counts, i.e.
         // 512 threads (256 in complex128), so that one loads while the other
         // computes: 1080-point columns of 961 x 13 images, 8 lines of 128
         // threads 78 us, of 64 threads 63 us; complex128 600-point columns, 8
         // lines of 64 threads 48 us, of 32 threads 38 us.
-        const int tcap = plan_match ? tmax : std::min(tmax, 2048 / prec);
+        // Not where the lines are few, nor where it would leave one line, read
+        // at element stride (350 complex128 columns of 2800 33.6 -> 17.6 us), nor
+        // two complex128 lines where the LDS holds one tile of four per CU and
+        // fours leave few lines idle (1000 columns of 1300 24.7 -> 17.7 us, but 135
+        // images of 10 columns of 1372 21.6 -> 28.1; complex64 loses: 984 columns
+        // of 2800 25.8 -> 32.4).
+        const int tcap = plan_match || few ? tmax : std::min(tmax, 2048 / prec);
         // a row of n0 lines that C does not divide is tiled raggedly (the
         // last tile of each row partly idle) rather than falling back to
         // element-strided row tiles
-        while (C * 2 <= cmax && (size_t)(C * 2) * line_bytes <= budget && C * 2 <= n0 && C * 2 * TL <= tcap)
+        const bool four = prec == 8 && 8 * line_bytes > lds_cap && (n0 + 3) / 4 * 4 <= n0 + n0 / 16;
+        while (C * 2 <= cmax && (size_t)(C * 2) * line_bytes <= budget && C * 2 <= n0 &&
+               C * 2 * TL <= (C == 1 || (C == 2 && four) ? tmax : tcap))
             C *= 2;
+        // complex128 tiles of the fixed kernels take the whole LDS from 1024
+        // points on: columns of 8 lines 35 us, of 4 lines 40 us (64 MiB each
+        // way).  That is one tile per CU instead of two.  On rows that start on
+        // cache lines it wins at any count (64 columns of 2048 points x 4: 10.9
+        // us, 14.2 without); on others where it adds neither a round of tiles (20
+        // images of 100 columns of 1024: 24 us, 15 without) nor idle lines (146 of 41:
+        // 55 us, 45) and the narrower ones are more than the CUs (335 columns of
+        // 2048: 13.6 us, 11.4).  4096 points have no narrower column tile.
+        if (plan_match && prec == 8 && q.L >= 1024 && C * 2 <= cmax && (size_t)(C * 2) * line_bytes <= lds_cap &&
+            C * 2 <= n0 && C * 2 * TL <= tmax) {
+            const bool aligned = (!in_col || q.ies % 8 == 0) && (!out_col || q.oes % 8 == 0) && n0 % (C * 2) == 0;
+            const int64_t rows = nl_total / n0, narrow = rows * ((n0 + C - 1) / C), wide = rows * ((n0 + C * 2 - 1) / (C * 2));
+            const int64_t cus = dev.cus;
+            if (C == 1 || aligned || (narrow > cus && wide * 2 <= narrow + narrow / 32 &&
+                                     (wide + cus - 1) / cus <= (narrow + 2 * cus - 1) / (2 * cus)))
+                C *= 2;
+        }
         // fewer than two tiles per CU: narrower ones, down to 16 lines (128- or
-        // 256-byte segments); fewer than one for two CUs: down to four lines
-        while (!plan->spec.tune.col_c &&
-               ((C > 16 && nl_total / C < 2 * dev.cus) || (C > 4 && nl_total / C < dev.cus / 2)))
+        // 256-byte segments); fewer than one for two CUs: down to four lines; long
+        // lines, fewer than one for four: two (complex64: 40 lines of 2187 12.0 ->
+        // 9.6 us, of 2000 10.9 -> 9.2; 130 complex128 lines of 144 5.6 -> 6.1).
+        // Fixed kernels keep a whole wavefront (48 complex128 lines of 64 5.1 us as
+        // 16 threads, 4.7 as 64).
+        while (!plan->spec.tune.col_c && !(plan_match && C * TL <= 64) &&
+               ((C > 16 && nl_total / C < 2 * dev.cus) || (C > 4 && nl_total / C < dev.cus / 2) ||
+                (C > 2 && q.L >= 1024 && nl_total / C < dev.cus / 4)))
             C /= 2;
         if (C < 2) { in_col = false; out_col = false; C = 1; }
     }
