@@ -315,9 +315,17 @@ __device__ __forceinline__ void store_pair(R* d, int64_t es, cplx<R> v)
     }
 }
 
-// Operands of butterfly j of stage 0, as the transform takes them (conjugated
-// for the backward direction).  src is the line's element 0; for the flags
-// that read reals it points at real elements.
+// Whether the backward direction's conjugation of the operands waits until the
+// stage's twiddles are asked for (conj_operands): conjugating waits for the
+// operands, and the twiddles' latency then comes on top.  3001 complex64 lines
+// of 1200 backward 14.3 us, 12.6 this way, as forward.  Complex128 has no
+// registers to spare for both: either direction loses 1-3%.
+template <typename R>
+constexpr bool kConjLate = sizeof(R) == 4;
+
+// Operands of butterfly j of stage 0, conjugated for the backward direction
+// unless kConjLate.  src is the line's element 0; for the flags that read reals
+// it points at real elements.
 template <typename R, int RAD, bool REAL>
 __device__ __forceinline__ void load_butterfly(const PassDesc& p, const cplx<R>* src, int j, int64_t gbase,
                                                cplx<R> (&v)[RAD])
@@ -371,7 +379,18 @@ __device__ __forceinline__ void load_butterfly(const PassDesc& p, const cplx<R>*
 #pragma unroll
         for (int i = 0; i < RAD; i++) v[i] = q[i * step];
     }
-    if (p.flags & kConjIn) {
+    if (!kConjLate<R> && (p.flags & kConjIn)) {
+#pragma unroll
+        for (int i = 0; i < RAD; i++) v[i].y = -v[i].y;
+    }
+}
+
+// The conjugation that load_butterfly left out (not of kChirpIn's products, nor
+// of reals).
+template <typename R, int RAD>
+__device__ __forceinline__ void conj_operands(const PassDesc& p, cplx<R> (&v)[RAD])
+{
+    if (kConjLate<R> && (p.flags & (kConjIn | kRealIn | kRealPromote | kChirpIn)) == kConjIn) {
 #pragma unroll
         for (int i = 0; i < RAD; i++) v[i].y = -v[i].y;
     }
@@ -467,12 +486,14 @@ __device__ __forceinline__ void store_butterfly(const PassDesc& p, cplx<R> (&v)[
     for (int i = 0; i < RAD; i++) put<R, NT>(q + i * step, v[i]);
 }
 
-// Stage 0: load, DFT, twiddle, write digit 0 (lanes contiguous).
-template <typename R, int RAD>
+// Stage 0 on loaded operands: DFT, twiddle, write digit 0 (lanes contiguous).
+// CONJ: v comes from load_butterfly.
+template <typename R, int RAD, bool CONJ>
 __device__ __forceinline__ void first_to_lds(const PassDesc& p, cplx<R>* line, int j, cplx<R> (&v)[RAD])
 {
     cplx<R> w[RAD - 1];
     load_twiddles<R, RAD>(stage_tw<R>(p, 0), (uint32_t)j, p.st[0].nbl, w);
+    if constexpr (CONJ) conj_operands<R, RAD>(p, v);
     Dft<RAD, R>::run(v);
     apply_twiddles<R, RAD>(v, w);
     const int step = p.st[0].lst;
@@ -488,7 +509,7 @@ __device__ __forceinline__ void first_stage(const PassDesc& p, cplx<R>* line, in
     for (int j = t; j < nbl; j += p.TL) {
         cplx<R> v[RAD];
         load_butterfly<R, RAD, REAL>(p, src, j, gbase, v);
-        first_to_lds<R, RAD>(p, line, j, v);
+        first_to_lds<R, RAD, true>(p, line, j, v);
     }
 }
 
@@ -528,6 +549,7 @@ __device__ __forceinline__ void single_stage(const PassDesc& p, const cplx<R>* s
 {
     cplx<R> v[RAD];
     load_butterfly<R, RAD, REAL>(p, src, 0, gin, v);
+    conj_operands<R, RAD>(p, v);
     Dft<RAD, R>::run(v);
     store_butterfly<R, RAD, REAL, NT>(p, v, 0, 1, dst, l0, gout);
 }
@@ -690,9 +712,9 @@ __device__ __forceinline__ void c2r_first_stage(const PassDesc& p, cplx<R>* line
             store_butterfly<R, RAD, true, false>(p, v, 0, 1, dst, 0, 0);
             return;
         }
-        first_to_lds<R, RAD>(p, line, j, v);
+        first_to_lds<R, RAD, false>(p, line, j, v);
         __builtin_amdgcn_sched_barrier(0);
-        if (!z || even) first_to_lds<R, RAD>(p, line, z ? nbl >> 1 : nbl - j, u);
+        if (!z || even) first_to_lds<R, RAD, false>(p, line, z ? nbl >> 1 : nbl - j, u);
     }
 }
 
@@ -926,7 +948,7 @@ __device__ __forceinline__ void bs_first(const PassDesc& p, cplx<R>* line, int t
                 }
             }
         }
-        first_to_lds<R, RAD>(p, line, j, v);
+        first_to_lds<R, RAD, false>(p, line, j, v);
     }
 }
 
