@@ -297,10 +297,13 @@ template <typename R, int MAXT, bool NT>
 static const void* fixed_sym(int L, bool split)
 {
     if (split) {
-        if constexpr (sizeof(R) == 4)
-            return L == 512 ? (const void*)&k_fixed_pass<R, 512, MAXT, true, NT> : nullptr;
+        // column tiles of 16 lines, the only ones that the planner gives it to
+        if constexpr (sizeof(R) == 4 && MAXT == 512)
+            return L == 512 ? (const void*)&k_fixed_pass<R, 512, 512, true, NT> : nullptr;
+        else if constexpr (sizeof(R) == 8 && MAXT == 256)
+            return L == 256 ? (const void*)&k_fixed_pass<R, 256, 256, true, NT> : nullptr;
         else
-            return L == 256 ? (const void*)&k_fixed_pass<R, 256, MAXT, true, NT> : nullptr;
+            return nullptr;
     }
     switch (L) {
         case 64: return MAXT == 256 ? (const void*)&k_fixed_pass<R, 64, 256, false, NT> : nullptr;

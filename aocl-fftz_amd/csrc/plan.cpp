@@ -901,10 +901,26 @@ static bool build_pass(Plan* plan, TableBuilder& tb, const PassReq& q, std::stri
     }
     ln.grid = (uint32_t)tiles;
     ln.lds_bytes = (uint32_t)((size_t)C * line_bytes);
-    // Exchange in halves only where more tiles than the two per CU that the
-    // full exchange holds are waiting: 28 x 65536 complex128 (448 tiles a pass)
-    // 27.9 us with it, 26.9 us without.
-    ln.split = ln.fixed && (in_col || out_col) && q.L == (prec == 4 ? 512 : 256) && tiles > 2 * dev.cus;
+    // Column exchanges in halves, where the LDS rather than the registers limits
+    // the workgroups of a CU and more tiles wait than the two that the whole
+    // exchange holds.  By what it measured (whole -> halves):
+    //   * complex128, 256 points: 64 MiB 24.2 -> 22.5 us, ragged 32 MiB 16.2 ->
+    //     14.1, 128 MiB 43.5 -> 40.0; 2^24 points in three passes 277 -> 271.  Not
+    //     beyond the Infinity Cache, where more lines in flight than it holds
+    //     cost: aligned rows from 512 MiB on 192 -> 204, others from 256 MiB 107 -> 120.
+    //   * complex64, 512 points, the reverse: 64 MiB 28.4 -> 30.5, 256 MiB 119.4
+    //     -> 116.8, 512 x 512 x 512 real in all 710 -> 694; short rows always lose
+    //     (64 lines, 256 MiB 114 -> 120).
+    //   * complex64, 256 and 1024 points: 64 MiB 23.3 -> 23.4 and 33.1 -> 35.5 us,
+    //     no kernel; complex128, 512 points would gain from 64 to 128 MiB (52.9 -> 47.5).
+    if (ln.fixed && (in_col || out_col) && tiles > 2 * dev.cus) {
+        const int64_t mib = (nl * q.L * esize) >> 20;
+        const bool aligned = n0 % C == 0 && (!in_col || (q.ies * esize) % 128 == 0) && (!out_col || (q.oes * esize) % 128 == 0);
+        if (prec == 8)
+            ln.split = q.L == 256 && ln.maxt == 256 && mib <= (aligned ? 256 : 128);
+        else
+            ln.split = q.L == 512 && ln.maxt == 512 && mib >= 256 && n0 > 4 * C;
+    }
     if (use_mfma) ln.lds_bytes += 64;  // per-wavefront maxima of the fp16 line scale
     // XCD-contiguous tile order: measured to help passes that read rows and
     // store columns (the four-step's transposing last pass) and to cost ~5%
