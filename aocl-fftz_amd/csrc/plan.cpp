@@ -936,12 +936,32 @@ static bool build_pass(Plan* plan, TableBuilder& tb, const PassReq& q, std::stri
     // Lines of 4 KiB and more count as whole (one partial line in 32); one store
     // has to cover 128 bytes of a row (64-point complex64 lines, 32 bytes: 13 -> 19
     // us), 256 of a column tile (128: 512^3 R2C's last pass 231 -> 234 us) on
-    // data beyond half of the Infinity Cache, which a reader finds there no more.
+    // data beyond half of the Infinity Cache.
+    // The next call may be another plan on this output, which it then finds in
+    // the Infinity Cache less often.  Time with / without for rows of 256 to 6000
+    // points: one plan alone; with a second plan reading its output; with that
+    // one in place.
+    //   output MiB                8      24      32      64      128     160     256
+    //   fixed kernels alone     .97-1.0 .72-.80 .76-.84 .91-.94 .95-.97 .81-.90 .79-.87
+    //     pair                  .95     .87-.96 .88-1.03 1.0-1.04 .95-.99 .84-.89 .94-.97
+    //     pair, in place        1.0     .94-1.0 .95-1.07 1.0-1.02 1.0-1.04 1.0-1.07 1.0-1.06
+    //   complex64 alone         .96-.99 .82-.92 .85-.93 .94-.97 .96-1.0 .70-.81 .69-.81
+    //     pair                  .94-.98 .95-1.08 .97-1.12 1.0-1.13 .93-.98 .83-.90 .94-1.0
+    //     pair, in place        .98-1.0 1.0-1.06 1.0-1.09 1.0-1.11 1.04-1.14 1.04-1.18 .96-1.0
+    //   complex128 alone        .92-.98 .82-.97 .83-.93 .91-.95 .91-.97 .79-.89 .75-.87
+    //     pair                  .93-.97 .88-.98 .94-1.03 .93-1.01 .91-.98 .84-.92 .89-.97
+    //     pair, in place        .96-1.0 .94-1.0 .97-1.0 .95-1.02 .94-1.04 .94-1.06 .91-1.0
+    // (generic kernels; Bluestein lines of either precision are as complex64.)
+    // So complex64 generic and Bluestein rows keep to plain stores between 32
+    // and 160 MiB, where a reader loses more than the plan gains.
     if (!(q.flags & kRealFlags) && q.out_role == Role::Out) {
         bool aligned = true;
         for (int k = out_col ? 1 : 0; k < 3; k++)
             if (ax[k].n > 1 && (ax[k].os * (int64_t)esize) % 128 != 0) aligned = false;
-        const bool rows = !out_col && q.oes == 1 && TL * esize >= 128 && (aligned || (int64_t)d.nvalid_out * esize >= 4096);
+        const int64_t mib = (nl * d.nvalid_out * esize) >> 20;
+        const bool reread = !plan_match && (prec == 4 || q.kind == KernelKind::Bluestein) && mib >= 32 && mib < 160;
+        const bool rows = !out_col && q.oes == 1 && TL * esize >= 128 && !reread &&
+                          (aligned || (int64_t)d.nvalid_out * esize >= 4096);
         const bool cols = out_col && aligned && (q.oes * esize) % 128 == 0 && C * esize >= 256 && n0 % C == 0 &&
                           nl * q.L * esize >= ((int64_t)128 << 20);
         if (rows || cols) d.flags |= kNtStore;

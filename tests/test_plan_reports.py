@@ -53,3 +53,12 @@ def test_stage_strides_and_batch_values_per_thread():
     for c in pj["classes"]:
         most = max([-(-pj["sizes"][t[0]]["L"] // pj["sizes"][t[0]]["TL"]) for t in c["tiles"]], default=0)
         assert c["E"] == most
+
+
+@pytest.mark.parametrize("n,batch,prec,nt", [
+    (64, 4096, "f", 0), (1024, 4096, "f", 1), (1024, 8192, "f", 1), (100, 17, "f", 0), (1200, 3001, "f", 1),
+    (1200, 3500, "f", 0), (1200, 17000, "f", 0), (1200, 18000, "f", 1), (1200, 4096, "d", 1), (1009, 1500, "d", 1),
+    (1009, 4000, "d", 0), (1009, 11000, "d", 1)])
+def test_stores_past_the_l2(n, batch, prec, nt):
+    # rows of whole cache lines; not where a reader of the output loses more than the plan gains
+    assert only([(n, 1, 1)], [(batch, n, n)], prec)["nt"] == nt
