@@ -41,9 +41,10 @@ constexpr bool rad_in_pairs(int set, int r) { return r <= (set == kRadTo8 ? 6 : 
 const void* kernel_symbol(KernelKind kind, int prec_bytes, int rad, bool nt, int maxt);
 
 // Uneven-batch persistent kernel (k_batch) of a tile class (0 small: 256
-// threads, 1 medium: 512, 2 large: 1024 in complex64, 512 in complex128) and
-// the counter reset kernel launched before it.
-const void* kernel_symbol_batch(int prec_bytes, int cls);
+// threads, 1 medium: 512, 2 large: 1024 in complex64, 512 in complex128), and the
+// counter reset kernel launched before it.  nt: results bypass the L2's
+// write-back (those of the medium and large class always do).
+const void* kernel_symbol_batch(int prec_bytes, int cls, bool nt);
 const void* kernel_symbol_reset();
 
 // Instantiation units behind kernel_symbol / kernel_symbol_batch (one
@@ -55,10 +56,10 @@ const void* kernel_symbol_pass_f64_pow2(KernelKind kind, bool nt, int maxt);
 const void* kernel_symbol_pass_f32_light(KernelKind kind, bool nt, int maxt);
 const void* kernel_symbol_pass_f64_light(KernelKind kind, bool nt, int maxt);
 const void* kernel_symbol_pass_f64_to8(KernelKind kind, bool nt, int maxt);
-const void* kernel_symbol_batch_f32_small();
+const void* kernel_symbol_batch_f32_small(bool nt);
 const void* kernel_symbol_batch_f32_medium();
 const void* kernel_symbol_batch_f32_large();
-const void* kernel_symbol_batch_f64_small();
+const void* kernel_symbol_batch_f64_small(bool nt);
 const void* kernel_symbol_batch_f64_medium();
 const void* kernel_symbol_batch_f64_large();
 

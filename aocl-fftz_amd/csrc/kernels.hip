@@ -33,9 +33,9 @@ const void* kernel_symbol(KernelKind kind, int prec_bytes, int rad, bool nt, int
     }
 }
 
-const void* kernel_symbol_batch(int prec_bytes, int cls)
+const void* kernel_symbol_batch(int prec_bytes, int cls, bool nt)
 {
-    if (cls == 0) return prec_bytes == 4 ? kernel_symbol_batch_f32_small() : kernel_symbol_batch_f64_small();
+    if (cls == 0) return prec_bytes == 4 ? kernel_symbol_batch_f32_small(nt) : kernel_symbol_batch_f64_small(nt);
     if (cls == 1) return prec_bytes == 4 ? kernel_symbol_batch_f32_medium() : kernel_symbol_batch_f64_medium();
     return prec_bytes == 4 ? kernel_symbol_batch_f32_large() : kernel_symbol_batch_f64_large();
 }

@@ -4,6 +4,6 @@
 
 namespace fftz {
 
-const void* kernel_symbol_batch_f32_large() { return (const void*)&k_batch<float, 1024>; }
+const void* kernel_symbol_batch_f32_large() { return (const void*)&k_batch<float, 1024, true>; }
 
 }  // namespace fftz

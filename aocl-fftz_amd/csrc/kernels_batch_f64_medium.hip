@@ -4,6 +4,6 @@
 
 namespace fftz {
 
-const void* kernel_symbol_batch_f64_medium() { return (const void*)&k_batch<double, 512>; }
+const void* kernel_symbol_batch_f64_medium() { return (const void*)&k_batch<double, 512, true>; }
 
 }  // namespace fftz

@@ -1080,7 +1080,7 @@ __global__ void __launch_bounds__(MAXT) k_bluestein(const PassDesc p_arg)
 // tile does not depend on the workgroup that runs it, so results are bitwise
 // identical run to run.
 // ---------------------------------------------------------------------------
-template <typename R, int MAXT>
+template <typename R, int MAXT, bool NT>
 __global__ void __launch_bounds__(MAXT) k_batch(const BatchArgs a)
 {
     // dynamic LDS: [tile index | tile data].  The tile index is made uniform
@@ -1110,9 +1110,9 @@ __global__ void __launch_bounds__(MAXT) k_batch(const BatchArgs a)
         // a queue entry covers one or more rounds of C lines
         for (int64_t lb = 0; lb < io.nlines; lb += C) {
             if (blue)
-                bluestein_body<R, kRadAll, true>(p, io, lds, lb, tid);
+                bluestein_body<R, kRadAll, NT>(p, io, lds, lb, tid);
             else
-                pass_body<R, kRadAll, kRealNone, true>(p, io, lds, lb, tid);
+                pass_body<R, kRadAll, kRealNone, NT>(p, io, lds, lb, tid);
             __syncthreads();
         }
         if (tid == 0) s_tile = nxt;

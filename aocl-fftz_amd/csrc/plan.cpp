@@ -1905,25 +1905,43 @@ Plan* batch_plan_create(const std::vector<BatchItem>& items, int prec, int dir, 
     // cost (queue atomic, descriptor loads, barriers) is amortised -- but its
     // rounds run one after the other, and a workgroup's last entry is the
     // launch's tail: an eighth of what a resident workgroup gets in all, between
-    // 16 KiB and 32 / 128 / 256 KiB.  Against 128 / 128 / 256 KiB throughout:
-    // 2000 items 2.18 -> 2.05 ms, 400 items 0.65 -> 0.48 ms, 100 items 0.43 ->
-    // 0.14 ms.
+    // 16 KiB and 128 / 256 KiB in the medium / large class.  Against 128 / 256 KiB
+    // throughout: 2000 items 2.18 -> 2.05 ms, 400 items 0.65 -> 0.48 ms, 100 items
+    // 0.43 -> 0.14 ms.  Entries of the small class are short, so that their number
+    // counts: 4096 points, or the largest half of that which gives seven for
+    // every four resident workgroups, down to 16 KiB (2000 items of 64 points each,
+    // complex64: 32 KiB 61 us, 16 KiB 70 us; 500 items of 16 to 256 points the
+    // reverse, 48 and 41 us; 128 KiB in a list with longer items 168 us, 135).
     const int64_t entry_env = env_int("FFTZ_BATCH_ENTRY_BYTES", 0);
-    const int64_t entry_most[3] = {32 * 1024, 128 * 1024, 256 * 1024}, resident[3] = {4, 2, 1};
-    int64_t entry_cls[3] = {0, 0, 0};
-    for (const BatchItem& it : items)
-        if (it.batch) entry_cls[sizes[(size_t)size_index[it.n]].cls] += it.n * it.batch * esize;
-    for (int c = 0; c < 3; c++)
-        entry_cls[c] = std::max<int64_t>(16 * 1024, std::min(entry_most[c], entry_cls[c] / (8 * dev.cus * resident[c])));
+    const int64_t resident[3] = {4, 2, 1};
+    auto entry_rounds = [&](const SizeInfo& si, int64_t bytes) {
+        return std::max<int64_t>(1, std::min<int64_t>(16, bytes / std::max<int64_t>(1, (int64_t)si.C * si.n * esize)));
+    };
+    int64_t entry_cls[3] = {4096 * esize, 128 * 1024, 256 * 1024}, bytes_cls[3] = {0, 0, 0}, short_cls[3] = {0, 0, 0};
+    for (const BatchItem& it : items) {
+        if (!it.batch) continue;
+        const int c = sizes[(size_t)size_index[it.n]].cls;
+        bytes_cls[c] += it.n * it.batch * esize;
+        if (it.n * esize < 2048) short_cls[c] += it.n * it.batch * esize;
+    }
+    for (int c = 1; c < 3; c++)
+        entry_cls[c] = std::max<int64_t>(16 * 1024, std::min(entry_cls[c], bytes_cls[c] / (8 * dev.cus * resident[c])));
+    for (; entry_cls[0] > 16 * 1024; entry_cls[0] /= 2) {
+        int64_t n = 0;
+        for (const BatchItem& it : items) {
+            const SizeInfo& si = sizes[(size_t)size_index[it.n]];
+            const int64_t step = (int64_t)si.C * entry_rounds(si, entry_cls[0]);
+            if (si.cls == 0) n += (it.batch + step - 1) / step;
+        }
+        if (4 * n >= 7 * dev.cus * resident[0]) break;
+    }
     std::vector<std::vector<std::pair<double, BatchTile>>> tiles(3);
     for (const BatchItem& it : items) {
         if (it.batch == 0) continue;
         const SizeInfo& si = sizes[(size_t)size_index[it.n]];
         const int64_t dist = it.dist ? it.dist : it.n;
         const int64_t entry_bytes = entry_env > 0 ? entry_env : entry_cls[si.cls];
-        const int64_t per_round = (int64_t)si.C * si.n * esize;
-        const int64_t rounds = std::max<int64_t>(1, std::min<int64_t>(16, entry_bytes / std::max<int64_t>(1, per_round)));
-        const int64_t step = (int64_t)si.C * rounds;
+        const int64_t step = (int64_t)si.C * entry_rounds(si, entry_bytes);
         for (int64_t l0 = 0; l0 < it.batch; l0 += step) {
             BatchTile bt{};
             bt.desc = (uint32_t)size_index[it.n];
@@ -1949,6 +1967,11 @@ Plan* batch_plan_create(const std::vector<BatchItem>& items, int prec, int dir, 
         std::stable_sort(tl.begin(), tl.end(), [](const auto& a, const auto& b) { return a.first > b.first; });
         BatchClass bc;
         bc.maxt = c == 0 ? 256 : (c == 1 ? 512 : big_threads);
+        // Short lines anywhere in the buffers are not whole cache lines: plain
+        // stores where most of the small class is below 2 KiB a line (3508 items of
+        // 16 to 64 complex128 points 102 -> 96 us, then read in order 212 -> 192; 4000
+        // of 16 to 256 points the reverse, 235 and 272).
+        bc.nt = c > 0 || 2 * short_cls[0] <= bytes_cls[0];
         bc.ntiles = (int)tl.size();
         size_t lds = 0;
         for (const SizeInfo& si : sizes)
@@ -2002,7 +2025,7 @@ Plan* batch_plan_create(const std::vector<BatchItem>& items, int prec, int dir, 
         return nullptr;
     }
     for (size_t c = 0; c < plan->bclasses.size(); c++)
-        (void)hipFuncSetAttribute(kernel_symbol_batch(prec, (int)c),
+        (void)hipFuncSetAttribute(kernel_symbol_batch(prec, (int)c, plan->bclasses[c].nt),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)dev.lds_per_block);
     plan->host_tables.clear();
     plan->host_tables.shrink_to_fit();
@@ -2337,7 +2360,7 @@ static std::string batch_json(const Plan* p)
             const PassDesc& d = hd[q[i].desc];
             E = std::max(E, (d.L + d.TL - 1) / d.TL);
         }
-        os << (c ? "," : "") << "{\"E\":" << E << ",\"maxt\":" << bc.maxt << ",\"lds\":" << bc.lds_bytes
+        os << (c ? "," : "") << "{\"E\":" << E << ",\"nt\":" << (bc.nt ? 1 : 0) << ",\"maxt\":" << bc.maxt << ",\"lds\":" << bc.lds_bytes
            << ",\"grid\":" << bc.grid << ",\"tiles\":[";
         for (int i = 0; q && i < bc.ntiles; i++)
             os << (i ? "," : "") << "[" << q[i].desc << "," << q[i].nlines << "," << q[i].bluestein << ","
@@ -2500,7 +2523,7 @@ static hipError_t launch_batch(Plan* p, unsigned* counters, const void* in, void
             a.in = in;
             a.out = out;
             void* args[] = {&a};
-            e = hipLaunchKernel(kernel_symbol_batch(p->spec.prec_bytes, (int)c), dim3(bc.grid),
+            e = hipLaunchKernel(kernel_symbol_batch(p->spec.prec_bytes, (int)c, bc.nt), dim3(bc.grid),
                                 dim3(bc.maxt), args, bc.lds_bytes, stream);
             if (e != hipSuccess) return e;
         }

@@ -68,6 +68,7 @@ struct BatchItem {
 // A persistent-kernel class of the uneven batch (small or large tiles).
 struct BatchClass {
     int maxt = 256;
+    bool nt = true;  // results bypass the L2's write-back
     uint32_t lds_bytes = 0;
     uint32_t grid = 0;
     int ntiles = 0;
