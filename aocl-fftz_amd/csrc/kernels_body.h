@@ -180,24 +180,37 @@ __device__ __forceinline__ void apply_twiddles(cplx<R> (&v)[RAD], const cplx<R> 
     for (int i = 1; i < RAD; i++) v[i] = cmul(v[i], w[i - 1]);
 }
 
+// Whether a stage asks for its twiddles only after its DFT.  Radix 11, 13 and 16
+// in complex128 hold 44 to 64 registers of operands and nearly as many of
+// twiddles, which decided the registers of every plain pass of kRadAll (199, two
+// wavefronts per SIMD, or 66 spilled at three; now 167) and made kRadLight spill
+// (168 and 4; now 161).  2666 lines of 1573 (13 x 11 x 11) 34.6 -> 30.8 us, the
+// 100 x 120 x 144 grid (16 x 9) there and back 85.5 -> 80.9, 104 chirp-z
+// transforms of 20011 (passes of 220 and 182) 177 -> 166.
+template <typename R, int RADSET, int RAD>
+constexpr bool kLateTw = sizeof(R) == 8 && (RADSET == kRadAll || RADSET == kRadLight) &&
+                         (RAD == 11 || RAD == 13 || RAD == 16);
+
 // Middle stage in place: DFT then twiddle (decimation in frequency), or, for
 // the second transform of a Bluestein pass, twiddle then DFT with the same
 // table (decimation in time: digits return from output to input order).
 // Addresses and twiddles of the first butterfly are fetched before the
 // barrier that makes the previous stage's results visible: their latency
 // (tables of long lines live in the L2 or beyond) overlaps the barrier.
-template <typename R, int RAD, bool DIT>
+// LATE: twiddles after the DFT (kLateTw).
+template <typename R, int RAD, bool DIT, bool LATE>
 __device__ __forceinline__ void mid_stage(const PassDesc& p, cplx<R>* line, int t, int s, bool live, bool wave_local)
 {
     const int nbl = live ? p.st[s].nbl : 0, step = p.st[s].lst;
     const cplx<R>* tw = stage_tw<R>(p, s);
+    static_assert(!(DIT && LATE));
     int j = t, base = 0;
+    uint32_t m = 0;
     cplx<R> w[RAD - 1];
     auto fetch = [&]() {
         if (j < nbl) {
-            uint32_t m;
             base = mid_base(p, s, j, m);
-            load_twiddles<R, RAD>(tw, m, step, w);
+            if constexpr (!LATE) load_twiddles<R, RAD>(tw, m, step, w);
         }
     };
     fetch();
@@ -210,6 +223,10 @@ __device__ __forceinline__ void mid_stage(const PassDesc& p, cplx<R>* line, int 
         for (int i = 0; i < RAD; i++) v[i] = q[i * step];
         if constexpr (DIT) apply_twiddles<R, RAD>(v, w);
         Dft<RAD, R>::run(v);
+        if constexpr (LATE) {
+            __builtin_amdgcn_sched_barrier(0);
+            load_twiddles<R, RAD>(tw, m, step, w);
+        }
         if constexpr (!DIT) apply_twiddles<R, RAD>(v, w);
 #pragma unroll
         for (int i = 0; i < RAD; i++) q[i * step] = v[i];
@@ -487,21 +504,25 @@ __device__ __forceinline__ void store_butterfly(const PassDesc& p, cplx<R> (&v)[
 }
 
 // Stage 0 on loaded operands: DFT, twiddle, write digit 0 (lanes contiguous).
-// CONJ: v comes from load_butterfly.
-template <typename R, int RAD, bool CONJ>
+// CONJ: v comes from load_butterfly.  LATE: twiddles after the DFT (kLateTw).
+template <typename R, int RAD, bool CONJ, bool LATE>
 __device__ __forceinline__ void first_to_lds(const PassDesc& p, cplx<R>* line, int j, cplx<R> (&v)[RAD])
 {
     cplx<R> w[RAD - 1];
-    load_twiddles<R, RAD>(stage_tw<R>(p, 0), (uint32_t)j, p.st[0].nbl, w);
+    if constexpr (!LATE) load_twiddles<R, RAD>(stage_tw<R>(p, 0), (uint32_t)j, p.st[0].nbl, w);
     if constexpr (CONJ) conj_operands<R, RAD>(p, v);
     Dft<RAD, R>::run(v);
+    if constexpr (LATE) {
+        __builtin_amdgcn_sched_barrier(0);
+        load_twiddles<R, RAD>(stage_tw<R>(p, 0), (uint32_t)j, p.st[0].nbl, w);
+    }
     apply_twiddles<R, RAD>(v, w);
     const int step = p.st[0].lst;
 #pragma unroll
     for (int i = 0; i < RAD; i++) line[j + i * step] = v[i];
 }
 
-template <typename R, int RAD, bool REAL>
+template <typename R, int RAD, bool REAL, bool LATE>
 __device__ __forceinline__ void first_stage(const PassDesc& p, cplx<R>* line, int t, const cplx<R>* src, int64_t gbase)
 {
     const int nbl = p.st[0].nbl;
@@ -509,7 +530,7 @@ __device__ __forceinline__ void first_stage(const PassDesc& p, cplx<R>* line, in
     for (int j = t; j < nbl; j += p.TL) {
         cplx<R> v[RAD];
         load_butterfly<R, RAD, REAL>(p, src, j, gbase, v);
-        first_to_lds<R, RAD, true>(p, line, j, v);
+        first_to_lds<R, RAD, true, LATE>(p, line, j, v);
     }
 }
 
@@ -712,9 +733,9 @@ __device__ __forceinline__ void c2r_first_stage(const PassDesc& p, cplx<R>* line
             store_butterfly<R, RAD, true, false>(p, v, 0, 1, dst, 0, 0);
             return;
         }
-        first_to_lds<R, RAD, false>(p, line, j, v);
+        first_to_lds<R, RAD, false, false>(p, line, j, v);
         __builtin_amdgcn_sched_barrier(0);
-        if (!z || even) first_to_lds<R, RAD, false>(p, line, z ? nbl >> 1 : nbl - j, u);
+        if (!z || even) first_to_lds<R, RAD, false, false>(p, line, z ? nbl >> 1 : nbl - j, u);
     }
 }
 
@@ -775,11 +796,11 @@ __device__ __forceinline__ void identity_line(const PassDesc& p, const cplx<R>* 
 }
 
 // Every middle stage begins with the barrier that ends the stage before it.
-template <typename R, int RADSET, bool DIT>
+template <typename R, int RADSET, bool DIT, bool LATE>
 __device__ __forceinline__ void mid_stage_any(const PassDesc& p, cplx<R>* line, int t, int s, bool live,
                                               bool wave_local)
 {
-    FFTZ_RADIX_SWITCH(p.st[s].radix, RADSET, (mid_stage<R, RAD, DIT>(p, line, t, s, live, wave_local)))
+    FFTZ_RADIX_SWITCH(p.st[s].radix, RADSET, (mid_stage<R, RAD, DIT, LATE && kLateTw<R, RADSET, RAD>>(p, line, t, s, live, wave_local)))
 }
 
 // Forms of the generic pass kernel: complex on both sides; a real side, with
@@ -789,7 +810,8 @@ enum RealForm : int { kRealNone = 0, kRealPair = 1, kRealWide = 2 };
 // One tile: C lines, threads (c, t) per side's mapping -- row (a wavefront
 // walks along a line) or column (it walks the same element of adjacent lines).
 // REAL passes carry the real-packed and promoted forms and are row-mapped.
-template <typename R, int RADSET, int REALK, bool NT>
+// LATE: wide radices may ask for their twiddles after the DFT (kLateTw).
+template <typename R, int RADSET, int REALK, bool NT, bool LATE>
 __device__ __forceinline__ void pass_body(const PassDesc& p, const TileIo& io, cplx<R>* lds, int64_t l_base, int tid)
 {
     constexpr bool REAL = REALK != kRealNone;
@@ -849,11 +871,11 @@ __device__ __forceinline__ void pass_body(const PassDesc& p, const TileIo& io, c
             }
         }
         if (!packed) {
-            FFTZ_RADIX_SWITCH(p.st[0].radix, RADSET, (first_stage<R, RAD, REAL>(p, line, ti, src, gin)))
+            FFTZ_RADIX_SWITCH(p.st[0].radix, RADSET, (first_stage<R, RAD, REAL, LATE && kLateTw<R, RADSET, RAD>>(p, line, ti, src, gin)))
         }
     }
     for (int s = 1; s + 1 < S; s++)
-        mid_stage_any<R, RADSET, false>(p, lds + cr * p.LP, tr, s, cr < p.C, wave_local);
+        mid_stage_any<R, RADSET, false, LATE>(p, lds + cr * p.LP, tr, s, cr < p.C, wave_local);
     stage_sync(wave_local);
     if (in_col != out_col) {
         const SlotLine slo = slot_line(p, io, l_base, co);
@@ -878,14 +900,14 @@ __device__ __forceinline__ void pass_body(const PassDesc& p, const TileIo& io, c
 
 template <typename R, int RADSET, int REALK, bool NT, int MAXT>
 __global__ void __launch_bounds__(MAXT)
-    __attribute__((amdgpu_waves_per_eu(REALK == kRealNone ? (RADSET == kRadLight && sizeof(R) == 8 ? 3 : 1) : REALK == kRealWide ? 1 : sizeof(R) == 4 ? 4 : RADSET == kRadTo8 ? 3 : 2))) k_fft_pass(const PassDesc p_arg)
+    __attribute__((amdgpu_waves_per_eu(REALK == kRealNone ? (sizeof(R) == 8 && (RADSET == kRadLight || RADSET == kRadAll) ? 3 : 1) : REALK == kRealWide ? 1 : sizeof(R) == 4 ? 4 : RADSET == kRadTo8 ? 3 : 2))) k_fft_pass(const PassDesc p_arg)
 {
     (void)p_arg;
     const PassDesc& p = kernarg_desc();
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
     cplx<R>* lds = reinterpret_cast<cplx<R>*>(smem_raw);
     const int64_t l_base = (int64_t)tile_of_block(p) * p.C;
-    pass_body<R, RADSET, REALK, NT>(p, io_of(p), lds, l_base, threadIdx.x);
+    pass_body<R, RADSET, REALK, NT, REALK == kRealNone>(p, io_of(p), lds, l_base, threadIdx.x);
 }
 
 // ---------------------------------------------------------------------------
@@ -948,7 +970,7 @@ __device__ __forceinline__ void bs_first(const PassDesc& p, cplx<R>* line, int t
                 }
             }
         }
-        first_to_lds<R, RAD, false>(p, line, j, v);
+        first_to_lds<R, RAD, false, false>(p, line, j, v);
     }
 }
 
@@ -1055,9 +1077,9 @@ __device__ __forceinline__ void bluestein_body(const PassDesc& p, const TileIo& 
     if (live) {
         FFTZ_RADIX_SWITCH(p.st[0].radix, RADSET, (bs_first<R, RAD>(p, line, t, src)))
     }
-    for (int s = 1; s + 1 < S; s++) mid_stage_any<R, RADSET, false>(p, line, t, s, live, wave_local);
+    for (int s = 1; s + 1 < S; s++) mid_stage_any<R, RADSET, false, false>(p, line, t, s, live, wave_local);
     FFTZ_RADIX_SWITCH(p.st[S - 1].radix, RADSET, (bs_center<R, RAD>(p, line, t, live, wave_local)))
-    for (int s = S - 2; s >= 1; s--) mid_stage_any<R, RADSET, true>(p, line, t, s, live, wave_local);
+    for (int s = S - 2; s >= 1; s--) mid_stage_any<R, RADSET, true, false>(p, line, t, s, live, wave_local);
     FFTZ_RADIX_SWITCH(p.st[0].radix, RADSET, (bs_final<R, RAD, NT>(p, line, t, dst, live, wave_local)))
 }
 
@@ -1112,7 +1134,7 @@ __global__ void __launch_bounds__(MAXT) k_batch(const BatchArgs a)
             if (blue)
                 bluestein_body<R, kRadAll, NT>(p, io, lds, lb, tid);
             else
-                pass_body<R, kRadAll, kRealNone, NT>(p, io, lds, lb, tid);
+                pass_body<R, kRadAll, kRealNone, NT, false>(p, io, lds, lb, tid);
             __syncthreads();
         }
         if (tid == 0) s_tile = nxt;

@@ -700,9 +700,17 @@ static bool build_pass(Plan* plan, TableBuilder& tb, const PassReq& q, std::stri
     // fixed kernels come in 256- and 512-thread variants (512 for wide column
     // tiles of L >= 256)
     const int tbig = (prec == 4 ? 1024 : 512) / ((q.flags & kRealFlags) && q.kind == KernelKind::Pass ? 2 : 1);
-    const int tmax = plan_match ? (q.L >= 256 ? 512 : 256) : tbig;
+    int tmax = plan_match ? (q.L >= 256 ? 512 : 256) : tbig;
     int64_t nl_total = 1;
     for (auto& a : q.lines) nl_total *= a.n;
+    // A complex128 workgroup of 512 threads is the only one on a CU but for
+    // kRadTo8 (three wavefronts per SIMD or fewer): 256 threads for rows where the
+    // LDS holds two tiles and the lines are more than the CUs (261 lines of 4004
+    // 18.9 -> 14.5 us, 1024 of 4095 43.5 -> 35.9; 256 of 4095 the reverse, 13.2
+    // and 14.4).  Columns have their own limit below.
+    if (!plan_match && prec == 8 && ln.rad != kRadTo8 && nl_total > dev.cus && !q.want_in_col && !q.want_out_col &&
+        2 * (size_t)lds_pad(need) * esize <= dev.lds_per_block)
+        tmax = std::min(tmax, 256);
     // threads per line, and the table and layout that go with the kernel
     int TL;
     bool few = false;  // few lines for column tiles

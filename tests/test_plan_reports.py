@@ -62,3 +62,10 @@ def test_stage_strides_and_batch_values_per_thread():
 def test_stores_past_the_l2(n, batch, prec, nt):
     # rows of whole cache lines; not where a reader of the output loses more than the plan gains
     assert only([(n, 1, 1)], [(batch, n, n)], prec)["nt"] == nt
+
+
+@pytest.mark.parametrize("n,batch,TL", [(4004, 261, 256), (4004, 256, 512), (4095, 1024, 256), (8190, 512, 512),
+                                        (5005, 600, 512)])
+def test_threads_of_complex128_rows(n, batch, TL):
+    # 256 where the LDS holds two tiles and there are more lines than CUs
+    assert only([(n, 1, 1)], [(batch, n, n)], "d")["TL"] == TL
