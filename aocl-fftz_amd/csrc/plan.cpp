@@ -83,33 +83,60 @@ struct d2 {
     double x, y;
 };
 
+// exp(-i theta) from u = (cos, sin) of theta's distance to the even end of its octant.
+static d2 unfold(int64_t oct, d2 u)
+{
+    double ct, st;  // cos, sin of theta
+    switch (oct) {
+        case 0: ct = u.x; st = u.y; break;
+        case 1: ct = u.y; st = u.x; break;
+        case 2: ct = -u.y; st = u.x; break;
+        case 3: ct = -u.x; st = u.y; break;
+        case 4: ct = -u.x; st = -u.y; break;
+        case 5: ct = -u.y; st = -u.x; break;
+        case 6: ct = u.y; st = -u.x; break;
+        default: ct = u.x; st = -u.y; break;
+    }
+    return {ct, -st};
+}
+
 static d2 root_fwd(int64_t p, int64_t n)
 {
     p %= n;
     if (p < 0) p += n;
-    const __int128 p8 = (__int128)p * 8;
-    const int64_t oct = (int64_t)(p8 / n);         // octant 0..7
-    const int64_t rem = (int64_t)(p8 - (__int128)oct * n);  // angle = (pi/4)(oct + rem/n)
-    double c, s;
-    const double a = (M_PI / 4.0) * ((double)rem / (double)n);
-    const double b = (M_PI / 4.0) * ((double)(n - rem) / (double)n);
-    // base angle theta = (pi/4) * (oct + rem/n); use the complementary
-    // angle on odd octants so the argument stays <= pi/4
-    double ct, st;  // cos, sin of theta
-    switch (oct) {
-        case 0: ct = cos(a); st = sin(a); break;
-        case 1: ct = sin(b); st = cos(b); break;
-        case 2: ct = -sin(a); st = cos(a); break;
-        case 3: ct = -cos(b); st = sin(b); break;
-        case 4: ct = -cos(a); st = -sin(a); break;
-        case 5: ct = -sin(b); st = -cos(b); break;
-        case 6: ct = sin(a); st = -cos(a); break;
-        default: ct = cos(b); st = -sin(b); break;
-    }
-    c = ct;
-    s = st;
-    return {c, -s};
+    // theta = (pi/4)(oct + rem/n), octant 0..7; below 2^60 in 64 bits.  The folded
+    // angle counts from the octant's end in odd octants, so it stays <= pi/4.
+    const bool narrow = n < ((int64_t)1 << 60);
+    const int64_t oct = narrow ? 8 * p / n : (int64_t)((__int128)p * 8 / n);
+    const int64_t rem = narrow ? 8 * p - oct * n : (int64_t)((__int128)p * 8 - (__int128)oct * n);
+    const double a = (M_PI / 4.0) * ((double)(oct & 1 ? n - rem : rem) / (double)n);
+    return unfold(oct, {cos(a), sin(a)});
 }
+
+// The n-th roots, root_fwd's values bit for bit.  Where 4 divides n the folded
+// angles of all octants are those of the first, so only its n / 8 cosines and
+// sines are computed.
+class RootTable {
+    const int64_t n_;
+    std::vector<d2> u_;
+
+public:
+    explicit RootTable(int64_t n) : n_(n)
+    {
+        if (n % 4) return;
+        u_.resize((size_t)(n / 8 + 1));
+        for (int64_t p = 0; 8 * p <= n; p++) {
+            const double a = (M_PI / 4.0) * ((double)(8 * p) / (double)n);
+            u_[(size_t)p] = {cos(a), sin(a)};
+        }
+    }
+    d2 operator()(int64_t p) const  // 0 <= p < n
+    {
+        if (u_.empty()) return root_fwd(p, n_);
+        const int64_t oct = 8 * p / n_, q = n_ / 4;
+        return unfold(oct, u_[(size_t)(oct & 1 ? (oct + 1) / 2 * q - p : p - oct / 2 * q)]);
+    }
+};
 
 // ---------------------------------------------------------------------------
 // Host FP64 FFT (recursive mixed radix) used only at setup, for the Bluestein
@@ -172,31 +199,29 @@ static bool smooth13(int64_t n)
     return n == 1;
 }
 
+// n as exactly S radices, the largest possible one first at each step.
+static bool pick_radices(int n, int S, std::vector<int>& out)
+{
+    if (S == 0) return n == 1;
+    for (int r : kRadices) {
+        if (n % r) continue;
+        int64_t most = 1;  // S - 1 radices reach at most 16^(S - 1)
+        for (int s = 1; s < S; s++) most *= kRadices[0];
+        if (n / r > most) continue;
+        out.push_back(r);
+        if (pick_radices(n / r, S - 1, out)) return true;
+        out.pop_back();
+    }
+    return false;
+}
+
 // Fewest radix stages from kRadices (largest first on ties).
 static bool factor_radices(int L, std::vector<int>& out)
 {
     out.clear();
     if (L == 1) return true;
-    std::map<int, std::pair<int, int>> memo;
-    std::function<int(int)> solve = [&](int n) -> int {
-        if (n == 1) return 0;
-        auto it = memo.find(n);
-        if (it != memo.end()) return it->second.first;
-        int best = 1 << 30, br = 0;
-        for (int r : kRadices) {
-            if (n % r) continue;
-            int c = solve(n / r);
-            if (c + 1 < best) { best = c + 1; br = r; }
-        }
-        memo[n] = {best, br};
-        return best;
-    };
-    if (solve(L) >= (1 << 30)) return false;
-    for (int n = L; n > 1;) {
-        int r = memo[n].second;
-        out.push_back(r);
-        n /= r;
-    }
+    if (!smooth13(L)) return false;
+    for (int S = 1; !pick_radices(L, S, out); S++) {}
     std::sort(out.begin(), out.end(), std::greater<int>());
     // A radix-2 stage costs nearly as much LDS traffic and addressing as any
     // other: 16 16 16 2 becomes 16 8 8 8 (8192-point complex64 lines).  The
@@ -353,8 +378,9 @@ static int64_t stage_twiddles(TableBuilder& tb, int prec, const std::vector<int>
     for (size_t s = 0; s < radix.size(); s++) {
         const int R = radix[s];
         twoff[s] = (int)tw.size();
+        const RootTable root((int64_t)R * ls);
         for (int c = 0; c < ls; c++)
-            for (int i = 1; i < R; i++) tw.push_back(root_fwd((int64_t)i * c, (int64_t)R * ls));
+            for (int i = 1; i < R; i++) tw.push_back(root((int64_t)i * c));
         ls *= R;
     }
     if (tw.empty()) tw.push_back({1.0, 0.0});
@@ -436,14 +462,40 @@ static int64_t digit_layout(TableBuilder& tb, int prec, const std::vector<int>& 
         d.st[s].mdiv = make_smalldiv((uint32_t)A);
         d.st[s].rdiv = make_smalldiv((uint32_t)R);
         d.st[s].twoff = (int)tw.size();
-        if (s + 1 < S)
+        if (s + 1 < S) {
+            const RootTable root((int64_t)R * A);
             for (int k = 1; k < R; k++)
-                for (int m = 0; m < A; m++) tw.push_back(root_fwd((int64_t)k * m, (int64_t)R * A));
+                for (int m = 0; m < A; m++) tw.push_back(root((int64_t)k * m));
+        }
     }
     int LP = std::max(lp_min, L);
     if (S >= 2) {
         const int lanes = prec == 4 ? 16 : 8;  // lanes (and banks, in elements) per LDS cycle
         const int A0 = d.st[0].lst;
+        // position of lane l in stage s: dig0 (A0 + pad) + rest + line pitch
+        std::vector<int> dig0((size_t)(64 * S), -1), rest((size_t)(64 * S), 0);
+        const int per = std::min(TL, 64);
+        for (int s = 1; s < S; s++)
+            for (int l = 0; l < 64; l++) {
+                const int j = l % per, k = s * 64 + l;
+                if (j >= d.st[s].nbl) continue;
+                dig0[(size_t)k] = j % radix[0];
+                int rem = j / radix[0];
+                if (s + 1 < S) {
+                    const int o = rem / d.st[s].lst;
+                    rest[(size_t)k] = o * radix[(size_t)s] * d.st[s].lst + rem % d.st[s].lst;
+                    continue;
+                }
+                for (int i = 1; i + 2 < S; i++) {
+                    rest[(size_t)k] += (rem % radix[(size_t)i]) * d.st[i].lst;
+                    rem /= radix[(size_t)i];
+                }
+                if (S >= 3) {
+                    rest[(size_t)k] += rem * d.st[S - 2].lst;
+                } else {
+                    dig0[(size_t)k] = j;
+                }
+            }
         int best = 0;
         long best_cost = -1;
         for (int pad = 0; pad < 8; pad++) {
@@ -452,26 +504,13 @@ static int64_t digit_layout(TableBuilder& tb, int prec, const std::vector<int>& 
             const int pitch = std::max(lp_min, radix[0] * a0) | 1;
             long cost = 0;
             for (int s = 1; s < S; s++) {
-                int bank[16];
                 for (int l0 = 0; l0 < 64; l0 += lanes) {
-                    for (int b = 0; b < lanes; b++) bank[b] = 0;
-                    int worst = 0;
+                    int bank[16] = {}, worst = 0;
                     for (int l = l0; l < l0 + lanes; l++) {
-                        const int c = l / std::min(TL, 64), j = l % std::min(TL, 64);
-                        if (j >= d.st[s].nbl) continue;
-                        int pos = 0;
-                        if (s + 1 == S) {
-                            int rem = j;
-                            for (int i = 0; i + 2 < S; i++) {
-                                pos += (rem % radix[(size_t)i]) * (i ? d.st[i].lst : a0);
-                                rem /= radix[(size_t)i];
-                            }
-                            pos += rem * (S >= 3 ? d.st[S - 2].lst : a0);
-                        } else {
-                            const int q = j / radix[0], o = q / d.st[s].lst, m = q % d.st[s].lst;
-                            pos = (j % radix[0]) * a0 + o * radix[(size_t)s] * d.st[s].lst + m;
-                        }
-                        worst = std::max(worst, ++bank[(pos + c * pitch) % lanes]);
+                        const int k = s * 64 + l;
+                        if (dig0[(size_t)k] < 0) continue;
+                        const int pos = dig0[(size_t)k] * a0 + rest[(size_t)k] + l / per * pitch;
+                        worst = std::max(worst, ++bank[pos & (lanes - 1)]);
                     }
                     // a middle stage reads and writes, the last only reads
                     cost += (long)worst * radix[(size_t)s] * (s + 1 == S ? 1 : 2);
@@ -1129,6 +1168,9 @@ static bool device_fft_fp64(std::vector<d2>& v)
 static void bluestein_tables(TableBuilder& tb, int prec, int64_t n, int64_t M, int64_t* chirp_off, int64_t* spec_off,
                              bool dry_run)
 {
+    // in one allocation with what follows (growing by doubling, the arena of a
+    // long transform was copied and its pages touched twice: n = 500009 26 -> 12 ms)
+    tb.buf.reserve(tb.buf.size() + (size_t)(n + M) * 2 * prec + (M > 32768 ? (size_t)1 << 20 : 4096));
     std::vector<d2> b((size_t)M, d2{0, 0});
     std::vector<d2> cb((size_t)n);
     for (int64_t k = 0; k < n; k++) {
@@ -1248,7 +1290,13 @@ static bool split_factors(int64_t N, int64_t fmax, std::vector<int64_t>& f)
 // holds, so from 512 points on the segments of a row shrink below 256 bytes
 // (complex128 tiles of 2^k take the whole LDS and hold out longer).  The last
 // pass reads rows and is affected on its store only.  The generic kernel adds
-// by its stages.
+// by its stages.  It does not know how many lines a generic tile gets: 4 lines of
+// 1440 x 1440 complex128 points take 189 us as the two passes it prefers, 161 as
+// three, but pricing such tiles up moved as many lengths the wrong way (5 lines
+// of 632,736 61.8 -> 79.7 us).  Powers of two are priced as the fixed kernels also
+// where the products of a Bluestein transform need the generic one; its two
+// wide passes were the faster at every length tried (131071: 39.5 against 43.3
+// us, 16 lines in complex128 132 against 165; 1048573: 88 against 91).
 static double pass_cost(int64_t f, bool last, int prec)
 {
     static const double col[2][6] = {{0.97, 1.0, 1.17, 1.4, 2.3, 4.0}, {0.95, 0.95, 1.12, 1.17, 1.45, 2.3}};  // 128 ..
@@ -1268,9 +1316,11 @@ static double pass_cost(int64_t f, bool last, int prec)
 static bool split_two(int64_t N, int prec, std::vector<int64_t>& f, double& cost)
 {
     cost = 1e300;
-    for (int64_t a = 16; a <= 2048 && a <= N; a++) {
+    if (N > 2048 * 2048) return false;
+    for (int64_t a = std::max<int64_t>(16, (N + 2047) / 2048); a <= 2048 && 16 * a <= N; a++) {
+        if ((uint32_t)N % (uint32_t)a) continue;
         const int64_t b = N / a;
-        if (N % a || b < 16 || b > 2048 || !smooth13(a) || !smooth13(b)) continue;
+        if (!smooth13(a) || !smooth13(b)) continue;
         // wide generic passes leave one or two lines per tile
         const int64_t generic = prec == 4 ? 2048 : 1536;
         if (((a & (a - 1)) && a > generic) || ((b & (b - 1)) && b > generic)) continue;
@@ -1652,7 +1702,8 @@ static bool plan_real(Plan* plan, TableBuilder& tb, std::vector<AxisSpec> dims, 
     int64_t rtw_off = -1;
     if (packed) {
         std::vector<d2> rtw((size_t)L);
-        for (int64_t k = 0; k < L; k++) rtw[(size_t)k] = root_fwd(k, n0);
+        const RootTable root(n0);
+        for (int64_t k = 0; k < L; k++) rtw[(size_t)k] = root(k);
         rtw_off = tb.add_complex(rtw, prec);
     }
     // complex geometry of the half-spectrum side
