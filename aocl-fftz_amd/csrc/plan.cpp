@@ -748,7 +748,7 @@ static bool build_pass(Plan* plan, TableBuilder& tb, const PassReq& q, std::stri
     // 18.9 -> 14.5 us, 1024 of 4095 43.5 -> 35.9; 256 of 4095 the reverse, 13.2
     // and 14.4).  Columns have their own limit below.
     if (!plan_match && prec == 8 && ln.rad != kRadTo8 && nl_total > dev.cus && !q.want_in_col && !q.want_out_col &&
-        2 * (size_t)lds_pad(need) * esize <= dev.lds_per_block)
+        tuned_e != 8 && tuned_e != 16 && 2 * (size_t)lds_pad(need) * esize <= dev.lds_per_block)
         tmax = std::min(tmax, 256);
     // threads per line, and the table and layout that go with the kernel
     int TL;
@@ -858,7 +858,7 @@ static bool build_pass(Plan* plan, TableBuilder& tb, const PassReq& q, std::stri
             const bool aligned = (!in_col || q.ies % 8 == 0) && (!out_col || q.oes % 8 == 0) && n0 % (C * 2) == 0;
             const int64_t rows = nl_total / n0, narrow = rows * ((n0 + C - 1) / C), wide = rows * ((n0 + C * 2 - 1) / (C * 2));
             const int64_t cus = dev.cus;
-            if (C == 1 || aligned || (narrow > cus && wide * 2 <= narrow + narrow / 32 &&
+            if (C == 1 || aligned || plan->spec.tune.col_c || (narrow > cus && wide * 2 <= narrow + narrow / 32 &&
                                      (wide + cus - 1) / cus <= (narrow + 2 * cus - 1) / (2 * cus)))
                 C *= 2;
         }
