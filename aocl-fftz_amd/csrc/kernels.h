@@ -9,8 +9,8 @@ enum class KernelKind { Pass, Real, RealWide, Bluestein };
 
 // Radices a generic kernel carries.  The widest butterfly it carries sets the
 // registers, and with them the wavefronts, of every launch; wavefronts per SIMD
-// of the plain pass and of Bluestein in complex64 / complex128: kRadAll 4 / 2,
-// kRadLight 5 / 3, kRadTo8 - / 4.
+// of the plain pass in complex64 / complex128: kRadAll 4 / 3, kRadLight 5 / 3,
+// kRadTo8 - / 4; of Bluestein: kRadAll 5 / 2, kRadLight 5 / 3, kRadTo8 - / 4.
 enum RadixSet : int {
     kRadPow2 = 0,   // 2, 4, 8, 16
     kRadAll = 1,    // 2 .. 13, 16

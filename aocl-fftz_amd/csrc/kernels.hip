@@ -1,6 +1,6 @@
 // Launch table of the LDS pass kernels: precision x radix set x block
 // limit.  The kernels themselves are instantiated in
-// kernels_pass_{f32,f64}_{mixed,pow2}.hip and
+// kernels_pass_{f32,f64}_{mixed,pow2,light}.hip, kernels_pass_f64_to8.hip and
 // kernels_batch_{f32,f64}_{small,medium,large}.hip (one translation unit
 // each, so they compile in parallel) from kernels_body.h.
 #include <hip/hip_runtime.h>

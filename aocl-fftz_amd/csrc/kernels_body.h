@@ -18,9 +18,9 @@
 // issue and LDS latency rather than HBM, at 75 VALU instructions per element
 // for three stages (a self-sorting form with its results moved and guarded
 // took 112).  Measured, before -> after: 3001 complex64 lines of 1200
-// (12 x 10 x 10) 26.7 -> 17.9 us; 9 lines of 1,000,000 as three passes of 100
-// 187 -> 112 us; 1500 complex128 lines of 1009 (Bluestein, M = 2048)
-// 37.1 -> 30.8 us; 2000 uneven items 2.87 -> 2.32 ms.  (The reference's
+// (12 x 10 x 10) 26.7 -> 17.9 us; 9 lines of 1,000,000, then planned as three
+// passes of 100, 187 -> 112 us; 1500 complex128 lines of 1009 (Bluestein, M =
+// 2048) 37.1 -> 30.8 us; 2000 uneven items 2.87 -> 2.32 ms.  (The reference's
 // self-sorting geometry, core/solvers/complex/pow2_iterative_solver_dft.c:27-78,
 // moves every stage's results instead.)
 //

@@ -224,8 +224,8 @@ static bool factor_radices(int L, std::vector<int>& out)
     for (int S = 1; !pick_radices(L, S, out); S++) {}
     std::sort(out.begin(), out.end(), std::greater<int>());
     // A radix-2 stage costs nearly as much LDS traffic and addressing as any
-    // other: 16 16 16 2 becomes 16 8 8 8 (8192-point complex64 lines).  The
-    // lengths of the fixed kernels keep their plan.
+    // other: 16 16 16 2 becomes 16 16 8 4 (lines of 8192 points).  The lengths of
+    // the fixed kernels keep their plan.
     if (out.size() >= 3 && out.back() == 2 && !((L & (L - 1)) == 0 && L <= 4096)) {
         std::vector<int> r = out;
         const size_t S = r.size();
@@ -393,10 +393,12 @@ static int64_t stage_twiddles(TableBuilder& tb, int prec, const std::vector<int>
 // element).
 //   * Wide enough that neighbouring lanes cover 64 bytes of a line, and a
 //     column tile fills a wavefront (mint).
-//   * At most 16 elements per thread: beyond that too few wavefronts fit next
-//     to the lines' LDS (1,000,000-point complex64, passes of 100: 12 per
-//     thread 97 us, 25 per thread 104 us; 100 x 120 x 144 complex128 grid, 12
-//     and 16 per thread 84.7 us, 25 to 32 per thread 87.1 us).
+//   * At most 16 elements per thread where maxt allows it: beyond that too few
+//     wavefronts fit next to the lines' LDS (1,000,000-point complex64, passes
+//     of 100: 12 per thread 97 us, 25 per thread 104 us; 100 x 120 x 144
+//     complex128 grid, 12 and 16 per thread 84.7 us, 25 to 32 per thread 87.1
+//     us).  Column passes allow 20 before they double maxt, complex128 rows stop
+//     at 256 threads where that keeps two workgroups on a CU (build_pass).
 //   * Among the widths within 8% of the least work, short lines take the
 //     narrowest (room for more lines) and long ones and pair stages the widest
 //     (more loads in flight per line).
@@ -417,7 +419,7 @@ static int line_threads(const std::vector<int>& radix, int L, int mint, int maxt
             const int items = (L / r + per - 1) / per;
             w += (double)((items + tl - 1) / tl) * tl * per * r * radix_stage_cost(r);
         }
-        return tl * 16 < L ? 1.15 * w : w;
+        return w;
     };
     int first = 1;
     while (first < widest && (first * 16 < L || first < mint)) first *= 2;
@@ -701,11 +703,12 @@ static bool build_pass(Plan* plan, TableBuilder& tb, const PassReq& q, std::stri
         if (q.kind == KernelKind::Pass && plan->spec.mfma_mode == kMfmaNone && radix_order_ok(q.L, *tr)) radix = *tr;
     d.nst = (int)radix.size();
     // The narrowest radix set that holds the line's radices: its kernel has the
-    // fewest registers.  Complex128, all radices -> set: 100 x 120 x 144 grid
-    // 91 -> 85 us (kRadLight), 2048 x 675 real batch of 4 214 -> 155 us
-    // (kRadTo8), 2894 lines of 1372 47.7 -> 41 us; complex64: 3001 lines of 1200
-    // 14.9 -> 14.1 us.  A complex64 set of radices up to 8 would save no
-    // wavefront worth having over kRadLight (78 against 92 VGPRs).
+    // fewest registers.  All radices -> set, when the sets were made (kernel time,
+    // of one build): complex128 100 x 120 x 144 grid 91 -> 85 us (kRadLight), 2048 x
+    // 675 real batch of 4 214 -> 155 us (kRadTo8), 2894 lines of 1372 47.7 -> 41 us;
+    // complex64 3001 lines of 1200 forward 14.9 -> 14.1 us.  A complex64 set of
+    // radices up to 8 would save no wavefront worth having over kRadLight (78
+    // against 92 VGPRs).
     const bool real = q.kind == KernelKind::Pass && (q.flags & kRealFlags);
     for (int set : {kRadAll, kRadPow2, kRadLight, kRadTo8}) {
         if ((set == kRadLight && real) || (set == kRadTo8 && prec == 4)) continue;
@@ -1054,10 +1057,13 @@ static int64_t bluestein_length(int64_t n)
         if (smooth13(m)) return m;
 }
 
-// Estimated vector instructions per element for one generic LDS stage of
-// radix r: the in-register DFT-r (real operations per element of the codelet
-// in codelets.h), the stage-twiddle product ((r - 1) / r complex products)
-// and the LDS addressing of one read and one write.
+// Relative cost per element of one generic LDS stage of radix r: the in-register
+// DFT-r (real operations per element of the codelet in codelets.h), the
+// stage-twiddle product ((r - 1) / r complex products) and the addressing of one
+// LDS read and write.  The last part was counted on self-sorting stages; the
+// in-place ones take about a third less in all, much the same for every radix
+// (74 instructions per element for 12 x 10 x 10 where this adds up to 77.5), so
+// the order of the choices made by it stands.
 static double radix_stage_cost(int r)
 {
     switch (r) {
